@@ -79,8 +79,8 @@ extern "C" {
 #define SPH_T_FORCE 4
 #define SPH_T_REDUCE 5
 /* the three launches inside SPH_T_KNN_DENSITY */
-#define SPH_T_KNN_WALK 6     /* tile walk of the bracketed fast path */
-#define SPH_T_KNN_FINISH 7   /* annulus selection, density, force records */
+#define SPH_T_KNN_WALK 6     /* bracketed walk, density, force records */
+#define SPH_T_KNN_FINISH 7   /* nothing (part of the walk) */
 #define SPH_T_KNN_FALLBACK 8 /* exact wavefront search of the remaining queries */
 #define SPH_NTIMERS 9
 
@@ -237,15 +237,16 @@ int sph_batch_reductions(sph_sim* s, int32_t sim, double out[6]);
 int sph_set_graph(sph_sim* s, int32_t on);
 /* Time force passes over the candidate cell grid resolutions (cells per
  * particle 0.5 ... 16) on the current state and keep the fastest, then tune
- * the kNN walk's tile shape on that grid one knob at a time: sub-tiles per
- * wave (8, 4), the lane group a wave starts with (64, 32 queries), and the
- * candidates per query above which a group is halved (24, 32, 16).  Only
+ * the kNN walk's shape on that grid one knob at a time: the sub-tiles (cells
+ * per axis) a group of 16 queries is looked up in (8, 4), the queries a wave
+ * takes (64, 32), and the candidates per query above which a group is halved
+ * (24, 32, 16).  Only
  * before the first step (SPH_ESTATE otherwise).  Either output may be NULL.
  * Outside the bitwise form the grid and shape change the order in which
  * neighbours are summed (results within the precision form's contract). */
 int sph_autotune(sph_sim* s, double* best_ms, double* best_cells_per_particle);
 /* The grid and walk shape in use: cells per particle, bracket half-width
- * around each query's last h, split threshold, first lane group, sub-tiles.
+ * around each query's last h, split threshold, queries per wave, sub-tiles.
  * The bracket adapts per simulation after every pass (widened by a quarter
  * when more than 1/128 of the queries fell outside it because h moved,
  * narrowed by a fifth when more than 1/128 overflow its annulus, within

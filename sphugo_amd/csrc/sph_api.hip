@@ -198,7 +198,7 @@ int sph::alloc_state(sph_sim* h, int64_t np, int nitems) {
     if ((rc = h->alloc(&f.id, np))) return rc;
   }
   if ((rc = h->alloc(&h->P[0].x, np)) || (rc = h->alloc(&h->P[0].y, np)) ||
-      (rc = h->alloc(&pb.xyp, np)) || (rc = h->alloc(&pb.uxy, np)))
+      (rc = h->alloc(&pb.xyp, np)))
     return rc;
   if ((rc = h->alloc(&pb.wrap, np)) || (rc = h->alloc(&pb.cstart, h->cell_capacity)) ||
       (rc = h->alloc(&pb.nbr, nbr_entries(np, pb.kmax))) ||
@@ -210,7 +210,6 @@ int sph::alloc_state(sph_sim* h, int64_t np, int nitems) {
       (rc = h->alloc(&pb.red_part, (int64_t)pb.nsims * kRedSplit * kNumRed)) ||
       (rc = h->alloc(&pb.retry, np)) || (rc = h->alloc(&pb.retry_count, 1)) ||
       (rc = h->alloc(&pb.runs, 4 * (int64_t)kRunQueue)) || (rc = h->alloc(&pb.run_count, 1)) ||
-      (rc = h->alloc(&pb.knn_cnt, np)) || (rc = h->alloc(&pb.knn_ann, (np + 63) / 64 * 64 * kAnn)) ||
       (rc = h->alloc(&pb.sort.keys, np)) || (rc = h->alloc(&pb.sort.vals, np)) ||
       (rc = h->alloc(&pb.sort.keys_alt, np)) || (rc = h->alloc(&pb.sort.vals_alt, np)) ||
       (rc = h->alloc(&pb.sort.counts, sort_counts_size(np))) || (rc = h->alloc(&pb.sort.tot, 256)) ||
@@ -524,8 +523,8 @@ extern "C" int sph_autotune(sph_sim* s, double* best_ms, double* best_cpp) {
       bcpp = cpp;
     }
   }
-  // then the walk's tile shape on that grid, one knob at a time (sub-tiles,
-  // first lane group, split threshold); the bracket width stays: it answers
+  // then the walk's shape on that grid, one knob at a time (sub-tiles,
+  // queries per wave, split threshold); the bracket width stays: it answers
   // to the motion between passes, which passes at rest cannot show
   if (!rc && !s->bitwise) {
     if ((rc = fetch_sims(s)) == 0) {

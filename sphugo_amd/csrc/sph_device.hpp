@@ -208,11 +208,11 @@ struct Item {
   int64_t first;
 };
 
-// Tile-search shape of the kNN walk (the autotuner's knobs): bracket
-// half-width around each query's last h, the largest candidate count per
-// query of a lane group before it is halved, the lane group a wave starts
-// with (queries searched together: 64, 32 or 16), and the sub-tiles a wave
-// filters its staged candidates for (4 or 8).
+// Shape of the kNN walk (the autotuner's knobs): bracket half-width around
+// each query's last h, the candidates per query (of a full group of 16) in a
+// group's cells above which the group is halved, the queries a wave takes (64,
+// 32 or 16, in groups of 16 one after the other), and the cells per axis that
+// a group's box is looked up in at most (4 or 8; the ABI calls it sub-tiles).
 struct WalkKnobs {
   double delta;
   int32_t split;
@@ -273,17 +273,6 @@ __device__ inline double kern_DF(int32_t kernel, double q) {
   if (q < 0.5) return (3 * q * q - 2 * q);
   return -(1 - q) * (1 - q);
 }
-// FP64 kernel value with fused multiply-adds (the plain FP64 form's density,
-// whose contract is 1e-12 relative; the bitwise form keeps kern_F)
-__device__ inline double kern_F_fma(int32_t kernel, double q) {
-  if (kernel == kWendland) {
-    const double a = 1 - q, a2 = a * a;
-    return a2 * a2 * fma(4.0, q, 1.0);
-  }
-  if (q < 0.5) return fma(q * q, q - 1, 1.0 / 6);
-  const double a = 1 - q;
-  return a * a * a * (1.0 / 3);
-}
 // FP64 derivative with fused multiply-adds (the plain FP64 form's force,
 // whose contract is 1e-12 relative; the bitwise form keeps kern_DF)
 __device__ inline double kern_DF_fma(int32_t kernel, double q) {
@@ -302,6 +291,14 @@ __device__ inline double kern_DF_fma(int32_t kernel, double q) {
 // over neighbours are instantiated per type (kern_visit) rather than
 // branching on it per pair.
 struct CubicF {
+  // FP64 kernel value with fused multiply-adds (the plain FP64 form's
+  // density, whose contract is 1e-12 relative; the bitwise form keeps kern_F)
+  __device__ static double F64(double q) {
+    const double a = 1 - q;
+    const double lo = fma(q * q, q - 1, 1.0 / 6);
+    const double hi = a * a * a * (1.0 / 3);
+    return q < 0.5 ? lo : hi;
+  }
   __device__ static float F(float q) {
     const float a = 1.f - q;
     const float lo = __builtin_fmaf(q * q, q - 1.f, 1.f / 6.f);
@@ -316,6 +313,10 @@ struct CubicF {
   }
 };
 struct WendlandF {
+  __device__ static double F64(double q) {
+    const double a = 1 - q, a2 = a * a;
+    return a2 * a2 * fma(4.0, q, 1.0);
+  }
   __device__ static float F(float q) {
     const float a = 1.f - q;
     const float a2 = a * a;
@@ -356,6 +357,20 @@ __device__ inline double rsq64(double x) {
   y = fma(y, r, y);
   r = fma(-hx * y, y, 0.5);
   return fma(y, r, y);
+}
+
+// sqrt(x) / h for hinv near 1 / h: one Newton step on the reciprocal square
+// root, then a residual step on the root and one on the quotient, which leave
+// both rounded as the exact operations round them (but for rare last-place
+// cases).  1 - q keeps its digits that way where q is near 1.
+__device__ inline double sqrt_over(double x, double h, double hinv) {
+  double y = __builtin_amdgcn_rsq(x);
+  const double t = 0.5 * x * y;
+  y = fma(y, fma(-t, y, 0.5), y);
+  const double s0 = x * y;
+  const double s = fma(fma(-s0, s0, x), 0.5 * y, s0);
+  const double q = s * hinv;
+  return fma(fma(-q, h, s), hinv, q);
 }
 
 // ---- wave helpers (wave64) ----

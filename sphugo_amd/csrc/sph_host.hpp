@@ -53,7 +53,6 @@ struct PassBuffers {
   int key_bits;
   Positions pos_cur;    // positions at rest (P0)
   double2* xyp;         // positions of the pass, interleaved (x, y)
-  uint2* uxy;           // FP32C: the same as 32-bit fixed point of the box
   Fields fcur;          // fields, current order
   Fields fnew;          // fields, order of this pass
   uint8_t* wrap;        // wrap code per particle of the pass
@@ -69,8 +68,6 @@ struct PassBuffers {
   uint32_t* retry_count;
   uint32_t* runs;          // queued cell chunks of the pass: (first, last, t0, nv) x kRunQueue
   uint32_t* run_count;
-  uint32_t* knn_cnt;       // per query: certain | annulus << 8, or ~0 (retry)
-  uint32_t* knn_ann;       // per query: annulus candidates (kAnn entries)
   int have_h;             // every particle has an h from an earlier pass
   int any_open;           // some simulation has an open axis (k_bbox, k_box run)
   WalkKnobs walk;         // tile-search shape of the kNN walk

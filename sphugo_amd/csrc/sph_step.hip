@@ -6,16 +6,14 @@
 //   sort_pairs      stable LSD radix sort of (key, index) (sph_sort.hip)
 //   k_permute       gather the state into cell order, apply the drift-1 /
 //                   predictor step (sim/sph.go:108-117) or the step-0
-//                   initialisation (:96-101), write the cell ranges and
-//                   (FP32C) the fixed-point positions
+//                   initialisation (:96-101), and write the cell ranges
 //   k_fill_runs     the cell ranges of sparse grid stretches k_permute queued
-//   k_knn           tile walk: a wavefront takes 64 consecutive queries,
-//                   stages the candidates of their cells through LDS and
-//                   sorts them against each query's bracket around its last
-//                   h: certain neighbours go to the list, the annulus to a
-//                   short side list; misses go to a retry list
-//   k_knn_finish    thread per query: exact selection of the annulus,
-//                   density and sound speed, the force record
+//   k_knn           bracketed walk: a wavefront searches groups of 16
+//                   consecutive queries, sorting the candidates of each
+//                   group's box against every query's bracket around its last
+//                   h, then selects the k-th neighbour exactly, sums the
+//                   density and writes sound speed and the force record;
+//                   misses go to a retry list
 //                   (sim/nearest-neighbour.go:28-165, sim/sph.go:306-323,
 //                   421-429)
 //   k_knn_fallback  exact wavefront-per-query search for the retry list (or
@@ -276,7 +274,7 @@ __global__ __launch_bounds__(256) void k_fill_runs(const uint32_t* __restrict__ 
 __global__ __launch_bounds__(kItem) void k_permute(
     const Item* __restrict__ items, int nitems, const SimDev* __restrict__ sims,
     const uint32_t* __restrict__ perm, const uint32_t* __restrict__ skeys, int mode,
-    Positions pin, Fields fin, double2* __restrict__ xyp, uint2* __restrict__ uxy, Fields fout,
+    Positions pin, Fields fin, double2* __restrict__ xyp, Fields fout,
     uint8_t* __restrict__ wrap, uint32_t* __restrict__ cstart, uint32_t* __restrict__ runs,
     uint32_t* __restrict__ run_count) {
   const Item it = items[xcd_item(nitems)];
@@ -341,11 +339,6 @@ __global__ __launch_bounds__(kItem) void k_permute(
       vpx = fin.vpx[i]; vpy = fin.vpy[i]; ep = fin.ep[i];
     }
     xyp[t] = make_double2(x, y);
-    // FP32C: the fixed-point form of the force record (units of L / 2^32,
-    // wrapped), whose 32-bit differences are minimum-image displacements
-    if (S->prec == kPrecFP32C)
-      uxy[t] = make_uint2((uint32_t)(int64_t)floor((x - S->x0) * (4294967296.0 / S->lx)),
-                          (uint32_t)(int64_t)floor((y - S->y0) * (4294967296.0 / S->ly)));
     fout.vx[t] = vx;
     fout.vy[t] = vy;
     fout.e[t] = e;
@@ -388,7 +381,6 @@ __device__ inline void cell_range(const SimDev* S, const uint32_t* __restrict__ 
 }
 
 constexpr int kV1Cells = 128;  // coarse cells of one search (<= 9 x 9 used)
-constexpr int kTileCells = 256;  // coarse cells of one tile box (<= 15 x 15 used)
 
 // Per-wave scratch of the exact wavefront search.
 struct SearchShared {
@@ -401,22 +393,6 @@ struct SearchShared {
   double sd2[kMaxK];
   uint32_t spk[kMaxK];
   double fterm[kMaxK];
-};
-
-// Per-wave scratch of the tile search (lane = query), KSUB sub-tiles.
-template <int KSUB>
-struct TileShared {
-  uint32_t pst[kTileCells];
-  int ppref[kTileCells + 1];
-  int8_t ptx[kTileCells];
-  int8_t pty[kTileCells];
-  double2 sxy[65];           // staged candidates; entry 64 is a NaN sentinel
-  uint32_t spk[65];
-  double sbb[KSUB][4];       // box of each sub-tile (x0, x1, y0, y1)
-  uint8_t slist[KSUB][64];   // staged candidates within reach of each sub-tile
-  uint32_t slpk[KSUB][64];   // their packed entries, in the same order
-  unsigned long long smask[KSUB];  // staged slots in each sub-tile's list
-  unsigned long long selfm[64];    // per query: staged slots that are itself
 };
 
 struct SearchOut {
@@ -454,7 +430,7 @@ __device__ inline NbrRow nbr_row(const uint32_t* nbr, int64_t t, int kstride) {
 // Writes the k entries of `row` (BITWISE: sorted descending by (d2, ID,
 // image), the reference's queue order) and returns tau and the density
 // kernel sum (BITWISE: summed farthest first, sim/sph.go:313-320).
-template <bool BITWISE, bool FP32C>
+template <bool BITWISE>
 __device__ SearchOut wave_search(const SimDev* S, int64_t t, double xq, double yq, double R,
                                  const double2* __restrict__ XY,
                                  const uint8_t* __restrict__ WR,
@@ -663,14 +639,12 @@ __device__ SearchOut wave_search(const SimDev* S, int64_t t, double xq, double y
   }
   const double h = sqrt(tau);
   const int kern = S->kernel;
+  // The kernel sum is in FP64 in every form: these searches are few and wait
+  // on loads, and their rows include the ill-conditioned ones (every neighbour
+  // near q = 1, where F(q) = (1 - q)^3 / 3 amplifies a rounding of q by
+  // 3 q / (1 - q)).
   double facc = 0.0;
-  float fs = 0.f, fc = 0.f;
-  // FP32C: q^2 = d^2 / tau formed in FP64 before the FP32 square root.  A
-  // rounded 1 / h shared by every term would move all q together, and
-  // F(q) = (1 - q)^3 / 3 amplifies that by 3q / (1 - q): a particle whose
-  // neighbours all sit near q = 1 (the edge of a dense clump) would lose
-  // 1e-5 of its density.
-  const double itau = 1.0 / tau;
+  const double hinv = 1.0 / h;
   int emitted = 0;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -681,17 +655,8 @@ __device__ SearchOut wave_search(const SimDev* S, int64_t t, double xq, double y
       const int pos = emitted + lane_prefix(m);
       if constexpr (!BITWISE) {
         row[pos] = pkr[s];
-        if constexpr (FP32C) {
-          // hardware square root (within 1 ulp), as in the walk's finish
-          const float q = __builtin_amdgcn_sqrtf((float)(v[s] * itau));
-          const float f = kern_Ff(kern, q > 1.f ? 1.f : q);
-          const float y = f - fc;
-          const float tt = fs + y;
-          fc = (tt - fs) - y;
-          fs = tt;
-        } else {
-          facc += kern_F(kern, sqrt(v[s]) / h);
-        }
+        facc += kern == kWendland ? WendlandF::F64(sqrt_over(v[s], h, hinv))
+                                  : CubicF::F64(sqrt_over(v[s], h, hinv));
       } else {
         sh.sd2[pos] = v[s];
         sh.spk[pos] = pkr[s];
@@ -700,22 +665,7 @@ __device__ SearchOut wave_search(const SimDev* S, int64_t t, double xq, double y
     emitted += __popcll(m);
   }
   if constexpr (!BITWISE) {
-    if constexpr (FP32C) {
-      // compensated tree sum: each level carries its rounding error
-      float s_ = fs, c_ = -fc;
-      for (int o = 32; o > 0; o >>= 1) {
-        const float so = __shfl_xor(s_, o, 64);
-        const float co = __shfl_xor(c_, o, 64);
-        const float sum = s_ + so;
-        const float bp = sum - s_;
-        const float err = (s_ - (sum - bp)) + (so - bp);
-        s_ = sum;
-        c_ = c_ + co + err;
-      }
-      out.facc = (double)s_ + (double)c_;
-    } else {
-      out.facc = group_sum(facc, 64);
-    }
+    out.facc = group_sum(facc, 64);
   } else {
     __builtin_amdgcn_wave_barrier();
     double dv = lane < k ? sh.sd2[lane] : -1.0;
@@ -837,395 +787,706 @@ __device__ inline double local_radius(const SimDev* S, const uint32_t* __restric
   }
 }
 
-// kNN + density + sound speed + force record.  A wave takes 64 consecutive
-// (Hilbert-ordered) queries.  Fast path (lane = query): the wave stages the
-// candidates of the tile's bounding box (grown by each query's bracket
-// radius) through LDS 64 at a time and every lane tests all of them against
-// its bracket [h_prev (1 - delta), h_prev (1 + delta)]: nearer candidates
-// are certain neighbours and go straight to the list; the annulus keeps at
-// most kAnn entries (written straight to global memory, which keeps the
-// wave's LDS small) from which the remaining ones are selected exactly.
-// Queries without a previous h, or whose bracket misses, fall back to the
-// exact wavefront search.  BITWISE uses the wavefront search for all.
-// Five waves per SIMD (a few spilled registers): the walk is issue-bound
-// with long LDS and gather latencies; its LDS (about 7 KB per wave) allows
-// five blocks per CU.
-template <bool BITWISE, bool FP32C, int KSUB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_knn(
+// Block-compensated FP32 sum: the terms of one round (4 or 8 neighbours)
+// add up plainly, and each round's partial joins the running sum through a
+// Kahan step.  Besides the compensated sum's own error this adds at most
+// (B - 1) 2^-24 of the sum of |terms| of a block of B, against four
+// operations per term for a Kahan step per term.
+struct BlockKahan {
+  float s = 0.f, c = 0.f, p = 0.f;
+  __device__ void add(float t) { p += t; }
+  __device__ void add_mul(float a, float b) { p = __builtin_fmaf(a, b, p); }
+  __device__ void flush() {
+    const float y = p - c;
+    const float tt = s + y;
+    c = (tt - s) - y;
+    s = tt;
+    p = 0.f;
+  }
+  __device__ double value() const { return (double)s - (double)c; }
+};
+
+// ---- the bracketed walk ----
+constexpr int kGrp = 16;         // queries searched together (a group)
+constexpr int kWalkCand = 240;   // candidates of a group's box, held in LDS
+constexpr int kWalkRounds = 4;   // the same in rounds of 64 (one candidate per lane)
+constexpr int kWalkRaw = 1024;   // candidates of the box's cells
+
+// Scratch of a walk wave: 10 KiB, so that sixteen waves share a CU's LDS (four
+// per SIMD, which its registers allow without spilling).
+struct WalkShared {
+  double2 xy[kWalkCand];        // candidates inside the group's box
+  uint32_t pk[kWalkCand];       // their packed entries
+  uint8_t row[kGrp][68];        // per query: candidate slots of its neighbours
+  uint8_t annl[kGrp][kAnn];     // per query: candidate slots in its annulus
+  union {
+    struct {
+      uint8_t mark[kWalkRaw];   // first candidate of cell c (lane c): c + 1
+      uint2 piece[64];          // per cell: sorted slot minus candidate number, image tile
+    } s;
+    double ad[kAnn][kGrp];      // annulus squared distances (entry, query)
+  } u;
+  // per query of the wave: x, y, then Rlo^2, Rhi^2 until its group is
+  // searched, and after it tau and the kernel sum; tau < 0: not found (kMiss*)
+  double4 q[64];
+};
+constexpr double kThinSum = 2e-3;  // FP32C kernel sums below it are redone in FP64
+constexpr double kMissWide = -1.0, kMissLo = -2.0, kMissAnn = -3.0, kMissHi = -4.0;
+static_assert(sizeof(WalkShared) == 10240, "sixteen waves per CU");
+
+typedef __attribute__((address_space(3))) uint8_t LdsByte;
+__device__ inline uint32_t lds_addr(const uint8_t* p) {
+  return (uint32_t)(uintptr_t)(LdsByte*)p;
+}
+__device__ inline LdsByte* lds_u8(uint32_t a) { return (LdsByte*)(uintptr_t)a; }
+
+// One wave's LDS operations complete in order; this keeps the compiler from
+// moving them across.
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Lane moves within rows of 16 (and, row by row, into the rows after): lanes
+// without a source read 0.
+template <int CTRL, int ROWS = 0xf>
+__device__ inline uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, true);
+}
+// minimum over each row of 16 lanes (every lane ends with it), of values that
+// are no NaN
+__device__ inline float row_min(float v) {
+  auto step = [](float a, uint32_t b) { return __builtin_amdgcn_fmed3f(a, __uint_as_float(b), -INFINITY); };
+  v = step(v, dpp<0xB1>(__float_as_uint(v)));   // lane ^ 1
+  v = step(v, dpp<0x4E>(__float_as_uint(v)));   // lane ^ 2
+  v = step(v, dpp<0x141>(__float_as_uint(v)));  // mirror of 8: the other quad
+  return step(v, dpp<0x140>(__float_as_uint(v)));
+}
+// inclusive scans over the wave: row shifts, then the last lane of each row
+// into the rows after it
+__device__ inline uint32_t scan_add(uint32_t v) {
+  v += dpp<0x111>(v);
+  v += dpp<0x112>(v);
+  v += dpp<0x114>(v);
+  v += dpp<0x118>(v);
+  v += dpp<0x142, 0xa>(v);
+  v += dpp<0x143, 0xc>(v);
+  return v;
+}
+__device__ inline uint32_t scan_max(uint32_t v) {
+  auto mx = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+  v = mx(v, dpp<0x111>(v));
+  v = mx(v, dpp<0x112>(v));
+  v = mx(v, dpp<0x114>(v));
+  v = mx(v, dpp<0x118>(v));
+  v = mx(v, dpp<0x142, 0xa>(v));
+  v = mx(v, dpp<0x143, 0xc>(v));
+  return v;
+}
+
+// The Hilbert index (hilbert2) of cell (x, y) at level c <= 15, three levels
+// per step: the orientation (swap, complement) entering three levels and their
+// three bits of x and y give the six index bits and the orientation that
+// leaves them.  The 256 bytes of that table sit in one register per lane
+// (lane l: entries 4 l .. 4 l + 3) and are looked up across the lanes.  A
+// level of zero bits above the first only flips the swap, so a start
+// orientation of their parity pads c to a multiple of three.
+struct HilbertTable {
+  uint32_t w[64];
+};
+constexpr HilbertTable make_hilbert_table() {
+  HilbertTable t{};
+  for (uint32_t i = 0; i < 256; ++i) {
+    uint32_t swap = i >> 6 & 1u, comp = i >> 7, d = 0;
+    for (int s = 2; s >= 0; --s) {
+      const uint32_t bx = (i >> (3 + s)) & 1u, by = (i >> s) & 1u;
+      const uint32_t rx = (swap ? by : bx) ^ comp;
+      const uint32_t ry = (swap ? bx : by) ^ comp;
+      d = (d << 2) | ((3u * rx) ^ ry);
+      const uint32_t m = ry ^ 1u;
+      swap ^= m;
+      comp ^= m & rx;
+    }
+    t.w[i >> 2] |= (d | swap << 6 | comp << 7) << (8 * (i & 3u));
+  }
+  return t;
+}
+__constant__ const HilbertTable kHilbertTable = make_hilbert_table();
+__device__ inline uint32_t hilbert_lookup(uint32_t table, uint32_t x, uint32_t y, int c) {
+  const int steps = (c + 2) / 3;
+  uint32_t d = 0, state = (uint32_t)(3 * steps - c) & 1u;
+  for (int s = 3 * (steps - 1); s >= 0; s -= 3) {
+    const uint32_t i = state << 6 | ((x >> s) & 7u) << 3 | ((y >> s) & 7u);
+    const uint32_t e =
+        (uint32_t)__builtin_amdgcn_ds_bpermute((int)i, (int)table) >> (8 * (i & 3u)) & 255u;
+    d = d << 6 | (e & 63u);
+    state = e >> 6;
+  }
+  return d;
+}
+
+// Squared distance of the candidate in slot `slot` from (xq, yq), in the
+// reference's order: ((p_i + o) - p_j)^2.  IMG: some candidate of the group
+// is seen through an image (p_i + 0 is p_i).
+template <bool IMG>
+__device__ inline double slot_d2(const WalkShared& sh, uint32_t slot, double xq, double yq,
+                                 double lx, double ly) {
+  const double2 pj = sh.xy[slot];
+  double ax = xq, ay = yq;
+  if constexpr (IMG) {
+    const uint32_t im = sh.pk[slot] & 15u;
+    ax = xq + (double)img_ix(im) * lx;
+    ay = yq + (double)img_iy(im) * ly;
+  }
+  const double ex = ax - pj.x, ey = ay - pj.y;
+  return ex * ex + ey * ey;
+}
+
+// Classifies the group's candidates (lane = candidate, NR rounds of 64 in
+// registers) for the queries of `gmask` one after the other: the query's
+// data is the same in every lane, so a comparison's result is the mask of
+// its certain neighbours (inside Rlo) or of its reach (up to Rhi), and a
+// candidate's place in the query's list is a prefix count of that mask.  No
+// lane waits for another's list, whatever the lists' lengths.  Lanes ql == i
+// of every row return query i's counts.  IMG: some candidate is seen through
+// an image.
+template <int NR, bool IMG>
+__device__ inline void classify(WalkShared& sh, const double4* gq, int ncand, uint32_t gmask, uint32_t t0, int k,
+                                double lx, double ly, int lane, int& c_lo, int& c_an) {
+  double x[NR], y[NR], ox[NR], oy[NR];
+  uint32_t j[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int s = r * 64 + lane;
+    const bool in = s < ncand;
+    const double2 p = sh.xy[in ? s : 0];
+    const uint32_t pk = sh.pk[in ? s : 0];
+    x[r] = in ? p.x : NAN;  // compares false with everything
+    y[r] = p.y;
+    j[r] = pk >> 4;
+    if constexpr (IMG) {
+      ox[r] = (double)img_ix(pk & 15u) * lx;
+      oy[r] = (double)img_iy(pk & 15u) * ly;
+    }
+  }
+  const int ql = lane & (kGrp - 1);
+  // LDS addresses as numbers: a list's base folds into its prefix count
+  const uint32_t rows = lds_addr(&sh.row[0][0]), anns = lds_addr(&sh.annl[0][0]);
+  for (uint32_t rem = gmask; rem; rem &= rem - 1u) {
+    const int i = __builtin_ctz(rem);
+    const double4 q = gq[i];
+    const uint32_t ti = t0 + (uint32_t)i;
+    unsigned long long mc[NR], ma[NR];
+    int nc = 0, na = 0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      double ex, ey;
+      if constexpr (IMG) {
+        ex = (q.x + ox[r]) - x[r];
+        ey = (q.y + oy[r]) - y[r];
+      } else {
+        ex = q.x - x[r];
+        ey = q.y - y[r];
+      }
+      const double d2 = ex * ex + ey * ey;
+      // one comparison per ballot: combined on the scalar unit.  Every image
+      // of the query itself is excluded.
+      const unsigned long long other = ballot(j[r] != ti);
+      const unsigned long long in = ballot(d2 < q.z) & other;
+      ma[r] = ballot(d2 <= q.w) & other & ~in;
+      mc[r] = in;
+      nc += __popcll(mc[r]);
+      na += __popcll(ma[r]);
+    }
+    if (nc < k && na <= kAnn && nc + na >= k) {
+      uint32_t at = rows + (uint32_t)i * 68u;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(mc[r] >> 32),
+                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mc[r], at));
+        if (__builtin_amdgcn_inverse_ballot_w64(mc[r])) *lds_u8(pos) = (uint8_t)(r * 64 + lane);
+        at += (uint32_t)__popcll(mc[r]);
+      }
+      at = anns + (uint32_t)i * kAnn;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(ma[r] >> 32),
+                                 __builtin_amdgcn_mbcnt_lo((uint32_t)ma[r], at));
+        if (__builtin_amdgcn_inverse_ballot_w64(ma[r])) *lds_u8(pos) = (uint8_t)(r * 64 + lane);
+        at += (uint32_t)__popcll(ma[r]);
+      }
+    }
+    c_lo = ql == i ? nc : c_lo;
+    c_an = ql == i ? na : c_an;
+  }
+}
+
+// The k-th distance of a group's queries, and their rows completed: lane
+// (ql, part) holds four of query ql's annulus entries (e = 4 part + i).  The
+// k - c_lo smallest by (d2, entry) are taken; an exact tie at the k-th
+// distance is resolved by (ID, image order).  Returns tau in the four lanes
+// of each query, and counts the queries with a tie.
+template <bool IMG>
+__device__ inline double select_annulus(WalkShared& sh, bool ok, int k, int c_lo, int c_an,
+                                        double xq, double yq, double lx, double ly, int ql,
+                                        int part, const uint32_t* __restrict__ ID,
+                                        unsigned& nties) {
+  const int need = k - c_lo;
+  uint32_t slot[4];
+  double ad[4], nx[4];
+  {
+    const uint32_t ids = *(const uint32_t*)&sh.annl[ql][4 * part];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool in = ok && 4 * part + i < c_an;
+      slot[i] = in ? (ids >> (8 * i)) & 255u : 0u;
+      const double d2 = slot_d2<IMG>(sh, slot[i], xq, yq, lx, ly);
+      ad[i] = in ? d2 : INFINITY;
+      // the next double: x < next(d2) is x <= d2
+      nx[i] = __longlong_as_double(__double_as_longlong(ad[i]) + 1);
+      sh.u.ad[4 * part + i][ql] = ad[i];
+    }
+  }
+  wave_fence();
+  // entries before each in the order (d2, entry): those of earlier quarters
+  // up to and including its distance, the others below it; ties inside the
+  // quarter by place
+  int before[4] = {0, 0, 0, 0};
+  const int most = ballot(ok && c_an > 12) ? 4 : ballot(ok && c_an > 8) ? 3
+                 : ballot(ok && c_an > 4)  ? 2 : 1;
+  for (int f4 = 0; f4 < most; ++f4) {
+    const bool earlier = f4 < part;
+    const double th0 = earlier ? nx[0] : ad[0], th1 = earlier ? nx[1] : ad[1];
+    const double th2 = earlier ? nx[2] : ad[2], th3 = earlier ? nx[3] : ad[3];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const double v = sh.u.ad[4 * f4 + f][ql];
+      before[0] += v < th0;
+      before[1] += v < th1;
+      before[2] += v < th2;
+      before[3] += v < th3;
+    }
+  }
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+#pragma unroll
+    for (int f = 0; f < i; ++f) before[i] += ad[f] == ad[i];
+  double tau = -1.0;
+  bool sel[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    sel[i] = ok && 4 * part + i < c_an && before[i] < need;
+    if (sel[i]) sh.row[ql][c_lo + before[i]] = (uint8_t)slot[i];
+    tau = sel[i] && ad[i] > tau ? ad[i] : tau;
+  }
+  {
+    const double o1 = __shfl_xor(tau, 16, 64);
+    tau = o1 > tau ? o1 : tau;
+    const double o2 = __shfl_xor(tau, 32, 64);
+    tau = o2 > tau ? o2 : tau;
+  }
+  // an entry left out at exactly the k-th distance (the others left out lie
+  // beyond it)
+  bool tie = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) tie = tie || (ok && 4 * part + i < c_an && !sel[i] && ad[i] == tau);
+  const unsigned long long tied = ballot(tie);
+  if (tied) {
+    const uint32_t tq = (uint32_t)(tied | tied >> 16 | tied >> 32 | tied >> 48) & 0xFFFFu;
+    nties += __builtin_popcount(tq);
+    wave_fence();
+    if (part == 0 && ((tq >> ql) & 1u)) {
+      int below = 0;
+      for (int e = 0; e < c_an; ++e) below += sh.u.ad[e][ql] < tau ? 1 : 0;
+      // the slots after the entries below tau take the tied entries with the
+      // smallest (ID, image order)
+      uint64_t prev = 0;
+      bool first = true;
+      for (int p = c_lo + below; p < k; ++p) {
+        uint64_t best = ~0ull;
+        uint32_t bslot = 0;
+        for (int e = 0; e < c_an; ++e) {
+          if (sh.u.ad[e][ql] != tau) continue;
+          const uint32_t sl = sh.annl[ql][e], pk = sh.pk[sl];
+          const uint64_t key = ((uint64_t)ID[pk >> 4] << 4) | img_order(pk & 15u);
+          if ((first || key > prev) && key < best) {
+            best = key;
+            bslot = sl;
+          }
+        }
+        sh.row[ql][p] = (uint8_t)bslot;
+        prev = best;
+        first = false;
+      }
+    }
+  }
+  wave_fence();
+  return tau;
+}
+
+// The kernel sum over the k neighbours of a group's queries, and their rows'
+// entries to memory: lane (ql, part) takes every fourth chunk of four
+// entries of query ql's row, so that the 16 queries' chunks leave as 256
+// contiguous bytes.  Returns the sum in the four lanes of each query.
+template <bool FP32C, bool IMG, typename KT>
+__device__ inline double row_density(const WalkShared& sh, NbrRow row, int k, double tau, double xq,
+                                     double yq, double lx, double ly, int ql, int part) {
+  double acc = 0.0;
+  BlockKahan fk;
+  // FP32C: q^2 = d^2 / tau formed in FP64 before the FP32 square root: a
+  // rounded 1 / h shared by every term would move all q together, and a
+  // particle whose neighbours all sit near q = 1 would lose 1e-5 of its density
+  const double itau = FP32C ? 1.0 / tau : 0.0;
+  const double h = FP32C ? 0.0 : sqrt(tau), hinv = FP32C ? 0.0 : rcp64(h);
+  auto visit = [&](int ch, int n) {
+    const uint32_t ids = *(const uint32_t*)&sh.row[ql][4 * ch];
+    uint32_t pk[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool in = i < n;
+      const uint32_t sl = in ? (ids >> (8 * i)) & 255u : 0u;
+      pk[i] = sh.pk[sl];
+      const double d2 = slot_d2<IMG>(sh, sl, xq, yq, lx, ly);
+      if constexpr (FP32C) {
+        // the k-th neighbour's q may round to a few ulp past 1, where F is of
+        // order ulp^3 (no clamp needed)
+        const float f = KT::F(__builtin_amdgcn_sqrtf((float)(d2 * itau)));
+        fk.add(in ? f : 0.f);
+      } else {
+        const double f = KT::F64(sqrt_over(d2, h, hinv));
+        acc += in ? f : 0.0;
+      }
+    }
+    if constexpr (FP32C) fk.flush();
+    *row.chunk(ch) = u32x4{pk[0], pk[1], pk[2], pk[3]};
+  };
+  int ch = part;
+  for (; 4 * ch + 4 <= k; ch += 4) visit(ch, 4);
+  if (4 * ch < k) visit(ch, k - 4 * ch);
+  if constexpr (FP32C) acc = fk.value();
+  acc += __shfl_xor(acc, 16, 64);
+  acc += __shfl_xor(acc, 32, 64);
+  return acc;
+}
+
+// kNN + density + sound speed + force record of the queries that have an h
+// from the last pass.  A wave takes up to 64 consecutive (Hilbert-ordered)
+// queries, lane = query, and searches groups of 16 of them one after the
+// other:
+//
+//   box       the box around the group's search circles (radius
+//             h_prev (1 + delta)), in cells of the finest grid; the cells of
+//             the coarsest level that covers it with at most nsub x nsub
+//             cells are looked up one per lane
+//   stage     the cells' particles, 64 at a time, filtered against the box
+//             and packed into LDS (position, packed entry)
+//   classify  lane = candidate: per query, certain neighbours (nearer than
+//             h_prev (1 - delta)) and the annulus up to h_prev (1 + delta)
+//   select    lane = (query, quarter of its annulus): exact distances, the
+//             k-th distance
+//   density   lane = (query, every fourth chunk of its row): the kernel sum
+//             from the LDS positions, the row to memory
+//
+// A group whose cells hold more than 16 * split candidates, or whose box more
+// than kWalkCand, is halved (cell order can put two distant regions in one
+// group), down to single queries, whose candidates are filtered by their own
+// circle; those still too wide, queries without an h and queries whose bracket
+// misses go to the exact search (k_knn_fallback).
+//
+// What bounds it: vector issue, 77 % of all issue slots at 4M clustered, k = 64
+// (about 130 vector instructions per query; 1.28 GB written, 0.29 GB read).
+// One query's candidates side by side in the lanes need no per-query lists and
+// no lane waits for the longest of 64 lists, and a group of 16 queries is a
+// short chain of loads, so small launches finish early.  Against the walk with
+// a query per lane and its separate selection and density kernel that this
+// replaced: 4M FP32C 1.40 -> 1.17 ms, 1M FP64 0.45 -> 0.35 ms, 77,777 at k = 19
+// 108 -> 31 us, 2,200 at k = 32 55 -> 13 us.  One wave per block: a wave that
+// ends frees its LDS at once (1.54 -> 1.39 ms); 10 KiB per wave and four waves
+// per SIMD without a spilled register, where five spilled 40 (1.39 -> 1.17 ms).
+template <bool FP32C>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_knn(
     const Item* __restrict__ items, int nitems, const SimDev* __restrict__ sims,
-    const double2* __restrict__ XY,
-    const uint8_t* __restrict__ WR, const uint32_t* __restrict__ cstart,
-    double* __restrict__ H, const double* __restrict__ EP, const double* __restrict__ VPX,
-    const double* __restrict__ VPY, const uint32_t* __restrict__ ID,
-    uint32_t* __restrict__ nbr, int kstride, double* __restrict__ RHO,
-    double* __restrict__ C, void* __restrict__ recp, KnnStats* __restrict__ stats,
-    uint2* __restrict__ retry, uint32_t* __restrict__ retry_count,
-    uint32_t* __restrict__ cnt, uint32_t* __restrict__ ann, WalkKnobs kn,
-    uint32_t* __restrict__ walk_miss) {
-  constexpr int kSub = KSUB;       // sub-tiles of a wave
-  constexpr int kSubW = 64 / KSUB; // consecutive queries per sub-tile
-  __shared__ TileShared<KSUB> wsh[4];
-  const int item_idx = xcd_item(nitems);
+    const double2* __restrict__ XY, const uint8_t* __restrict__ WR,
+    const uint32_t* __restrict__ cstart, double* __restrict__ H, const double* __restrict__ EP,
+    const double* __restrict__ VPX, const double* __restrict__ VPY,
+    const uint32_t* __restrict__ ID, uint32_t* __restrict__ nbr, int kstride,
+    double* __restrict__ RHO, double* __restrict__ C, void* __restrict__ recp,
+    KnnStats* __restrict__ stats, uint2* __restrict__ retry, uint32_t* __restrict__ retry_count,
+    WalkKnobs kn, uint32_t* __restrict__ walk_miss, int wpi) {
+  __shared__ WalkShared sh;
+  const int lane0 = threadIdx.x;
+  // wpi blocks (of one wave) per item (4, 8 or 16), each taking 256 / wpi
+  // queries
+  const int blk = xcd_item(nitems * wpi);
+  const int item_idx = blk / wpi;
   const Item it = items[item_idx];
+  const int per = kItem / wpi;
+  const int w0 = (blk - item_idx * wpi) * per;
+  if (w0 >= it.count) return;
+  const int nq = it.count - w0 < per ? it.count - w0 : per;
   const SimDev* S = sims + it.sim;
-  const int wv = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  TileShared<KSUB>& ts = wsh[wv];
   const int k = S->k;
   const double lx = S->lx, ly = S->ly;
-  // per-lane outcomes, counted with ballots at the end (each lane once)
-  bool miss_lo = false, miss_hi = false, miss_ann = false, split_fb = false;
-
-  const int qi = wv * 64 + lane;
-  const bool valid = qi < it.count;
-  const int64_t t = it.first + (valid ? qi : 0);
-  const double2 pq = XY[t];
-  const double xq = pq.x, yq = pq.y;
-  const double hp = H[t];
-  const NbrRow row = nbr_row(nbr, t, kstride);
-  bool fast = !BITWISE && valid && hp > 0;
-  bool resolved = false;
-  double tau = 0.0;
-  if constexpr (!BITWISE) {
+  const int lg = S->lg;
+  const int raw_cap = kn.split * kGrp < kWalkRaw ? kn.split * kGrp : kWalkRaw;
+  // ---- this lane's own query ----
+  const bool valid = lane0 < nq;
+  const uint32_t tw = (uint32_t)(it.first + w0);
+  const uint32_t t = tw + (valid ? lane0 : 0);
+  unsigned long long can;
+  // the search circle's box in finest cells, widened by 1/64 of a cell (far
+  // beyond the rounding to float of at most 6 * 2^13 cells)
+  float qx0, qx1, qy0, qy1;
+  {
+    const double2 pq = XY[t];
+    const double hp = H[t];
     const double delta = S->walk_delta;
+    can = ballot(valid && hp > 0);
     const double Rlo = hp * (1 - delta), Rhi = hp * (1 + delta);
-    const double Rlo2 = Rlo * Rlo, Rhi2 = Rhi * Rhi;
     const double Rm = Rhi * (1 + 1e-12) + 1e-15 * (lx + ly);
-    int c_lo = 0, c_an = 0;
-    // certain neighbours collect in cbuf and leave in 16-byte stores
-    u32x4 cbuf = {0u, 0u, 0u, 0u};
-    u32x4* cptr = row.chunk(0);  // next chunk of the row to fill
-    const double xqm = xq - lx, xqp = xq + lx, yqm = yq - ly, yqp = yq + ly;
-    // annulus candidates go straight out, entry e of query t at
-    // tile(t) * 64 kAnn + 64 e + t % 64, so the lanes' writes of one entry
-    // index fill the same lines
-    uint32_t* annrow = ann + (t >> 6) * (int64_t)(64 * kAnn) + (t & 63);
-    // Lane groups: aligned blocks of consecutive queries.  A block whose
-    // box holds more than kn.split candidates per query is halved (cell
-    // order can put two distant regions in one wave); blocks below 8 lanes
-    // go to the wavefront search, which handles them at lower cost.
-    unsigned long long pending = ballot(fast);
-    const int gsz0 = kn.group;
-    int gsz = gsz0;
+    const double fx = (pq.x - S->x0) * S->ivx, fy = (pq.y - S->y0) * S->ivy;
+    const double rx = Rm * S->ivx + 0.015625, ry = Rm * S->ivy + 0.015625;
+    qx0 = (float)(fx - rx);
+    qx1 = -(float)(fx + rx);
+    qy0 = (float)(fy - ry);
+    qy1 = -(float)(fy + ry);
+    sh.q[lane0] = make_double4(pq.x, pq.y, Rlo * Rlo, Rhi * Rhi);
+  }
+  unsigned nties = 0;
+  const uint32_t table = kHilbertTable.w[lane0];
+  const uint32_t* cells = cstart + S->coff;
+
+  for (int g = 0; g * kGrp < nq; ++g) {
+    const uint32_t t0 = tw + (uint32_t)(g * kGrp);
+    double4* gq = sh.q + g * kGrp;
+    uint32_t pending = (uint32_t)(can >> (g * kGrp)) & 0xFFFFu;
+    int gsz = kGrp;
     while (pending) {
-      const int l0 = __builtin_ctzll(pending);
-      const int ga = l0 & ~(gsz - 1);
-      const bool grp = fast && ((pending >> lane) & 1ull) && lane >= ga && lane < ga + gsz;
-      const unsigned long long gm = ballot(grp);
-      double bx0 = grp ? xq - Rm : INFINITY, bx1 = grp ? xq + Rm : -INFINITY;
-      double by0 = grp ? yq - Rm : INFINITY, by1 = grp ? yq + Rm : -INFINITY;
-      for (int o = 32; o > 0; o >>= 1) {
-        bx0 = fmin(bx0, __shfl_xor(bx0, o, 64));
-        by0 = fmin(by0, __shfl_xor(by0, o, 64));
-        bx1 = fmax(bx1, __shfl_xor(bx1, o, 64));
-        by1 = fmax(by1, __shfl_xor(by1, o, 64));
+      // per iteration, so that no address made of it is kept in a register
+      // across the groups
+      int lane = lane0;
+      asm("" : "+v"(lane));
+      const int ql = lane & (kGrp - 1), part = lane >> 4;
+      const int l0 = __builtin_ctz(pending);
+      const uint32_t gmask = pending & (((1u << gsz) - 1u) << (l0 & ~(gsz - 1)));
+      const bool grp = (gmask >> ql) & 1u;  // of the row's query ql
+      auto row_box = [&](float v) {  // row g holds the group's own lanes
+        return __int_as_float(__builtin_amdgcn_readlane(
+            __float_as_int(row_min(grp ? v : INFINITY)), g * kGrp));
+      };
+      const float bx0 = row_box(qx0), bx1 = -row_box(qx1);
+      const float by0 = row_box(qy0), by1 = -row_box(qy1);
+      // cells of 2^s finest cells: the box spans at most nsub of them per axis
+      int s = 0;
+      {
+        const float m =
+            __builtin_fmaxf(bx1 - bx0, by1 - by0) * (kn.nsub == 4 ? 1.f / 2.99f : 1.f / 6.99f);
+        if (m > 1.f) s = __builtin_amdgcn_frexp_expf(m);
+        s = __builtin_amdgcn_readfirstlane(s < lg ? s : lg);
       }
-      const int c = level_for(S, bx1 - bx0, by1 - by0, 14.0);
-      const int64_t nc = 1LL << c;
-      const double icx = (double)nc / lx, icy = (double)nc / ly;
-      int64_t X0 = (int64_t)floor((bx0 - S->x0) * icx), X1 = (int64_t)floor((bx1 - S->x0) * icx);
-      int64_t Y0 = (int64_t)floor((by0 - S->y0) * icy), Y1 = (int64_t)floor((by1 - S->y0) * icy);
+      const int c = lg - s, nc = 1 << c;
+      const float down = __int_as_float((127 - s) << 23);  // 2^-s
+      int64_t X0 = (int)floorf(bx0 * down), X1 = (int)floorf(bx1 * down);
+      int64_t Y0 = (int)floorf(by0 * down), Y1 = (int)floorf(by1 * down);
       clamp_span(X0, X1, nc, S->open & 1);
       clamp_span(Y0, Y1, nc, S->open & 2);
-      const int nX = (int)(X1 - X0 + 1), nY = (int)(Y1 - Y0 + 1);
-      const int ncell = nX * nY;
-      int npieces = 0, ncand = 0;
-      for (int cb = 0; cb < ncell; cb += 64) {
-        const int ci = cb + lane;
-        bool have = false;
-        uint32_t pa = 0, pb = 0;
-        int tx = 0, ty = 0;
-        if (ci < ncell) {
-          const int64_t Xc = X0 + ci % nX, Yc = Y0 + ci / nX;
-          tx = (int)floordiv_pow2(Xc, c);
-          ty = (int)floordiv_pow2(Yc, c);
-          cell_range(S, cstart, c, (uint32_t)(Xc - tx * nc), (uint32_t)(Yc - ty * nc), pa, pb);
-          have = pb > pa;
-        }
-        const unsigned long long m = ballot(have);
-        const int len = have ? (int)(pb - pa) : 0;
-        const int incl = wave_incl_scan(len);
-        if (have) {
-          const int pos = npieces + lane_prefix(m);
-          ts.pst[pos] = pa;
-          ts.ppref[pos] = ncand + incl - len;
-          ts.ptx[pos] = (int8_t)tx;
-          ts.pty[pos] = (int8_t)ty;
-        }
-        npieces += __popcll(m);
-        ncand += __shfl(incl, 63, 64);
+      uint32_t pa = 0, pb = 0;
+      const int xc = (int)X0 + (lane & 7), yc = (int)Y0 + (lane >> 3);
+      const int tx = xc >> c, ty = yc >> c;
+      const uint32_t hix =
+          hilbert_lookup(table, (uint32_t)(xc & (nc - 1)), (uint32_t)(yc & (nc - 1)), c);
+      if ((lane & 7) <= (int)(X1 - X0) && (lane >> 3) <= (int)(Y1 - Y0)) {
+        const uint32_t* p = cells + ((uint64_t)hix << (2 * s));
+        pa = p[0];
+        pb = p[1ull << (2 * s)];
       }
-      npieces = __builtin_amdgcn_readfirstlane(npieces);
-      ncand = __builtin_amdgcn_readfirstlane(ncand);
-      const int gs = __popcll(gm);
-      if (ncand > kn.split * gs) {
-        if (gsz > 8) {
+      const int len = (int)(pb - pa);
+      const int incl = (int)scan_add((uint32_t)len);
+      const int nraw = __builtin_amdgcn_readlane(incl, 63);
+      int ncand = 0;
+      unsigned long long images = 0ull;
+      // a single query's candidates are filtered by its own circle below
+      bool fits = nraw <= (gsz > 1 ? raw_cap : kWalkRaw);
+      if (fits) {
+        wave_fence();
+        ((u32x4*)sh.u.s.mark)[lane] = u32x4{0u, 0u, 0u, 0u};
+        wave_fence();
+        if (len > 0) {
+          sh.u.s.mark[incl - len] = (uint8_t)(lane + 1);
+          sh.u.s.piece[lane] = make_uint2(pa - (uint32_t)(incl - len),
+                                          (uint32_t)((tx + 2) | ((ty + 2) << 3)));
+        }
+        wave_fence();
+        const double gw = (double)S->gx;
+        const double dbx0 = bx0, dbx1 = bx1, dby0 = by0, dby1 = by1;
+        uint32_t carry = 0;
+        // four rounds' positions are loaded before the first is used
+        for (int base = 0; base < nraw && ncand <= kWalkCand; base += 64 * kWalkRounds) {
+          uint32_t j[kWalkRounds], tile[kWalkRounds];
+          double2 pj[kWalkRounds];
+          uint8_t wc[kWalkRounds];
+#pragma unroll
+          for (int r = 0; r < kWalkRounds; ++r) {
+            if (base + r * 64 < nraw) {  // uniform
+              const int u = base + r * 64 + lane < nraw ? base + r * 64 + lane : nraw - 1;
+              // the last mark at or before u: lanes past the end see u's own,
+              // which the scan has passed already
+              const uint32_t sc = scan_max((uint32_t)sh.u.s.mark[u]);
+              const uint32_t id = sc > carry ? sc : carry;
+              carry = readlane_u(id, 63);
+              const uint2 pc = sh.u.s.piece[id - 1];
+              j[r] = pc.x + (uint32_t)u;
+              tile[r] = pc.y;
+              wc[r] = WR[j[r]];
+              pj[r] = XY[j[r]];
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < kWalkRounds; ++r) {
+            const int rest = nraw - base - r * 64;
+            if (rest > 0) {
+              unsigned long long in = rest >= 64 ? ~0ull : (1ull << rest) - 1ull;
+              double px = (pj[r].x - S->x0) * S->ivx;
+              double py = (pj[r].y - S->y0) * S->ivy;
+              uint32_t pk = (j[r] << 4) | 5u;
+              // a particle in the search's own tile is seen directly
+              const unsigned long long im = ballot(wc[r] != tile[r]);
+              if (im) {
+                int ix, iy;
+                const bool vis = cand_image((int)(tile[r] & 7u) - 2, (int)(tile[r] >> 3) - 2, wc[r],
+                                            ix, iy);
+                px -= (double)ix * gw;
+                py -= (double)iy * gw;
+                pk = (j[r] << 4) | img_code(ix, iy);
+                in &= ballot(vis);
+              }
+              in &= ballot(px >= dbx0) & ballot(px <= dbx1) & ballot(py >= dby0) & ballot(py <= dby1);
+              if (gsz == 1) {
+                const double4 q = gq[l0];
+                const double ex = q.x - (pj[r].x - (double)img_ix(pk & 15u) * lx);
+                const double ey = q.y - (pj[r].y - (double)img_iy(pk & 15u) * ly);
+                in &= ballot(ex * ex + ey * ey <= q.w * (1 + 1e-9));
+              }
+              images |= in & im;
+              const int pos = ncand + lane_prefix(in);
+              ncand += __popcll(in);
+              if (ncand <= kWalkCand) {
+                if (__builtin_amdgcn_inverse_ballot_w64(in)) {
+                  sh.xy[pos] = pj[r];
+                  sh.pk[pos] = pk;
+                }
+              } else {
+                ncand = kWalkCand + 1;
+              }
+            }
+          }
+        }
+        fits = ncand <= kWalkCand;
+      }
+      if (!fits) {
+        if (gsz > 1) {
           gsz >>= 1;
         } else {
-          if (grp) {
-            fast = false;
-            split_fb = true;
-          }
-          pending &= ~gm;
-          gsz = gsz0;
+          if (grp && part == g) gq[ql].z = kMissWide;
+          pending &= ~gmask;
+          gsz = kGrp;
         }
-        __builtin_amdgcn_wave_barrier();
         continue;
       }
-      if (lane == 0) ts.ppref[npieces] = ncand;
-      {
-        // boxes of the sub-tiles (kSubW consecutive queries each)
-        double sx0 = grp ? xq - Rm : INFINITY, sx1 = grp ? xq + Rm : -INFINITY;
-        double sy0 = grp ? yq - Rm : INFINITY, sy1 = grp ? yq + Rm : -INFINITY;
-        for (int o = kSubW >> 1; o > 0; o >>= 1) {
-          sx0 = fmin(sx0, __shfl_xor(sx0, o, 64));
-          sy0 = fmin(sy0, __shfl_xor(sy0, o, 64));
-          sx1 = fmax(sx1, __shfl_xor(sx1, o, 64));
-          sy1 = fmax(sy1, __shfl_xor(sy1, o, 64));
-        }
-        if ((lane & (kSubW - 1)) == 0) {
-          ts.sbb[lane / kSubW][0] = sx0;
-          ts.sbb[lane / kSubW][1] = sx1;
-          ts.sbb[lane / kSubW][2] = sy0;
-          ts.sbb[lane / kSubW][3] = sy1;
-        }
-        if (lane == 0) {
-          ts.sxy[64] = make_double2(NAN, NAN);
-          ts.spk[64] = 0u;
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-      const int my_sub = lane / kSubW;
-      double sbx0[kSub], sbx1[kSub], sby0[kSub], sby1[kSub];
-#pragma unroll
-      for (int g = 0; g < kSub; ++g) {
-        sbx0[g] = readlane_d(ts.sbb[g][0], 0);
-        sbx1[g] = readlane_d(ts.sbb[g][1], 0);
-        sby0[g] = readlane_d(ts.sbb[g][2], 0);
-        sby1[g] = readlane_d(ts.sbb[g][3], 0);
-      }
-      int nsteps = 0;
-      while ((1 << nsteps) < npieces) ++nsteps;
-      ts.selfm[lane] = 0ull;
-      const int64_t wave_t0 = it.first + (int64_t)wv * 64;
-      // Stage s takes every nst-th candidate (lane l: candidate l * nst + s),
-      // so each stage samples the whole box evenly and the eight sub-tile
-      // lists come out about equally long: every lane runs the longest one.
-      const int nst = (ncand + 63) >> 6;
-      // piece of this lane's candidate: a binary search for the first
-      // stage, then (candidate u + 1 after u, every piece non-empty) at most
-      // one step forward per stage
-      int lo = 0;
-      {
-        const int u0 = lane * nst;
-        if (u0 < ncand) {
-          int hi = npieces - 1;
-          for (int s = 0; s < nsteps; ++s) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (ts.ppref[mid] <= u0) lo = mid; else hi = mid - 1;
-          }
-        }
-      }
-      for (int base = 0; base < ncand; base += 64) {
-        // stage 64 candidates
-        const int u = lane * nst + (base >> 6);
-        double cxv = NAN, cyv = 0.0;
-        uint32_t cpk = 0;
-        bool interior = true;
-        if (u < ncand) {
-          if (ts.ppref[lo + 1] <= u) ++lo;
-          const uint32_t j = ts.pst[lo] + (uint32_t)(u - ts.ppref[lo]);
-          int ix, iy;
-          if (cand_image(ts.ptx[lo], ts.pty[lo], WR[j], ix, iy)) {
-            const double2 pj = XY[j];
-            cxv = pj.x;
-            cyv = pj.y;
-            interior = (ix == 0) && (iy == 0);
-          }
-          cpk = (j << 4) | img_code(ix, iy);
-          // an image of one of this wave's own queries: mark it in that
-          // query's self mask (ordered after the query's own clear below)
-          const int64_t so = (int64_t)j - wave_t0;
-          if (so >= 0 && so < 64) atomicOr(&ts.selfm[so], 1ull << lane);
-        }
-        ts.sxy[lane] = make_double2(cxv, cyv);
-        ts.spk[lane] = cpk;
-        const bool all_interior = ballot(interior) == ~0ull;
-        // per sub-tile, the staged candidates inside its box (in stage order)
-        int nm = 0;
-        {
-          const double px = cxv - (double)img_ix(cpk & 15u) * lx;
-          const double py = cyv - (double)img_iy(cpk & 15u) * ly;
-#pragma unroll
-          for (int g = 0; g < kSub; ++g) ts.slist[g][lane] = 64;
-#pragma unroll
-          for (int g = 0; g < kSub; ++g) {
-            const bool in = px >= sbx0[g] && px <= sbx1[g] && py >= sby0[g] && py <= sby1[g];
-            const unsigned long long m = ballot(in);
-            if (in) {
-              const int pos = lane_prefix(m);
-              ts.slist[g][pos] = (uint8_t)lane;
-              ts.slpk[g][pos] = cpk;
-            }
-            if (lane == 0) ts.smask[g] = m;
-            const int c = __popcll(m);
-            nm = c > nm ? c : nm;
-          }
-        }
-        __builtin_amdgcn_wave_barrier();
-        nm = (__builtin_amdgcn_readfirstlane(nm) + 3) & ~3;
-        const uint8_t* mylist = ts.slist[my_sub];
-        const uint32_t* mypk = ts.slpk[my_sub];
-        // list positions of this query's own images (every image of the
-        // query itself is excluded): a staged slot u in the sub-tile's list
-        // sits at the count of list slots below u
-        unsigned long long spos = 0ull;
-        {
-          const unsigned long long msub = ts.smask[my_sub];
-          unsigned long long sm = ts.selfm[lane] & msub;
-          ts.selfm[lane] = 0ull;
-          while (sm) {
-            const int us = __builtin_ctzll(sm);
-            sm &= sm - 1ull;
-            spos |= 1ull << __popcll(msub & ((1ull << us) - 1ull));
-          }
-        }
-        // Blocks of 32 list positions: first every lane classifies its
-        // candidates into bit masks, shifting one bit per position into
-        // each (certain: inside Rlo, reach: up to Rhi), then emits the set
-        // bits in list order.  Certain neighbours shift through a 4-entry
-        // register buffer (oldest in x) that leaves as one 16-byte chunk
-        // store every fourth entry.
-        for (int mb = 0; mb < nm; mb += 32) {
-          const int mend = nm < mb + 32 ? nm : mb + 32;
-          uint32_t cmask = 0u, hmask = 0u;
-// One position: compare into VCC, then add-with-carry mask + mask + VCC
-// shifts the bit in (one instruction per mask where the compiler emits a
-// select and a shift-or).  s_nop 1 gives the two wait states an FP64
-// compare's VCC write needs before a VALU reads it.
-#define SPH_CLASSIFY(D2)                                                                \
-  {                                                                                     \
-    const double d2v_ = (D2);                                                           \
-    asm("v_cmp_lt_f64 vcc, %1, %2\n\ts_nop 1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"         \
-        : "+v"(cmask) : "v"(d2v_), "v"(Rlo2) : "vcc");                                  \
-    asm("v_cmp_le_f64 vcc, %1, %2\n\ts_nop 1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"         \
-        : "+v"(hmask) : "v"(d2v_), "v"(Rhi2) : "vcc");                                  \
+      wave_fence();
+      int c_lo = 0, c_an = 0;
+      const double xq = gq[ql].x, yq = gq[ql].y;
+      const int nr = (ncand + 63) >> 6;
+#define SPH_CLASSIFY(NR)                                                                        \
+  {                                                                                             \
+    if (images) classify<NR, true>(sh, gq, ncand, gmask, t0, k, lx, ly, lane, c_lo, c_an);          \
+    else classify<NR, false>(sh, gq, ncand, gmask, t0, k, lx, ly, lane, c_lo, c_an);                \
   }
-          if (all_interior) {
-            for (int m = mb; m < mend; m += 4) {
-              const uint32_t i4 = *(const uint32_t*)(mylist + m);
-              const uint32_t i0 = i4 & 255u, i1 = (i4 >> 8) & 255u, i2 = (i4 >> 16) & 255u,
-                             i3 = i4 >> 24;
-              const double2 e0 = ts.sxy[i0], e1 = ts.sxy[i1], e2 = ts.sxy[i2], e3 = ts.sxy[i3];
-              const double a0 = xq - e0.x, b0 = yq - e0.y;
-              const double a1 = xq - e1.x, b1 = yq - e1.y;
-              const double a2 = xq - e2.x, b2 = yq - e2.y;
-              const double a3 = xq - e3.x, b3 = yq - e3.y;
-              SPH_CLASSIFY(a0 * a0 + b0 * b0);
-              SPH_CLASSIFY(a1 * a1 + b1 * b1);
-              SPH_CLASSIFY(a2 * a2 + b2 * b2);
-              SPH_CLASSIFY(a3 * a3 + b3 * b3);
-            }
-          } else {
-            for (int m = mb; m < mend; ++m) {
-              const uint32_t im = mylist[m];
-              const uint32_t pk = ts.spk[im];
-              const int ix = img_ix(pk & 15u), iy = img_iy(pk & 15u);
-              const double ax = ix == 0 ? xq : (ix < 0 ? xqm : xqp);
-              const double ay = iy == 0 ? yq : (iy < 0 ? yqm : yqp);
-              const double2 e = ts.sxy[im];
-              const double ex = ax - e.x;
-              const double ey = ay - e.y;
-              SPH_CLASSIFY(ex * ex + ey * ey);
-            }
-          }
+      if (nr == 3) SPH_CLASSIFY(3)
+      else if (nr == 4) SPH_CLASSIFY(4)
+      else if (nr == 2) SPH_CLASSIFY(2)
+      else SPH_CLASSIFY(1)
 #undef SPH_CLASSIFY
-          // position m of the block was shifted in at bit mend - 1 - m;
-          // reversed and shifted down, it sits at bit m - mb
-          const int sh = 32 - (mend - mb);
-          const uint32_t keep = grp ? ~(uint32_t)(spos >> mb) : 0u;
-          cmask = (__builtin_bitreverse32(cmask) >> sh) & keep;
-          uint32_t amask = (__builtin_bitreverse32(hmask) >> sh) & keep & ~cmask;
-          // the entries of the block's positions, read once per emitted bit
-          const uint32_t* blpk = mypk + mb;
-          while (cmask) {
-            const uint32_t pk = blpk[__builtin_ctz(cmask)];
-            cmask &= cmask - 1u;
-            cbuf.x = cbuf.y;
-            cbuf.y = cbuf.z;
-            cbuf.z = cbuf.w;
-            cbuf.w = pk;
-            if ((c_lo & 3) == 3 && c_lo < k) {
-              *cptr = cbuf;
-              cptr += 64;
+      wave_fence();
+      const bool ok = grp && c_lo < k && c_an <= kAnn && c_lo + c_an >= k;
+      auto finish = [&](auto img) {
+        constexpr bool IMG = decltype(img)::value;
+        const double tau =
+            select_annulus<IMG>(sh, ok, k, c_lo, c_an, xq, yq, lx, ly, ql, part, ID, nties);
+        if (ok) {
+          const NbrRow row = nbr_row(nbr, (int64_t)t0 + ql, kstride);
+          double facc = 0.0;
+          kern_visit(S->kernel, [&](auto kt) {
+            facc = row_density<FP32C, IMG, decltype(kt)>(sh, row, k, tau, xq, yq, lx, ly, ql, part);
+            // FP32C: a rounding of q of 2^-24 moves F(q) ~ (1 - q)^3 by
+            // 3 q / (1 - q) times that, at most 2^-24 2.1 (k / sum)^(1/3) of
+            // the sum: beyond 6e-6 where 64 terms add to less than kThinSum
+            // (every neighbour near q = 1: the edge of a compact clump, tiny
+            // k).  Those few are summed in FP64.
+            if constexpr (FP32C) {
+              if (facc < kThinSum)
+                facc = row_density<false, IMG, decltype(kt)>(sh, row, k, tau, xq, yq, lx, ly, ql, part);
             }
-            ++c_lo;
-          }
-          while (amask) {
-            const uint32_t pk = blpk[__builtin_ctz(amask)];
-            amask &= amask - 1u;
-            if (c_an < kAnn) annrow[64 * c_an] = pk;
-            ++c_an;
+          });
+          if (part == 0) {
+            gq[ql].z = tau;
+            gq[ql].w = facc;
           }
         }
-        __builtin_amdgcn_wave_barrier();
-      }
-      pending &= ~gm;
-      gsz = gsz0;
+      };
+      if (images) finish(std::true_type{}); else finish(std::false_type{});
+      if (grp && !ok && part == 0)
+        gq[ql].z = c_lo >= k ? kMissLo : (c_an > kAnn ? kMissAnn : kMissHi);
+      pending &= ~gmask;
+      gsz = kGrp;
     }
-    // hand the resolvable queries to k_knn_finish: certain neighbours are
-    // in the row, annulus candidates go to `ann`
-    if (fast) {
-      miss_lo = c_lo >= k;
-      miss_ann = !miss_lo && c_an > kAnn;
-      miss_hi = !miss_lo && !miss_ann && c_lo + c_an < k;
-    }
-    if (fast && c_lo < k && c_an <= kAnn && c_lo + c_an >= k) {
-      // the last c_lo % 4 certain entries sit at the top of the buffer
-      const int rem = c_lo & 3;
-      if (rem) {
-        uint32_t* r0 = &row[c_lo & ~3];
-        if (rem == 1) {
-          r0[0] = cbuf.w;
-        } else if (rem == 2) {
-          r0[0] = cbuf.z;
-          r0[1] = cbuf.w;
-        } else {
-          r0[0] = cbuf.y;
-          r0[1] = cbuf.z;
-          r0[2] = cbuf.w;
-        }
-      }
-      resolved = true;
-    }
-    if (valid) cnt[t] = resolved ? ((uint32_t)c_lo | ((uint32_t)c_an << 8)) : 0xFFFFFFFFu;
   }
-  // misses go to the retry list, searched by k_knn_fallback
-  const bool need = valid && !resolved;
-  const unsigned long long m = ballot(need);
+  wave_fence();
+  const double4 out = sh.q[lane0];
+  const bool tried = (can >> lane0) & 1ull;
+  const bool resolved = tried && out.z >= 0.0;
+  if (resolved)
+    write_result<FP32C>(S, t, out.x, out.y, out.z, out.w, EP, VPX, VPY, H, RHO, C, recp);
+  // what is left goes to the exact search
+  const bool left = valid && !resolved;
+  const unsigned long long m = ballot(left);
   if (m) {
     uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(retry_count, (uint32_t)__popcll(m));
+    if (lane0 == 0) base = atomicAdd(retry_count, (uint32_t)__popcll(m));
     base = readlane_u(base, 0);
-    if (need) retry[base + lane_prefix(m)] = make_uint2((uint32_t)t, (uint32_t)item_idx);
+    if (left) retry[base + lane_prefix(m)] = make_uint2(t, (uint32_t)item_idx);
   }
   // counters: queries with an h that needed the exact search, and why
-  const unsigned long long nfall = __popcll(m & ballot(hp > 0));
-  const unsigned long long nlo = __popcll(ballot(miss_lo)), nhi = __popcll(ballot(miss_hi));
-  const unsigned long long nann = __popcll(ballot(miss_ann)), nsplit = __popcll(ballot(split_fb));
-  if (lane == 0) {
+  const unsigned nfall = __popcll(m & can);
+  const unsigned nlo = __popcll(can & ballot(out.z == kMissLo));
+  const unsigned nann = __popcll(can & ballot(out.z == kMissAnn));
+  const unsigned nhi = __popcll(can & ballot(out.z == kMissHi));
+  const unsigned nsplit = __popcll(can & ballot(out.z == kMissWide));
+  if (lane0 == 0) {
     // the simulation's bracket misses (k_reduce adapts its delta)
     uint32_t* ms = walk_miss + ((int64_t)it.sim * kMissSlots + (blockIdx.x & (kMissSlots - 1))) *
                                    kMissStride;
-    if (nlo + nhi) atomicAdd(ms, (uint32_t)(nlo + nhi));
-    if (nann) atomicAdd(ms + 1, (uint32_t)nann);
+    if (nlo + nhi) atomicAdd(ms, nlo + nhi);
+    if (nann) atomicAdd(ms + 1, nann);
     KnnStats* sp = stat_slot(stats);
     stat_add(&sp->retries, nfall);
+    stat_add(&sp->ties, nties);
     stat_add(&sp->miss_lo, nlo);
     stat_add(&sp->miss_hi, nhi);
     stat_add(&sp->miss_ann, nann);
     stat_add(&sp->split_fallback, nsplit);
   }
+}
+
+// Waves per item of the walk: each takes group / 16 groups of queries, and
+// where that would leave fewer than 16384 waves (four per SIMD resident on
+// 1024 SIMDs, four rounds of them) down to one group each, so that a small
+// launch is as short as one group's search.  Results do not depend on it (a
+// group's search knows nothing of the others).
+inline int walk_waves_per_item(int nitems, int group) {
+  int wpi = 4 * (64 / group);
+  while (wpi < 16 && (int64_t)nitems * wpi < 16384) wpi *= 2;
+  return wpi;
 }
 
 // Byte offset of record j of an array of T, from a packed entry
@@ -1363,205 +1624,6 @@ __device__ inline void row_visit(const NbrRow row, int k, uint32_t self, const S
   }
 }
 
-// Block-compensated FP32 sum: the terms of one round (4 or 8 neighbours)
-// add up plainly, and each round's partial joins the running sum through a
-// Kahan step.  Besides the compensated sum's own error this adds at most
-// (B - 1) 2^-24 of the sum of |terms| of a block of B, against four
-// operations per term for a Kahan step per term.
-struct BlockKahan {
-  float s = 0.f, c = 0.f, p = 0.f;
-  __device__ void add(float t) { p += t; }
-  __device__ void add_mul(float a, float b) { p = __builtin_fmaf(a, b, p); }
-  __device__ void flush() {
-    const float y = p - c;
-    const float tt = s + y;
-    c = (tt - s) - y;
-    s = tt;
-    p = 0.f;
-  }
-  __device__ double value() const { return (double)s - (double)c; }
-};
-
-// Completes the fast-path queries: the r = k - c_lo smallest annulus
-// candidates by (d2, ID, image) fill the row, then density, sound speed and
-// the force record.  One thread per query.
-template <bool FP32C>
-__global__ __launch_bounds__(256) void k_knn_finish(
-    const Item* __restrict__ items, int nitems, const SimDev* __restrict__ sims,
-    const double2* __restrict__ XY, const uint2* __restrict__ UXY, double* __restrict__ H,
-    const double* __restrict__ EP, const double* __restrict__ VPX,
-    const double* __restrict__ VPY, const uint32_t* __restrict__ ID, uint32_t* __restrict__ nbr,
-    int kstride, double* __restrict__ RHO, double* __restrict__ C, void* __restrict__ recp,
-    const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ ann,
-    KnnStats* __restrict__ stats) {
-  const Item it = items[xcd_item(nitems)];
-  const int lane = threadIdx.x & 63;
-  const bool valid = (int)threadIdx.x < it.count;
-  const int64_t t = it.first + (valid ? threadIdx.x : 0);
-  const uint32_t cp = cnt[t];
-  // the block's window of positions in LDS for the density sums, slots
-  // [first - 128, first + 384) (most neighbours of Hilbert-ordered queries)
-  constexpr int kWin = 512;
-  constexpr int kBack = 128;
-  __shared__ double2 wxy[kWin];
-  __shared__ uint2 wuxy[FP32C ? kWin : 1];
-  const int64_t wb = it.first - kBack;
-  {
-    const SimDev* S = sims + it.sim;
-    if constexpr (FP32C) stage_window<uint2, kWin>(wuxy, UXY, wb, S->off, S->off + S->n);
-    else stage_window<double2, kWin>(wxy, XY, wb, S->off, S->off + S->n);
-    __syncthreads();
-  }
-  const WinSrc<double2, kWin> xys{XY, wxy, (uint32_t)wb};
-  const WinSrc<uint2, FP32C ? kWin : 1> uxys{UXY, wuxy, (uint32_t)wb};
-  unsigned long long nties = 0;
-  if (valid && cp != 0xFFFFFFFFu) {
-    const SimDev* S = sims + it.sim;
-    const int k = S->k;
-    const double lx = S->lx, ly = S->ly;
-    const int c_lo = (int)(cp & 255u), c_an = (int)((cp >> 8) & 255u);
-    const int r = k - c_lo;
-    const double2 pq = XY[t];
-    const double xq = pq.x, yq = pq.y;
-    const NbrRow row = nbr_row(nbr, t, kstride);
-    // annulus squared distances, recomputed exactly as in the walk; slots
-    // from c_an on stand for the query itself at infinite distance, after
-    // every entry.  Every query owns kAnn annulus slots, so FP32C reads all
-    // of them unconditionally (no load waits behind a branch; the unused
-    // ones hold stale values); FP64, whose density loop holds more registers,
-    // keeps the occupancy of reading only the c_an it has.
-    const uint32_t* ai = ann + (t >> 6) * (int64_t)(64 * kAnn) + (t & 63);  // stride 64
-    const uint32_t self_pk = ((uint32_t)t << 4) | 5u;
-    uint32_t ap[kAnn];
-    double ad[kAnn];
-#pragma unroll
-    for (int e = 0; e < kAnn; ++e) {
-      if constexpr (FP32C) {
-        const uint32_t raw = ai[64 * e];
-        ap[e] = e < c_an ? raw : self_pk;
-      } else {
-        ap[e] = e < c_an ? ai[64 * e] : self_pk;
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < kAnn; ++e) {
-      const uint32_t pk = ap[e];
-      const double2 pj = XY[pk >> 4];
-      // p_i + (-L) rounds as the walk's p_i - L, and p_i + 0 is p_i
-      const double ax = xq + (double)img_ix(pk & 15u) * lx;
-      const double ay = yq + (double)img_iy(pk & 15u) * ly;
-      const double ex = ax - pj.x, ey = ay - pj.y;
-      if constexpr (FP32C) {
-        const double d2 = ex * ex + ey * ey;
-        ad[e] = e < c_an ? d2 : INFINITY;
-      } else {
-        ad[e] = e < c_an ? ex * ex + ey * ey : INFINITY;
-      }
-    }
-    // the r smallest by (d2, slot): entry e is taken when fewer than r
-    // entries precede it in that order, and goes to row position c_lo plus
-    // that count (a fixed 16 x 15 comparisons, where a selection loop runs
-    // as often as the largest r of the wave)
-    double tau = -1.0;
-    uint32_t taken = 0u;
-#pragma unroll
-    for (int e = 0; e < kAnn; ++e) {
-      int before = 0;
-#pragma unroll
-      for (int f = 0; f < kAnn; ++f)
-        if (f != e) before += (f < e ? ad[f] <= ad[e] : ad[f] < ad[e]) ? 1 : 0;
-      if (e < c_an && before < r) {
-        row[c_lo + before] = ap[e];
-        tau = ad[e] > tau ? ad[e] : tau;
-        taken |= 1u << e;
-      }
-    }
-    // an annulus entry left out with d2 == tau: resolve the tie exactly
-    bool tie = false;
-#pragma unroll
-    for (int e = 0; e < kAnn; ++e)
-      tie = tie || (e < c_an && !((taken >> e) & 1u) && ad[e] == tau);
-    if (tie) {
-      ++nties;
-      int below = 0;
-#pragma unroll
-      for (int e = 0; e < kAnn; ++e) below += ad[e] < tau ? 1 : 0;
-      // the k - c_lo - below slots after the entries below tau take the
-      // tied entries with the smallest (ID, image order)
-      uint64_t prev = 0;
-      bool first = true;
-      for (int s_ = c_lo + below; s_ < k; ++s_) {
-        uint64_t best = ~0ull;
-        uint32_t bpk = 0;
-        for (int e = 0; e < c_an; ++e) {
-          if (ad[e] != tau) continue;
-          const uint64_t key = ((uint64_t)ID[ap[e] >> 4] << 4) | img_order(ap[e] & 15u);
-          if ((first || key > prev) && key < best) {
-            best = key;
-            bpk = ap[e];
-          }
-        }
-        row[s_] = bpk;
-        prev = best;
-        first = false;
-      }
-    }
-    // density over the row's k neighbours
-    const double h = sqrt(tau);
-    const int kern = S->kernel;
-    double facc;
-    if constexpr (FP32C) {
-      BlockKahan acc;
-      kern_visit(kern, [&](auto kt) {
-        using KT = decltype(kt);
-        // q of the k-th neighbour may round to a few ulp past 1, where F is
-        // of order ulp^3 (no clamp needed)
-        auto kahan = [&](float q) { acc.add(KT::F(q)); };
-        auto flush = [&]() { acc.flush(); };
-        // displacements from the fixed-point positions (the minimum image,
-        // exact to L / 2^32) while every neighbour lies within half a box,
-        // scaled straight to units of h; otherwise from the FP64 positions.
-        // Square roots in hardware (within 1 ulp): the FP32 form's error
-        // budget holds them.
-        if (fixed_point_ok(h, lx, ly)) {
-          const uint2 me = UXY[t];
-          const float gx = (float)(lx * 0x1p-32 / h), gy = (float)(ly * 0x1p-32 / h);
-          const float cx = centred_step(xq, S->x0, lx) * gx, cy = centred_step(yq, S->y0, ly) * gy;
-          row_visit<8>(row, k, (uint32_t)t, uxys, [&](uint32_t, uint2 pj) {
-#pragma clang fp contract(fast)
-            const float ex = __builtin_fmaf((float)(int32_t)(pj.x - me.x), gx, cx);
-            const float ey = __builtin_fmaf((float)(int32_t)(pj.y - me.y), gy, cy);
-            kahan(__builtin_amdgcn_sqrtf(__builtin_fmaf(ey, ey, ex * ex)));
-          }, flush);
-        } else {
-          // q^2 in FP64 before the FP32 square root (see wave_search)
-          const double itau = 1.0 / tau;
-          row_visit<8>(row, k, (uint32_t)t, ArrSrc<double2>{XY}, [&](uint32_t pk, double2 pj) {
-            const double ex = (xq + (double)img_ix(pk & 15u) * lx) - pj.x;
-            const double ey = (yq + (double)img_iy(pk & 15u) * ly) - pj.y;
-            kahan(__builtin_amdgcn_sqrtf((float)((ex * ex + ey * ey) * itau)));
-          }, flush);
-        }
-      });
-      facc = acc.value();
-    } else {
-      double acc = 0.0;
-      const double hinv64 = 1.0 / h;
-      row_visit<8>(row, k, (uint32_t)t, xys, [&](uint32_t pk, double2 pj) {
-#pragma clang fp contract(fast)
-        const double ex = (xq + (double)img_ix(pk & 15u) * lx) - pj.x;
-        const double ey = (yq + (double)img_iy(pk & 15u) * ly) - pj.y;
-        const double d2 = ex * ex + ey * ey;
-        acc += kern_F_fma(kern, (d2 * rsq64(d2)) * hinv64);
-      });
-      facc = acc;
-    }
-    write_result<FP32C>(S, t, xq, yq, tau, facc, EP, VPX, VPY, H, RHO, C, recp);
-  }
-  for (int o = 32; o > 0; o >>= 1) nties += __shfl_xor(nties, o, 64);
-  if (lane == 0) stat_add(&stat_slot(stats)->ties, nties);
-}
-
 // Exact wavefront search for the queries of the retry list (or, in
 // all-queries mode, for every particle: first pass and bitwise order).
 // Waves stride over the list, so the slow searches spread over the GPU.
@@ -1604,7 +1666,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const double xq = pq.x, yq = pq.y, hp = H[t];
     const double R0 = hp > 0 ? hp * 1.1 : local_radius(S, cstart, xq, yq);
     const unsigned long long nfail0 = nfail;
-    const SearchOut so = wave_search<BITWISE, FP32C>(S, t, xq, yq, R0, XY, WR, cstart, ID,
+    const SearchOut so = wave_search<BITWISE>(S, t, xq, yq, R0, XY, WR, cstart, ID,
                                                      nbr_row(nbr, t, kstride), sh, nretry, nties, nfail);
     if (lane == 0 && nfail != nfail0) atomicOr(err + 1 + items[item].sim, 2);
     if (lane == 0 && so.tau > 0)
@@ -2022,7 +2084,7 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
   mark(1, 1);
   mark(2, 0);
   hipLaunchKernelGGL(k_permute, grd_all, blk, 0, st, b.items_all, b.nitems_all, b.sims, perm, skeys,
-                     perm_mode, b.pos_cur, b.fcur, b.xyp, b.uxy, b.fnew, b.wrap, b.cstart, b.runs,
+                     perm_mode, b.pos_cur, b.fcur, b.xyp, b.fnew, b.wrap, b.cstart, b.runs,
                      b.run_count);
   hipLaunchKernelGGL(k_fill_runs, dim3(1024), dim3(256), 0, st, b.runs, b.run_count, skeys,
                      b.cstart);
@@ -2034,12 +2096,11 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
     // that drew quick searches make room for others (a few % faster than
     // one resident round)
     const int fb_grid = fastpath ? 4096 : (b.nitems < 4096 ? b.nitems : 4096);
-#define SPH_KNN(F32, NSUB)                                                                    \
-  hipLaunchKernelGGL((k_knn<false, F32, NSUB>), grd, dim3(256), 0, st, b.items, b.nitems,      \
-                     b.sims, b.xyp, b.wrap, b.cstart, b.fnew.h, b.fnew.ep,                      \
-                     b.fnew.vpx, b.fnew.vpy, b.fnew.id, b.nbr, b.kmax, b.fnew.rho, b.fnew.c,    \
-                     b.rec, b.stats, b.retry, b.retry_count, b.knn_cnt, b.knn_ann, b.walk,      \
-                     b.walk_miss)
+#define SPH_KNN(F32)                                                                          \
+  hipLaunchKernelGGL((k_knn<F32>), dim3(b.nitems * wpi), dim3(64), 0, st, b.items,            \
+                     b.nitems, b.sims, b.xyp, b.wrap, b.cstart, b.fnew.h, b.fnew.ep,           \
+                     b.fnew.vpx, b.fnew.vpy, b.fnew.id, b.nbr, b.kmax, b.fnew.rho, b.fnew.c,   \
+                     b.rec, b.stats, b.retry, b.retry_count, b.walk, b.walk_miss, wpi)
 #define SPH_FB(BW, F32)                                                                       \
   hipLaunchKernelGGL((k_knn_fallback<BW, F32>), dim3(fb_grid), dim3(256), 0, st, b.items,     \
                      b.nitems, b.sims, b.xyp, b.wrap, b.cstart, b.fnew.h,                       \
@@ -2047,25 +2108,11 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
                      b.fnew.c, b.rec, b.stats, b.retry, b.retry_count, fastpath ? 0 : 1, b.err)
     mark(6, 0);
     if (fastpath) {
-      const bool f32 = b.prec == kPrecFP32C;
-      if (b.walk.nsub == 4) {
-        if (f32) SPH_KNN(true, 4); else SPH_KNN(false, 4);
-      } else {
-        if (f32) SPH_KNN(true, 8); else SPH_KNN(false, 8);
-      }
+      const int wpi = walk_waves_per_item(b.nitems, b.walk.group);
+      if (b.prec == kPrecFP32C) SPH_KNN(true); else SPH_KNN(false);
     }
     mark(6, 1);
     mark(7, 0);
-    if (fastpath) {
-      if (b.prec == kPrecFP32C)
-        hipLaunchKernelGGL((k_knn_finish<true>), grd, dim3(256), 0, st, b.items, b.nitems, b.sims,
-                           b.xyp, b.uxy, b.fnew.h, b.fnew.ep, b.fnew.vpx, b.fnew.vpy, b.fnew.id, b.nbr,
-                           b.kmax, b.fnew.rho, b.fnew.c, b.rec, b.knn_cnt, b.knn_ann, b.stats);
-      else
-        hipLaunchKernelGGL((k_knn_finish<false>), grd, dim3(256), 0, st, b.items, b.nitems, b.sims,
-                           b.xyp, b.uxy, b.fnew.h, b.fnew.ep, b.fnew.vpx, b.fnew.vpy, b.fnew.id, b.nbr,
-                           b.kmax, b.fnew.rho, b.fnew.c, b.rec, b.knn_cnt, b.knn_ann, b.stats);
-    }
     mark(7, 1);
     mark(8, 0);
     if (b.bitwise) SPH_FB(true, false);
