@@ -239,8 +239,8 @@ int sph_set_graph(sph_sim* s, int32_t on);
  * particle 0.5 ... 16) on the current state and keep the fastest, then tune
  * the kNN walk's shape on that grid one knob at a time: the sub-tiles (cells
  * per axis) a group of 16 queries is looked up in (8, 4), the queries a wave
- * takes (64, 32), and the candidates per query above which a group is halved
- * (24, 32, 16).  Only
+ * takes (64, 32), and the share of candidates above which a group is halved
+ * (24, 32, 16 times 24).  Only
  * before the first step (SPH_ESTATE otherwise).  Either output may be NULL.
  * Outside the bitwise form the grid and shape change the order in which
  * neighbours are summed (results within the precision form's contract). */

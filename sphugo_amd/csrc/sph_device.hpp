@@ -209,8 +209,8 @@ struct Item {
 };
 
 // Shape of the kNN walk (the autotuner's knobs): bracket half-width around
-// each query's last h, the candidates per query (of a full group of 16) in a
-// group's cells above which the group is halved, the queries a wave takes (64,
+// each query's last h, a 24th of the candidates in the cells of a group of 16
+// queries above which the group is halved, the queries a wave takes (64,
 // 32 or 16, in groups of 16 one after the other), and the cells per axis that
 // a group's box is looked up in at most (4 or 8; the ABI calls it sub-tiles).
 struct WalkKnobs {

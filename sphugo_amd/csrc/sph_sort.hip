@@ -506,7 +506,8 @@ int64_t sort_counts_size(int64_t n) {
   // of any n' <= n (a serve pool sorts its occupied part).  The count table of
   // the sorts up to kMidMax has at most kMidBlocks rows of two digits a word.
   const int64_t large = (int64_t)256 * ((n + kSortTile - 1) / kSortTile);
-  const int64_t mid = (int64_t)kMidBlocks << (kMaxW - 1);
+  const int64_t rows = (n + 2 * kMidThreads - 1) / (2 * kMidThreads);
+  const int64_t mid = (rows < kMidBlocks ? rows : kMidBlocks) << (kMaxW - 1);
   return large > mid ? large : mid;
 }
 

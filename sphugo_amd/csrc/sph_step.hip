@@ -1187,11 +1187,15 @@ __device__ inline double row_density(const WalkShared& sh, NbrRow row, int k, do
 //   density   lane = (query, every fourth chunk of its row): the kernel sum
 //             from the LDS positions, the row to memory
 //
-// A group whose cells hold more than 16 * split candidates, or whose box more
-// than kWalkCand, is halved (cell order can put two distant regions in one
-// group), down to single queries, whose candidates are filtered by their own
-// circle; those still too wide, queries without an h and queries whose bracket
-// misses go to the exact search (k_knn_fallback).
+// A group whose cells hold more than 24 * split candidates (576: a box of 16
+// queries at k = 64 usually holds 250 in its cells; staging a few hundred more
+// costs less than two half groups: 4M 1.17 -> 1.12 ms against 384), or whose box
+// more than kWalkCand, is halved (cell order can put two distant regions in one
+// group), with kWalkRaw in place of 24 * split from then on.  Groups of 4 that
+// are still too wide go to the exact search, as queries without an h and
+// queries whose bracket misses do: its waves take one such query each, side by
+// side, where halving down to single queries kept one wave busy (30,000
+// clustered: 196 against 136 us per step).
 //
 // What bounds it: vector issue, 77 % of all issue slots at 4M clustered, k = 64
 // (about 130 vector instructions per query; 1.28 GB written, 0.29 GB read).
@@ -1199,7 +1203,7 @@ __device__ inline double row_density(const WalkShared& sh, NbrRow row, int k, do
 // no lane waits for the longest of 64 lists, and a group of 16 queries is a
 // short chain of loads, so small launches finish early.  Against the walk with
 // a query per lane and its separate selection and density kernel that this
-// replaced: 4M FP32C 1.40 -> 1.17 ms, 1M FP64 0.45 -> 0.35 ms, 77,777 at k = 19
+// replaced: 4M FP32C 1.40 -> 1.12 ms, 1M FP64 0.45 -> 0.33 ms, 77,777 at k = 19
 // 108 -> 31 us, 2,200 at k = 32 55 -> 13 us.  One wave per block: a wave that
 // ends frees its LDS at once (1.54 -> 1.39 ms); 10 KiB per wave and four waves
 // per SIMD without a spilled register, where five spilled 40 (1.39 -> 1.17 ms).
@@ -1228,12 +1232,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const int k = S->k;
   const double lx = S->lx, ly = S->ly;
   const int lg = S->lg;
-  const int raw_cap = kn.split * kGrp < kWalkRaw ? kn.split * kGrp : kWalkRaw;
+  const int raw_cap = kn.split * 24 < kWalkRaw ? kn.split * 24 : kWalkRaw;
   // ---- this lane's own query ----
   const bool valid = lane0 < nq;
   const uint32_t tw = (uint32_t)(it.first + w0);
   const uint32_t t = tw + (valid ? lane0 : 0);
   unsigned long long can;
+  const uint32_t wrap = WR[t];
   // the search circle's box in finest cells, widened by 1/64 of a cell (far
   // beyond the rounding to float of at most 6 * 2^13 cells)
   float qx0, qx1, qy0, qy1;
@@ -1268,7 +1273,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
       asm("" : "+v"(lane));
       const int ql = lane & (kGrp - 1), part = lane >> 4;
       const int l0 = __builtin_ctz(pending);
-      const uint32_t gmask = pending & (((1u << gsz) - 1u) << (l0 & ~(gsz - 1)));
+      // of the block of gsz queries that holds l0, those in l0's own image tile:
+      // a query that drifted over a periodic boundary stays a box length away
+      // from its slot's neighbours until the wrap
+      const unsigned long long tile = ballot(wrap == readlane_u(wrap, g * kGrp + l0));
+      const uint32_t gmask = pending & (((1u << gsz) - 1u) << (l0 & ~(gsz - 1))) &
+                             (uint32_t)(tile >> (g * kGrp));
       const bool grp = (gmask >> ql) & 1u;  // of the row's query ql
       auto row_box = [&](float v) {  // row g holds the group's own lanes
         return __int_as_float(__builtin_amdgcn_readlane(
@@ -1305,8 +1315,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const int nraw = __builtin_amdgcn_readlane(incl, 63);
       int ncand = 0;
       unsigned long long images = 0ull;
-      // a single query's candidates are filtered by its own circle below
-      bool fits = nraw <= (gsz > 1 ? raw_cap : kWalkRaw);
+      bool fits = nraw <= (gsz == kGrp ? raw_cap : kWalkRaw);
       if (fits) {
         wave_fence();
         ((u32x4*)sh.u.s.mark)[lane] = u32x4{0u, 0u, 0u, 0u};
@@ -1361,12 +1370,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                 in &= ballot(vis);
               }
               in &= ballot(px >= dbx0) & ballot(px <= dbx1) & ballot(py >= dby0) & ballot(py <= dby1);
-              if (gsz == 1) {
-                const double4 q = gq[l0];
-                const double ex = q.x - (pj[r].x - (double)img_ix(pk & 15u) * lx);
-                const double ey = q.y - (pj[r].y - (double)img_iy(pk & 15u) * ly);
-                in &= ballot(ex * ex + ey * ey <= q.w * (1 + 1e-9));
-              }
               images |= in & im;
               const int pos = ncand + lane_prefix(in);
               ncand += __popcll(in);
@@ -1384,7 +1387,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         fits = ncand <= kWalkCand;
       }
       if (!fits) {
-        if (gsz > 1) {
+        if (gsz > 4) {
           gsz >>= 1;
         } else {
           if (grp && part == g) gq[ql].z = kMissWide;
