@@ -410,12 +410,11 @@ static int run_pass(sph_sim* s, int perm_mode, int force_mode) {
 }
 
 int sph::check_device_flags(sph_sim* s) {
-  int err = 0;
-  KnnStats slots[kStatSlots];
-  HIPCHK(hipMemcpyAsync(&err, s->pb.err, sizeof(int), hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipMemcpyAsync(slots, s->pb.stats, sizeof slots, hipMemcpyDeviceToHost, s->st));
+  int err = 0, rc = enqueue_flags(s, 1);
+  if (rc) return rc;
   HIPCHK(hipStreamSynchronize(s->st));
-  const KnnStats st = sum_stats(slots);
+  KnnStats st;
+  take_flags(s, &st, &err, 1);
   s->last_stats = st;
   if (err) return fail(SPH_ERANGE, "a particle left the periodic images [-L, 2L) of the box");
   if (st.failures) return fail(SPH_ERANGE, "kNN: %llu searches found fewer than k neighbours",
@@ -615,8 +614,7 @@ extern "C" int sph_set_tuning(sph_sim* s, const double in[5]) {
 
 extern "C" int sph_synchronize(sph_sim* s) {
   if (!s) return fail(SPH_EINVAL, "null handle");
-  HIPCHK(hipStreamSynchronize(s->st));
-  return check_device_flags(s);
+  return check_device_flags(s);  // waits for the handle's work
 }
 
 extern "C" int sph_step(sph_sim* s, int32_t nsteps) {
@@ -638,9 +636,7 @@ extern "C" int sph_read_field(sph_sim* s, int32_t field, double* out) {
   s->bind();
   int rc = enqueue_read_field(s->pb, field, -1, s->d_scratch, s->st);
   if (rc) return fail(SPH_EDEVICE, "readback launch failed");
-  HIPCHK(hipMemcpyAsync(out, s->d_scratch, s->np * sizeof(double), hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  return 0;
+  return copy_out(s, out, s->d_scratch, s->np * sizeof(double));
 }
 
 extern "C" int sph_write_field(sph_sim* s, int32_t field, const double* in) {
@@ -667,10 +663,8 @@ extern "C" int sph_read_neighbours(sph_sim* s, uint32_t* ids, double* d2) {
   s->bind();
   rc = enqueue_read_neighbours(s->pb, s->d_nids, s->d_nd2, nullptr, nullptr, s->st);
   if (rc) return fail(SPH_EDEVICE, "neighbour readback launch failed");
-  HIPCHK(hipMemcpyAsync(ids, s->d_nids, total * sizeof(uint32_t), hipMemcpyDeviceToHost, s->st));
-  if (d2) HIPCHK(hipMemcpyAsync(d2, s->d_nd2, total * sizeof(double), hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  return 0;
+  if ((rc = copy_out(s, ids, s->d_nids, total * sizeof(uint32_t)))) return rc;
+  return d2 ? copy_out(s, d2, s->d_nd2, total * sizeof(double)) : 0;
 }
 
 extern "C" int sph_read_neighbour_pos(sph_sim* s, double* px, double* py) {
@@ -684,17 +678,12 @@ extern "C" int sph_read_neighbour_pos(sph_sim* s, double* px, double* py) {
   s->bind();
   rc = enqueue_read_neighbours(s->pb, s->d_nids, s->d_nd2, s->d_npx, s->d_npy, s->st);
   if (rc) return fail(SPH_EDEVICE, "neighbour readback launch failed");
-  HIPCHK(hipMemcpyAsync(px, s->d_npx, total * sizeof(double), hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipMemcpyAsync(py, s->d_npy, total * sizeof(double), hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  return 0;
+  if ((rc = copy_out(s, px, s->d_npx, total * sizeof(double)))) return rc;
+  return copy_out(s, py, s->d_npy, total * sizeof(double));
 }
 
 int sph::fetch_sims(sph_sim* s) {
-  HIPCHK(hipMemcpyAsync(s->hsims.data(), s->pb.sims, s->hsims.size() * sizeof(SimDev),
-                        hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  return 0;
+  return copy_out(s, s->hsims.data(), s->pb.sims, s->hsims.size() * sizeof(SimDev));
 }
 
 extern "C" int sph_reductions(sph_sim* s, double out[6]) {
@@ -767,10 +756,11 @@ extern "C" int sph_set_timing(sph_sim* s, int32_t on) {
 
 extern "C" int sph_knn_stats(sph_sim* s, int64_t* retries, int64_t* ties) {
   if (!s) return fail(SPH_EINVAL, "null handle");
-  KnnStats slots[kStatSlots];
-  HIPCHK(hipMemcpyAsync(slots, s->pb.stats, sizeof slots, hipMemcpyDeviceToHost, s->st));
+  KnnStats st;
+  int err, rc = enqueue_flags(s, 1);
+  if (rc) return rc;
   HIPCHK(hipStreamSynchronize(s->st));
-  const KnnStats st = sum_stats(slots);
+  take_flags(s, &st, &err, 1);
   if (retries) *retries = (int64_t)st.retries;
   if (ties) *ties = (int64_t)st.ties;
   return 0;
@@ -778,10 +768,11 @@ extern "C" int sph_knn_stats(sph_sim* s, int64_t* retries, int64_t* ties) {
 
 extern "C" int sph_knn_counters(sph_sim* s, int64_t out[7]) {
   if (!s || !out) return fail(SPH_EINVAL, "null argument");
-  KnnStats slots[kStatSlots];
-  HIPCHK(hipMemcpyAsync(slots, s->pb.stats, sizeof slots, hipMemcpyDeviceToHost, s->st));
+  KnnStats st;
+  int err, rc = enqueue_flags(s, 1);
+  if (rc) return rc;
   HIPCHK(hipStreamSynchronize(s->st));
-  const KnnStats st = sum_stats(slots);
+  take_flags(s, &st, &err, 1);
   const unsigned long long v[7] = {st.retries, st.ties, st.failures, st.miss_lo,
                                    st.miss_hi, st.miss_ann, st.split_fallback};
   for (int i = 0; i < 7; ++i) out[i] = (int64_t)v[i];
@@ -812,10 +803,7 @@ extern "C" int sph_batch_read_field(sph_sim* s, int32_t sim, int32_t field, doub
   s->bind();
   if (enqueue_read_field(s->pb, field, sim, s->d_scratch, s->st))
     return fail(SPH_EDEVICE, "readback launch failed");
-  HIPCHK(hipMemcpyAsync(out, s->d_scratch, s->sim_n[sim] * sizeof(double), hipMemcpyDeviceToHost,
-                        s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  return 0;
+  return copy_out(s, out, s->d_scratch, s->sim_n[sim] * sizeof(double));
 }
 
 extern "C" int sph_batch_write_field(sph_sim* s, int32_t sim, int32_t field, const double* in) {

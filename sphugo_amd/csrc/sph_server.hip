@@ -103,7 +103,7 @@ struct sph_server {
   int* d_rc = nullptr;
   double* d_stage = nullptr;  // kNumRes rows of capacity
   std::vector<int> h_err;  // error flags: [0] any, [1 + slot] per job slot
-  KnnStats h_stats[kStatSlots] = {};
+  KnnStats h_stats = {};
   unsigned long long seen_failures = 0;
   // slots freed and item lists changed at the end of a tick, uploaded at the
   // start of the next one (host buffers of a pending copy are not reused)
@@ -344,13 +344,12 @@ bool tick(sph_server* s) {
   for (Job* j : finishing)
     if (!rc) rc = enqueue_readback(s, j);
   if (!rc) {
-    hipError_t e = hipMemcpyAsync(s->h_err.data(), c.pb.err, s->h_err.size() * sizeof(int),
-                                  hipMemcpyDeviceToHost, c.st);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(s->h_stats, c.pb.stats, sizeof s->h_stats, hipMemcpyDeviceToHost, c.st);
-    if (e == hipSuccess && s->ev_tick[1]) e = hipEventRecord(s->ev_tick[1], c.st);
-    if (e == hipSuccess) e = hipStreamSynchronize(c.st);
+    rc = enqueue_flags(&c, (int)s->h_err.size());
+    hipError_t e = hipSuccess;
+    if (!rc && s->ev_tick[1]) e = hipEventRecord(s->ev_tick[1], c.st);
+    if (!rc && e == hipSuccess) e = hipStreamSynchronize(c.st);
     if (e != hipSuccess) rc = fail(SPH_EDEVICE, "tick: %s", hipGetErrorString(e));
+    if (!rc) take_flags(&c, &s->h_stats, s->h_err.data(), (int)s->h_err.size());
   }
   std::lock_guard<std::mutex> lk(s->mu);
   if (rc) {
@@ -372,7 +371,7 @@ bool tick(sph_server* s) {
   float gms = 0.f;
   if (s->ev_tick[0] && hipEventElapsedTime(&gms, s->ev_tick[0], s->ev_tick[1]) == hipSuccess)
     s->gpu_ms_sum += gms;
-  const unsigned long long failures = sum_stats(s->h_stats).failures;
+  const unsigned long long failures = s->h_stats.failures;
   bool flagged = s->h_err[0] != 0;
   for (int q = 0; q < s->max_jobs && !flagged; ++q) flagged = s->h_err[1 + q] != 0;
   if (flagged || failures != s->seen_failures) {

@@ -32,6 +32,17 @@ using sph::PassBuffers;
 using sph::Positions;
 using sph::SimDev;
 
+namespace sph {
+// Pinned blocks of a handle's readbacks (sph_stage.hip), taken when first used.
+struct Stage {
+  char* small = nullptr;   // one small copy
+  char* ring = nullptr;    // slots of a large copy
+  hipEvent_t ev[8] = {};   // per slot: filled
+};
+void stage_open(Stage& s);
+void stage_close(Stage& s);
+}  // namespace sph
+
 struct sph_sim {
   int device = 0;
   std::vector<SimDev> hsims;
@@ -64,6 +75,11 @@ struct sph_sim {
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   double grid_cpp = 4.0;        // cells per particle of the cell grid
   int64_t cell_capacity = 0;    // cstart entries allocated
+  sph::Stage stage;
+
+  sph_sim() { sph::stage_open(stage); }
+  sph_sim(const sph_sim&) = delete;
+  sph_sim& operator=(const sph_sim&) = delete;
 
   template <class T>
   int alloc(T** p, int64_t count) {
@@ -89,6 +105,7 @@ struct sph_sim {
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
     if (st) (void)hipStreamDestroy(st);
+    sph::stage_close(stage);
   }
   void bind() {
     pb.fcur = F[cur];
@@ -128,6 +145,7 @@ struct sph_sim {
     std::swap(gexec, o.gexec);
     std::swap(grid_cpp, o.grid_cpp);
     std::swap(cell_capacity, o.cell_capacity);
+    std::swap(stage, o.stage);
   }
 };
 
@@ -140,6 +158,13 @@ void set_grid(SimDev& d, int lg);
 void init_open_box(SimDev& d, const double* x, const double* y, int64_t n);
 int check_params(const sph_params* p, int64_t n);
 int fetch_sims(sph_sim* s);
+// readback staging (sph_stage.hip): copy `bytes` (a multiple of 4) of a device
+// array to the host after the stream's work so far; returns when they are there
+int copy_out(sph_sim* s, void* dst, const void* dev, size_t bytes);
+// write the first nerr error flags and the counters' sums to the handle's
+// pinned block (enqueue_flags), and read them there once the stream is done
+int enqueue_flags(sph_sim* s, int nerr);
+void take_flags(sph_sim* s, sph::KnnStats* stats, int* err, int nerr);
 int check_device_flags(sph_sim* s);
 int alloc_state(sph_sim* h, int64_t np, int nitems);
 int grid_log2(int64_t n, double cpp);

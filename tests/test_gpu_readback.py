@@ -1,0 +1,69 @@
+"""Readback staging at its size limits (GPU): the one-block copy, the slots of
+the ring (one to more than it holds, a last slot of any length), with one, two
+and four host threads, and from several threads at once.  What was written is
+read back bit for bit."""
+import threading
+
+import numpy as np
+import pytest
+
+from sphugo_amd import _lib as L
+from sphugo_amd import ics
+
+pytestmark = pytest.mark.gpu
+
+
+def _sim(n, k=2):
+    st = ics.uniform(n, seed=n)
+    return L.Sim(L.default_params(k=k, mass=1.0, hor=(0, 1), vert=(0, 1)), st["x"], st["y"])
+
+
+@pytest.mark.parametrize("n", [2, 3, 32767, 32768, 32769, 131072, 131073, 262143, 524289,
+                               1048576, 1048577, 1179651, 2359301])
+def test_fields_round_trip(n):
+    g = _sim(n)
+    r = np.random.default_rng(n)
+    for f in ("vx", "e"):
+        v = r.standard_normal(n)
+        g.set(f, v)
+        assert (g.get(f) == v).all(), f
+    # into memory that was there already, and starts at an odd address
+    raw = np.full(8 * n + 24, 7, np.uint8)
+    for off in (8, 1):
+        buf = np.frombuffer(raw.data, np.uint8)[off:off + 8 * n]
+        L.check(L.lib().sph_read_field(g._h, L.FIELD["e"],
+                                       buf.ctypes.data_as(L._D)))
+        assert (np.frombuffer(buf.tobytes(), np.float64) == v).all()
+        assert raw[off - 1] == 7 and (raw[off + 8 * n:] == 7).all()
+        raw[:] = 7
+
+
+def test_neighbour_rows_of_odd_length():
+    g = _sim(10007, k=7)
+    g.calculate_forces()
+    ids, d2 = g.neighbours()
+    only, _ = g.neighbours(with_d2=False)
+    assert (ids == only).all() and (np.diff(d2, axis=1) >= 0).all()
+    assert (d2[:, -1] ** 0.5 == g.get("h")).all()
+
+
+def test_reads_from_several_threads():
+    sims = [_sim(n) for n in (3000, 200001, 1500001)]
+    vals = []
+    for i, g in enumerate(sims):
+        v = np.random.default_rng(i).standard_normal(g.n)
+        g.set("vy", v)
+        vals.append(v)
+    bad = []
+
+    def read(g, v):
+        for _ in range(5):
+            if not (g.get("vy") == v).all():
+                bad.append(g.n)
+
+    ts = [threading.Thread(target=read, args=a) for a in zip(sims, vals)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
