@@ -2207,65 +2207,88 @@ int enqueue_write_field(PassBuffers& b, int field, int sim, const double* dev_in
 // Neighbour rows by ID: IDs of the neighbours, recomputed squared distances
 // (same formula as the search) and, if px is not null, the neighbours'
 // positions seen through the query's image offset o (NNPos = p_j - o,
-// sim/nearest-neighbour.go:81,152), sorted ascending by (d2, ID).  Entries of a
-// row past the simulation's k (batches of mixed k) read ID 0xFFFFFFFF and
-// NaN, so every output entry is written.
-__global__ void k_read_nbrs(const Item* __restrict__ items, int nitems,
-                            const SimDev* __restrict__ sims, const double2* __restrict__ XY, Fields f,
-                            const uint32_t* __restrict__ nbr, int kstride, int kout,
-                            uint32_t* __restrict__ ids, double* __restrict__ d2o,
-                            double* __restrict__ px, double* __restrict__ py) {
-  const Item it = items[blockIdx.x];
-  if ((int)threadIdx.x >= it.count) return;
+// sim/nearest-neighbour.go:81,152), sorted ascending by (d2, ID), equal ones (one
+// particle through several images) in list order.  Entries of a row past the
+// simulation's k (batches of mixed k) read ID 0xFFFFFFFF and NaN, so every
+// output entry is written.
+//
+// Lane = entry, G = 32 or 64 lanes per row: each counts the entries before its
+// own in that order (k broadcast reads from LDS) and writes to that place of the
+// row, so that a row leaves as one contiguous piece.  With a thread per row,
+// sorting by insertion in global memory, 50,021 rows of 32 took 262 us (521 us
+// with positions).
+constexpr int kReadRows = 32;  // rows of a block
+template <int G>
+__global__ __launch_bounds__(256) void k_read_nbrs(const Item* __restrict__ items, int nitems,
+                                                   const SimDev* __restrict__ sims,
+                                                   const double2* __restrict__ XY, Fields f,
+                                                   const uint32_t* __restrict__ nbr, int kstride,
+                                                   int kout, uint32_t* __restrict__ ids,
+                                                   double* __restrict__ d2o,
+                                                   double* __restrict__ px,
+                                                   double* __restrict__ py) {
+  constexpr int kRows = 256 / G;  // rows at once
+  __shared__ double sd[kRows][G];
+  __shared__ uint32_t sid[kRows][G];
+  const int item_idx = blockIdx.x / (kItem / kReadRows);
+  const int q0 = blockIdx.x % (kItem / kReadRows) * kReadRows;
+  const Item it = items[item_idx];
   const SimDev* S = sims + it.sim;
-  const int64_t t = it.first + threadIdx.x;
   const int k = S->k;
-  const int64_t row = (int64_t)f.id[t] + S->off;
-  uint32_t* ro = ids + row * kout;
-  double* rd = d2o + row * kout;
-  double* rx = px ? px + row * kout : nullptr;
-  double* ry = py ? py + row * kout : nullptr;
-  const double xi = XY[t].x, yi = XY[t].y;
-  for (int n = 0; n < k; ++n) {
-    const uint32_t pk = nbr_row(nbr, t, kstride)[n];
-    const uint32_t j = pk >> 4;
-    const double ox = (double)img_ix(pk & 15u) * S->lx;
-    const double oy = (double)img_iy(pk & 15u) * S->ly;
-    const double2 pj = XY[j];
-    const double ex = (xi + ox) - pj.x, ey = (yi + oy) - pj.y;
-    const double d2 = ex * ex + ey * ey;
-    const uint32_t id = f.id[j];
-    int m = n;
-    while (m > 0 && (rd[m - 1] > d2 || (rd[m - 1] == d2 && ro[m - 1] > id))) {
-      rd[m] = rd[m - 1];
-      ro[m] = ro[m - 1];
-      if (rx) {
-        rx[m] = rx[m - 1];
-        ry[m] = ry[m - 1];
+  const double lx = S->lx, ly = S->ly;
+  const int r = threadIdx.x / G, e = threadIdx.x % G;
+  // a row's lanes lie in one wave, whose LDS operations complete in order
+  for (int q = q0 + r; q < q0 + kReadRows && q < it.count; q += kRows) {
+    const int64_t t = it.first + q;
+    const double2 pi = XY[t];
+    double d2 = NAN, x = NAN, y = NAN;
+    uint32_t id = 0xFFFFFFFFu;
+    if (e < k) {
+      const uint32_t pk = nbr_row(nbr, t, kstride)[e];
+      const uint32_t j = pk >> 4;
+      const double ox = (double)img_ix(pk & 15u) * lx;
+      const double oy = (double)img_iy(pk & 15u) * ly;
+      const double2 pj = XY[j];
+      const double ex = (pi.x + ox) - pj.x, ey = (pi.y + oy) - pj.y;
+      d2 = ex * ex + ey * ey;
+      id = f.id[j];
+      x = pj.x - ox;
+      y = pj.y - oy;
+    }
+    wave_fence();
+    sd[r][e] = d2;
+    sid[r][e] = id;
+    wave_fence();
+    int at = e;
+    if (e < k) {
+      at = 0;
+      for (int m = 0; m < k; ++m) {
+        const double v = sd[r][m];
+        const uint32_t w = sid[r][m];
+        at += v < d2 || (v == d2 && (w < id || (w == id && m < e)));
       }
-      --m;
     }
-    rd[m] = d2;
-    ro[m] = id;
-    if (rx) {
-      rx[m] = pj.x - ox;
-      ry[m] = pj.y - oy;
-    }
-  }
-  for (int n = k; n < kout; ++n) {
-    ro[n] = 0xFFFFFFFFu;
-    rd[n] = NAN;
-    if (rx) {
-      rx[n] = NAN;
-      ry[n] = NAN;
+    if (e < kout) {
+      const int64_t o = ((int64_t)f.id[t] + S->off) * kout + at;
+      ids[o] = id;
+      d2o[o] = d2;
+      if (px) {
+        px[o] = x;
+        py[o] = y;
+      }
     }
   }
 }
 
 int enqueue_read_neighbours(const PassBuffers& b, uint32_t* dev_ids, double* dev_d2,
                             double* dev_px, double* dev_py, hipStream_t st) {
-  hipLaunchKernelGGL(k_read_nbrs, dim3(b.nitems), dim3(kItem), 0, st, b.items, b.nitems, b.sims,
-                     b.xyp, b.fcur, b.nbr, b.kmax, b.kout, dev_ids, dev_d2, dev_px, dev_py);
+  const dim3 grd(b.nitems * (kItem / kReadRows));
+#define SPH_READ(G)                                                                               \
+  hipLaunchKernelGGL((k_read_nbrs<G>), grd, dim3(256), 0, st, b.items, b.nitems, b.sims, b.xyp,   \
+                     b.fcur, b.nbr, b.kmax, b.kout, dev_ids, dev_d2, dev_px, dev_py)
+  if (b.kout <= 32) SPH_READ(32);
+  else SPH_READ(64);
+#undef SPH_READ
   return (int)hipGetLastError();
 }
 

@@ -67,3 +67,39 @@ def test_reads_from_several_threads():
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("ks", [(2,), (32,), (33,), (64,), (31, 64), (16, 32)])
+def test_neighbour_rows_of_each_width(ks):
+    """Rows of 32 and 64 lanes, alone and in batches of mixed k, on lattices
+    (exact ties) and in boxes so small that a particle is its neighbours'
+    neighbour through several images: ascending (d2, ID), the oracle's IDs and
+    distances, positions at those distances, and the fill past a row's k."""
+    import oracle as O
+    sts, ps = [], []
+    for i, k in enumerate(ks):
+        a = (np.arange(13) + 0.5) / 13
+        x, y = [v.ravel().copy() for v in np.meshgrid(a, a, indexing="ij")]
+        if i % 2:
+            x, y = ics.uniform(37, seed=k)["x"], ics.uniform(37, seed=k)["y"]
+        n = len(x)
+        sts.append({"x": x, "y": y, "vx": np.zeros(n), "vy": np.zeros(n), "e": np.ones(n)})
+        ps.append(L.default_params(k=k, mass=1.0 / n, hor=(0, 1), vert=(0, 1)))
+    g = L.Batch(ps, sts)
+    g.calculate_forces()
+    ids, d2 = g.neighbours()
+    px, py = g.neighbour_pos()
+    first = 0
+    for k, st in zip(ks, sts):
+        n = len(st["x"])
+        o = O.OracleSim(O.default_params(knn_mode=O.KNN_EXACT, k=k, mass=1.0 / n, hor=(0, 1),
+                                         vert=(0, 1)), st["x"], st["y"], st["vx"], st["vy"], st["e"])
+        o.calculate_forces()
+        oi, od = o.neighbours()
+        rows = slice(first, first + n)
+        assert (ids[rows, :k].astype(np.int64) == oi).all() and (d2[rows, :k] == od).all()
+        q = (st["x"][:, None] - px[rows, :k]) ** 2 + (st["y"][:, None] - py[rows, :k]) ** 2
+        assert np.abs(q - od).max() <= 1e-14
+        assert (ids[rows, k:] == 0xFFFFFFFF).all() and np.isnan(d2[rows, k:]).all()
+        assert np.isnan(px[rows, k:]).all() and np.isnan(py[rows, k:]).all()
+        first += n
