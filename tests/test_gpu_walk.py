@@ -66,3 +66,28 @@ def test_walk_resolves_most_queries():
     g.calculate_forces()
     c1 = g.knn_counters()
     assert c1["retries"] - c0["retries"] <= st["n"] // 20, (c0, c1)
+
+
+def _lattice(m):
+    a = (np.arange(m) + 0.5) / m
+    x, y = [v.ravel().copy() for v in np.meshgrid(a, a, indexing="ij")]
+    n = m * m
+    return {"x": x, "y": y, "vx": np.sin(40 * y), "vy": np.cos(30 * x), "e": 1.0 + x,
+            "mass": 1.0 / n}
+
+
+@pytest.mark.parametrize("name,k", [("lattice", 32), ("lattice", 40), ("lattice", 64),
+                                    ("uniform", 2), ("uniform", 31), ("clumps", 64), ("tiny", 36),
+                                    ("tiny", 64)])
+def test_bitwise_walk_is_exact(name, k):
+    """Bitwise form: the pass that walks gives the oracle's bits, as the pass of
+    exact searches before it does, exact ties (lattice) and neighbours through
+    several images (ten particles) included."""
+    st = {"lattice": lambda: _lattice(24), "uniform": lambda: ics.uniform(4099, seed=k),
+          "clumps": lambda: _clumps(4099, k), "tiny": lambda: ics.uniform(10, seed=4)}[name]()
+    g, o = _pair(st, k, flags=L.FLAG_BITWISE)
+    for _ in range(2):
+        _check_knn(g, o)
+        for f in ("rho", "c", "h", "ax", "ay", "edot"):
+            assert (g.get(f) == o.get(f)).all(), f
+        g.calculate_forces()
