@@ -23,13 +23,6 @@ __host__ __device__ inline int red_parts(int nitems) {
 constexpr int kMissSlots = 16;
 constexpr int kMissStride = 32;   // u32 per copy (one cache line)
 constexpr int kAnn = 16;          // kNN annulus entries kept per query
-// cell ranges: a permute wave whose particles span more than kWaveCells
-// cells queues them, in chunks of at most kRunChunk cells, for a parallel
-// fill (kRunQueue chunks per pass; a wave that finds the queue full writes
-// its cells itself)
-constexpr int kWaveCells = 4096;
-constexpr int kRunChunk = 4096;
-constexpr int kRunQueue = 65536;
 
 // Go folds 6*40/(Pi*7), 4*7/(Pi*4), 8*7/(Pi*4) exactly and rounds once
 // (sim/sph.go:266,275,293,303); these are the correctly rounded values.
@@ -40,6 +33,9 @@ constexpr double kWendlandDFPref = 0x1.1d34a60108f72p+2;
 enum : int32_t { kMonaghan = 0, kWendland = 1 };
 enum : int32_t { kPrecFP64 = 0, kPrecFP32C = 1 };
 enum : uint32_t { kFlagBitwise = 1u, kFlagTiming = 2u };
+// -1 (kPerSim) selects each simulation's own mode (SimDev::pmode / fmode)
+enum PermuteMode : int { kPerSim = -1, kPermPredict = 0, kPermInit = 1, kPermKeep = 2 };
+enum ForceMode : int { kForceKick = 0, kForceNoKick = 1 };
 
 // Per-simulation parameters and device-updated scalars.
 struct SimDev {
@@ -243,14 +239,14 @@ __device__ inline void stat_add(unsigned long long* p, unsigned long long v) {
   if (v) atomicAdd(p, v);
 }
 
-// Work-item index for this block, arranged so that each of the 8 XCDs
-// (which receive blocks round-robin) walks a contiguous run of items and
-// keeps its own L2 warm on one band of the particle array.
-__device__ inline int xcd_item(int nitems) {
-  const int b = blockIdx.x;
+// Work-item index for block b, arranged so that each of the 8 XCDs (which
+// receive blocks round-robin) walks a contiguous run of items and keeps its own
+// L2 warm on one band of the particle array.
+__device__ inline int xcd_item(int nitems, int b) {
   const int q = nitems >> 3, r = nitems & 7, x = b & 7;
   return x * q + (x < r ? x : r) + (b >> 3);
 }
+__device__ inline int xcd_item(int nitems) { return xcd_item(nitems, (int)blockIdx.x); }
 
 __device__ inline int64_t floordiv(int64_t a, int64_t b) {
   int64_t q = a / b;
@@ -260,6 +256,68 @@ __device__ inline int64_t floordiv(int64_t a, int64_t b) {
 // floor(a / 2^s): the arithmetic shift (every grid and level has 2^s cells
 // per axis, so no 64-bit division is needed on the device)
 __device__ inline int64_t floordiv_pow2(int64_t a, int s) { return a >> s; }
+
+// binning
+struct CellIdx {
+  int64_t ux, uy;  // unwrapped cell
+  bool ok;
+};
+
+__device__ inline CellIdx cell_of(const SimDev* S, double x, double y) {
+  double fx = floor((x - S->x0) * S->ivx);
+  double fy = floor((y - S->y0) * S->ivy);
+  const double lox = -2.0 * S->gx, hix = 3.0 * S->gx - 1;
+  const double loy = -2.0 * S->gy, hiy = 3.0 * S->gy - 1;
+  // an open axis has no images: its box (k_box) holds every pass position
+  // inside cells [0, G) with a wide margin; the clamp only pins the index
+  if (S->open & 1) fx = fx < 0 ? 0.0 : (fx > S->gx - 1 ? (double)(S->gx - 1) : fx);
+  if (S->open & 2) fy = fy < 0 ? 0.0 : (fy > S->gy - 1 ? (double)(S->gy - 1) : fy);
+  CellIdx c;
+  c.ok = (fx >= lox) && (fx <= hix) && (fy >= loy) && (fy <= hiy);
+  c.ux = c.ok ? (int64_t)fx : 0;
+  c.uy = c.ok ? (int64_t)fy : 0;
+  return c;
+}
+
+// What a particle's cell key is made of: the pass position (drift 1 applied
+// where the pass predicts), its cell, the cell's place on the curve.
+struct KeySrc {
+  const SimDev* sims;
+  const double *x, *y, *vx, *vy;
+  int mode;               // PermuteMode, kPerSim: each simulation's own
+  int* err;
+  uint32_t* retry_count;  // cleared for the pass by whichever launch makes keys
+  // loaded apart from its use, so that several particles' loads are in flight
+  struct Raw {
+    double x, y, vx, vy;
+  };
+  __device__ Raw load(const SimDev* S, int64_t t) const {
+    Raw r = {x[t], y[t], 0.0, 0.0};
+    if ((mode < 0 ? S->pmode : mode) == kPermPredict) {
+      r.vx = vx[t];
+      r.vy = vy[t];
+    }
+    return r;
+  }
+  __device__ uint32_t key(const SimDev* S, int sim, const Raw& r) const {
+    const int lg = S->lg;  // read before the error flags' atomics
+    const int64_t coff = S->coff;
+    double px = r.x, py = r.y;
+    if ((mode < 0 ? S->pmode : mode) == kPermPredict) {
+      const double dt = S->dt_half;
+      px = px + r.vx * dt;
+      py = py + r.vy * dt;
+    }
+    const CellIdx c = cell_of(S, px, py);
+    if (!c.ok) {
+      atomicOr(err, 1);
+      atomicOr(err + 1 + sim, 1);
+    }
+    const int64_t cx = c.ux - (floordiv_pow2(c.ux, lg) << lg);
+    const int64_t cy = c.uy - (floordiv_pow2(c.uy, lg) << lg);
+    return (uint32_t)(coff + hilbert2((uint32_t)cx, (uint32_t)cy, lg));
+  }
+};
 
 // Reference kernel functions, evaluated in Go's order with no contraction.
 #pragma clang fp contract(off)

@@ -16,8 +16,12 @@ struct SortBuffers {
   uint32_t* tot;     // [256]
 };
 
-int sort_pairs(SortBuffers& sb, int64_t n, int bits, hipStream_t st, bool first_identity,
+// Sorts (key, particle index) pairs; `make`: the keys are not in sb.keys but made
+// by the sort's first launch, of one simulation's particles 0 .. n - 1 (only
+// where sort_makes_keys says so).
+int sort_pairs(SortBuffers& sb, int64_t n, int bits, hipStream_t st, const KeySrc* make,
                uint32_t** keys_out, uint32_t** vals_out);
+bool sort_makes_keys(int64_t n);
 int64_t sort_counts_size(int64_t n);
 
 // One structure-of-arrays set of per-particle fields (positions separate).
@@ -29,10 +33,6 @@ struct Fields {
 struct Positions {
   double *x, *y;
 };
-
-// -1 (kPerSim) selects each simulation's own mode (SimDev::pmode / fmode)
-enum PermuteMode : int { kPerSim = -1, kPermPredict = 0, kPermInit = 1, kPermKeep = 2 };
-enum ForceMode : int { kForceKick = 0, kForceNoKick = 1 };
 
 struct PassBuffers {
   const Item* items;     // work items of the simulations
@@ -66,8 +66,6 @@ struct PassBuffers {
   int red_parts_max;    // the largest red_parts over the simulations (1: one stage)
   uint2* retry;           // kNN retry list (np entries)
   uint32_t* retry_count;
-  uint32_t* runs;          // queued cell chunks of the pass: (first, last, t0, nv) x kRunQueue
-  uint32_t* run_count;
   int have_h;             // every particle has an h from an earlier pass
   int any_open;           // some simulation has an open axis (k_bbox, k_box run)
   WalkKnobs walk;         // tile-search shape of the kNN walk

@@ -204,18 +204,34 @@ constexpr int kOneMax = kOneThreads * kOnePer;
 
 // Digit counts of each tile, block-major, two to a word (a tile's count fits
 // 16 bits).
-template <int PER>
-__global__ __launch_bounds__(kMidThreads) void k_sort_count(const uint32_t* __restrict__ keys,
+// MAKE: the keys are made here (of simulation 0) and written out.
+template <int PER, bool MAKE>
+__global__ __launch_bounds__(kMidThreads) void k_sort_count(uint32_t* __restrict__ keys, KeySrc src,
                                                             int n, int shift, int w,
                                                             uint32_t* __restrict__ counts) {
   __shared__ uint32_t hist[1 << kMaxW];
   const int tid = threadIdx.x, nd = 1 << w;
   const int base = blockIdx.x * kMidThreads * PER;
   uint32_t key[PER];
+  if constexpr (MAKE) {
+    KeySrc::Raw raw[PER];
 #pragma unroll
-  for (int r = 0; r < PER; ++r) {
-    const int i = base + r * kMidThreads + tid;
-    key[r] = i < n ? keys[i] : 0u;
+    for (int r = 0; r < PER; ++r) {
+      const int i = base + r * kMidThreads + tid;
+      raw[r] = src.load(src.sims, i < n ? i : n - 1);
+    }
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+      const int i = base + r * kMidThreads + tid;
+      key[r] = src.key(src.sims, 0, raw[r]);
+      if (i < n) keys[i] = key[r];
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+      const int i = base + r * kMidThreads + tid;
+      key[r] = i < n ? keys[i] : 0u;
+    }
   }
   for (int d = tid; d < nd; d += kMidThreads) hist[d] = 0;
   __syncthreads();
@@ -226,6 +242,7 @@ __global__ __launch_bounds__(kMidThreads) void k_sort_count(const uint32_t* __re
   __syncthreads();
   for (int p = tid; p < nd / 2; p += kMidThreads)
     counts[(int64_t)blockIdx.x * (nd / 2) + p] = hist[2 * p] | hist[2 * p + 1] << 16;
+  if (MAKE && blockIdx.x == 0 && tid == 0) *src.retry_count = 0u;
 }
 
 // exclusive scan of the block's values, one per thread
@@ -381,11 +398,9 @@ __global__ __launch_bounds__(kOneThreads) void k_sort_one(const uint32_t* __rest
   const int end = base + rounds * 64 < n ? base + rounds * 64 : n;
   uint32_t key[kOnePer], val[kOnePer], loc[kOnePer];
 #pragma unroll
-  for (int r = 0; r < kOnePer; ++r) {
-    const int i = first + r * 64;
-    key[r] = i < end ? kin[i] : 0u;
-    val[r] = (uint32_t)i;
-  }
+  for (int r = 0; r < kOnePer; ++r) key[r] = first + r * 64 < end ? kin[first + r * 64] : 0u;
+#pragma unroll
+  for (int r = 0; r < kOnePer; ++r) val[r] = (uint32_t)(first + r * 64);
   for (int p = 0; p < passes; ++p) {
     for (int d = tid; d < kWaves * kD / 2; d += kOneThreads) ((uint32_t*)cnt)[d] = 0u;
     __syncthreads();
@@ -443,8 +458,14 @@ static void with_width(int w, F&& f) {
   else f(std::integral_constant<int, kMaxW>{});
 }
 
-int sort_pairs(SortBuffers& sb, int64_t n, int bits, hipStream_t st,
-               bool first_identity, uint32_t** keys_out, uint32_t** vals_out) {
+// Between the one-block sort (whose single block made 2,200 keys no faster than
+// a launch of its own: 4.5 us) and 8 keys per thread (1,048,576 keys: 16.3 us
+// against 9.7 + 4.9 us apart); at 77,777 keys 4.8 us against 4.7 + 2.4, at 262,144
+// 5.2 against 4.8 + 4.7.
+bool sort_makes_keys(int64_t n) { return n > kOneMax && n <= kMidMax / 2; }
+
+int sort_pairs(SortBuffers& sb, int64_t n, int bits, hipStream_t st, const KeySrc* make,
+               uint32_t** keys_out, uint32_t** vals_out) {
   const int nblocks = (int)((n + kSortTile - 1) / kSortTile);
   uint32_t* kin = sb.keys;
   uint32_t* vin = sb.vals;
@@ -455,7 +476,8 @@ int sort_pairs(SortBuffers& sb, int64_t n, int bits, hipStream_t st,
     const int passes = (bits + kMaxW - 1) / kMaxW;
     with_width((bits + passes - 1) / passes, [&](auto width) {
       constexpr int W = decltype(width)::value;
-      if (n <= kOneMax && first_identity) {
+      const KeySrc src = make ? *make : KeySrc{};
+      if (n <= kOneMax) {
         hipLaunchKernelGGL((k_sort_one<W>), dim3(1), dim3(kOneThreads), 0, st, kin, kout, vout,
                            (int)n, passes);
         kin = kout;
@@ -467,11 +489,15 @@ int sort_pairs(SortBuffers& sb, int64_t n, int bits, hipStream_t st,
         constexpr int P = decltype(per)::value;
         const int nb = (int)((n + kMidThreads * P - 1) / (kMidThreads * P));
         for (int p = 0; p < passes; ++p) {
-          hipLaunchKernelGGL((k_sort_count<P>), dim3(nb), dim3(kMidThreads), 0, st, kin, (int)n,
-                             p * W, W, sb.counts);
+          if (make && p == 0)
+            hipLaunchKernelGGL((k_sort_count<P, true>), dim3(nb), dim3(kMidThreads), 0, st, kin, src,
+                               (int)n, p * W, W, sb.counts);
+          else
+            hipLaunchKernelGGL((k_sort_count<P, false>), dim3(nb), dim3(kMidThreads), 0, st, kin,
+                               src, (int)n, p * W, W, sb.counts);
           hipLaunchKernelGGL((k_sort_move<W, P>), dim3(nb), dim3(kMidThreads), 0, st, kin, vin,
                              kout, vout, (int)n, p * W, sb.counts, nb,
-                             (p == 0 && first_identity) ? 1 : 0);
+                             p == 0 ? 1 : 0);
           std::swap(kin, kout);
           std::swap(vin, vout);
         }
@@ -493,7 +519,7 @@ int sort_pairs(SortBuffers& sb, int64_t n, int bits, hipStream_t st,
                        nblocks);
     hipLaunchKernelGGL(k_sort_scatter, dim3(nblocks), dim3(kSortThreads), 0, st, kin, vin,
                        kout, vout, n, shift, sb.counts, sb.tot, nblocks,
-                       (p == 0 && first_identity) ? 1 : 0);
+                       p == 0 ? 1 : 0);
     uint32_t* t = kin; kin = kout; kout = t;
     t = vin; vin = vout; vout = t;
   }

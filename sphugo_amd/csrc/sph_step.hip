@@ -2,12 +2,14 @@
 //
 //   k_keys          cell key of each particle's pass position: Hilbert index
 //                   of a power-of-two grid plus the simulation's cell offset
-//                   (replaces Treebuild/Partition, sim/core.go:126-224)
+//                   (replaces Treebuild/Partition, sim/core.go:126-224); made by
+//                   the sort itself for one simulation of up to a million
+//                   particles
 //   sort_pairs      stable LSD radix sort of (key, index) (sph_sort.hip)
 //   k_permute       gather the state into cell order, apply the drift-1 /
 //                   predictor step (sim/sph.go:108-117) or the step-0
-//                   initialisation (:96-101), and write the cell ranges
-//   k_fill_runs     the cell ranges of sparse grid stretches k_permute queued
+//                   initialisation (:96-101); other blocks of the launch
+//                   write the cell ranges
 //   k_knn           bracketed walk: a wavefront searches groups of 16
 //                   consecutive queries, sorting the candidates of each
 //                   group's box against every query's bracket around its last
@@ -30,35 +32,13 @@
 // association order; the library is compiled with -ffp-contract=off so no
 // product is fused into an add there.  Only the FP32C pair terms enable
 // contraction, block by block.
+#include <algorithm>
 #include <type_traits>
 
 #include "sph_device.hpp"
 #include "sph_host.hpp"
 
 namespace sph {
-
-// ------------------------------------------------------------------------
-// binning
-struct CellIdx {
-  int64_t ux, uy;  // unwrapped cell
-  bool ok;
-};
-
-__device__ inline CellIdx cell_of(const SimDev* S, double x, double y) {
-  double fx = floor((x - S->x0) * S->ivx);
-  double fy = floor((y - S->y0) * S->ivy);
-  const double lox = -2.0 * S->gx, hix = 3.0 * S->gx - 1;
-  const double loy = -2.0 * S->gy, hiy = 3.0 * S->gy - 1;
-  // an open axis has no images: its box (k_box) holds every pass position
-  // inside cells [0, G) with a wide margin; the clamp only pins the index
-  if (S->open & 1) fx = fx < 0 ? 0.0 : (fx > S->gx - 1 ? (double)(S->gx - 1) : fx);
-  if (S->open & 2) fy = fy < 0 ? 0.0 : (fy > S->gy - 1 ? (double)(S->gy - 1) : fy);
-  CellIdx c;
-  c.ok = (fx >= lox) && (fx <= hix) && (fy >= loy) && (fy <= hiy);
-  c.ux = c.ok ? (int64_t)fx : 0;
-  c.uy = c.ok ? (int64_t)fy : 0;
-  return c;
-}
 
 // Cell span [a, b] of a search at a level with nc cells per axis, limited to
 // the images the reference visits: [-2 nc, 3 nc) on a periodic axis (the
@@ -181,144 +161,143 @@ __global__ __launch_bounds__(256) void k_box(SimDev* __restrict__ sims,
 }
 
 __global__ __launch_bounds__(kItem) void k_keys(const Item* __restrict__ items, int nitems,
-                                                const SimDev* __restrict__ sims,
-                                                const double* __restrict__ X,
-                                                const double* __restrict__ Y,
-                                                const double* __restrict__ VX,
-                                                const double* __restrict__ VY, int mode,
-                                                uint32_t* __restrict__ keys, int* err,
-                                                uint32_t* __restrict__ retry_count,
-                                                uint32_t* __restrict__ run_count,
+                                                KeySrc src, uint32_t* __restrict__ keys,
                                                 uint32_t hole_cpp) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *retry_count = 0u;
-    *run_count = 0u;
-  }
   const Item it = items[xcd_item(nitems)];
   if ((int)threadIdx.x >= it.count) return;
   const int64_t t = it.first + threadIdx.x;
   if (it.sim < 0) {
     // unused pool slot: a key of its own position keeps it in place
     keys[t] = (uint32_t)(t * hole_cpp);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *src.retry_count = 0u;
     return;
   }
-  const SimDev* S = sims + it.sim;
-  if (mode < 0) mode = S->pmode;
-  double x = X[t], y = Y[t];
-  if (mode == kPermPredict) {
-    const double dt = S->dt_half;
-    x = x + VX[t] * dt;
-    y = y + VY[t] * dt;
-  }
-  CellIdx c = cell_of(S, x, y);
-  if (!c.ok) {
-    atomicOr(err, 1);
-    atomicOr(err + 1 + it.sim, 1);
-  }
-  const int64_t cx = c.ux - (floordiv_pow2(c.ux, S->lg) << S->lg);
-  const int64_t cy = c.uy - (floordiv_pow2(c.uy, S->lg) << S->lg);
-  keys[t] = (uint32_t)(S->coff + hilbert2((uint32_t)cx, (uint32_t)cy, S->lg));
+  const SimDev* S = src.sims + it.sim;
+  keys[t] = src.key(S, it.sim, src.load(S, t));
+  if (blockIdx.x == 0 && threadIdx.x == 0) *src.retry_count = 0u;
 }
 
-// Queues the cells [lo, hi] of a permute wave for k_fill_runs, in chunks of
-// at most kRunChunk cells (wave-uniform call): cell q of a chunk starts at
-// t0 plus the number of the wave's nv keys (skeys[t0 .. t0 + nv)) below q.
-// Returns false, leaving the cells to the caller, when the queue is full
-// (its reserved slots below the queue's end then hold empty chunks).
-__device__ inline bool queue_cells(uint32_t* __restrict__ runs, uint32_t* __restrict__ run_count,
-                                   int64_t lo, int64_t hi, int64_t t0, int nv, int lane) {
-  const uint32_t nch = (uint32_t)((hi - lo + kRunChunk) / kRunChunk);
-  uint32_t at = 0;
-  if (lane == 0) at = atomicAdd(run_count, nch);
-  at = __shfl(at, 0, 64);
-  const bool fits = at + nch <= (uint32_t)kRunQueue;
-  for (uint32_t c = (uint32_t)lane; c < nch && at + c < (uint32_t)kRunQueue; c += 64) {
-    const int64_t f = lo + (int64_t)c * kRunChunk;
-    const int64_t l = f + kRunChunk - 1 < hi ? f + kRunChunk - 1 : hi;
-    uint32_t* r = runs + 4 * (int64_t)(at + c);
-    r[0] = fits ? (uint32_t)f : 1u;
-    r[1] = fits ? (uint32_t)l : 0u;
-    r[2] = (uint32_t)t0;
-    r[3] = (uint32_t)nv;
+// Number of keys below `target` in the sorted skeys[lo, hi), plus lo, by one wave:
+// 64 probes at a time.
+__device__ inline int64_t wave_lower_bound(const uint32_t* __restrict__ skeys, int64_t lo,
+                                           int64_t hi, uint32_t target, int lane) {
+  while (hi - lo > 64) {
+    const int64_t step = (hi - lo + 63) >> 6;
+    const int64_t p = lo + lane * step;
+    const int below = __popcll(ballot(p < hi && skeys[p] < target));
+    const int64_t l = lo;
+    lo = below ? l + (below - 1) * step + 1 : l;
+    hi = l + below * step < hi ? l + below * step : hi;
+    if (hi < lo) hi = lo;
   }
-  return fits;
+  const int64_t p = lo + lane;
+  return lo + __popcll(ballot(p < hi && skeys[p] < target));
 }
 
-// The queued chunks of cells of this pass, a block per chunk: the chunk's
-// wave keys in LDS, each cell a binary search over them.
-__global__ __launch_bounds__(256) void k_fill_runs(const uint32_t* __restrict__ runs,
-                                                   const uint32_t* __restrict__ run_count,
-                                                   const uint32_t* __restrict__ skeys,
-                                                   uint32_t* __restrict__ cstart) {
-  __shared__ uint32_t keys[64];
-  const uint32_t c = *run_count;
-  const uint32_t n = c < (uint32_t)kRunQueue ? c : (uint32_t)kRunQueue;
-  for (uint32_t r = blockIdx.x; r < n; r += gridDim.x) {  // uniform per block
-    const int64_t f = runs[4 * (int64_t)r], l = runs[4 * (int64_t)r + 1];
-    const uint32_t t0 = runs[4 * (int64_t)r + 2];
-    const int nv = (int)runs[4 * (int64_t)r + 3];
-    __syncthreads();
-    if ((int)threadIdx.x < nv) keys[threadIdx.x] = skeys[(int64_t)t0 + threadIdx.x];
-    __syncthreads();
-    for (int64_t q = f + threadIdx.x; q <= l; q += 256) {
-      int a = 0, b = nv;  // the number of keys below q
-      while (a < b) {
-        const int mid = (a + b) >> 1;
-        if ((int64_t)keys[mid] >= q) b = mid; else a = mid + 1;
-      }
-      cstart[q] = t0 + (uint32_t)a;
+// The cell ranges of the shares of `nit` consecutive items, from `it` on, of
+// their simulation's cells [coff, coff + G^2): cell q starts at the first
+// particle whose key is >= q.  The block finds the particles of its cells in the
+// sorted keys, counts them per cell in LDS and writes the counts' running sum,
+// so every cell and key is touched once wherever the particles are.  Bound by
+// latency (two searches, then one chain per 2,048 cells), so it runs beside the
+// permuting blocks.  Written by the permuting waves instead, each the cells up
+// to its particles' keys, a sparse stretch of the grid held a wave and needed a
+// queue and a launch of its own.  Permute with cell ranges, before and now:
+// 2,200 particles 10.0 -> 4.7 us, 4,700 in a tube 23.2 -> 6.8, 12 simulations
+// served together 24 -> 12.3, 77,777 14 -> 9.1, 262,144 14.4 -> 10.0, 1M clustered
+// 42.8 -> 38.7, 4M 144.6 -> 149.5.  Cells outside every simulation's range are
+// never read.
+constexpr int kCellChunk = 2048;
+__device__ inline void item_cells(const Item& it, int nit, const SimDev* S,
+                                  const uint32_t* __restrict__ skeys,
+                                  uint32_t* __restrict__ cstart) {
+  __shared__ uint32_t cnt[kCellChunk];
+  __shared__ uint32_t wsum[kItem / 64];
+  __shared__ int64_t bound[2];
+  constexpr int kOwn = kCellChunk / kItem;  // counters scanned by a thread
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t off = S->off, end = off + S->n;
+  const int64_t cells = (int64_t)S->gx * S->gy;
+  const int64_t ni = (S->n + kItem - 1) / kItem, li = (it.first - off) / kItem;
+  const int64_t c0 = cells * li / ni, c1 = cells * (li + nit) / ni;
+  int64_t a = -1;
+  for (int64_t c = c0; c < c1; c += kCellChunk) {
+    const int nc = (int)(c1 - c < kCellChunk ? c1 - c : kCellChunk);
+    // the chunk's particles [a, b); the next chunk goes on at b
+    if (wv == 0 && a < 0) {
+      const int64_t v = wave_lower_bound(skeys, off, end, (uint32_t)(S->coff + c), lane);
+      if (lane == 0) bound[0] = v;
     }
+    if (wv == 1) {
+      const int64_t v = wave_lower_bound(skeys, off, end, (uint32_t)(S->coff + c + nc), lane);
+      if (lane == 0) bound[1] = v;
+    }
+    for (int i = tid; i < kCellChunk; i += kItem) cnt[i] = 0u;
+    __syncthreads();
+    if (a < 0) a = bound[0];
+    const int64_t b = bound[1];
+    // eight loads in flight per thread (a dense chunk holds many particles)
+    for (int64_t t = a + tid; t < b; t += 8 * kItem) {
+      uint32_t key[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) key[u] = t + u * kItem < b ? skeys[t + u * kItem] : 0u;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (t + u * kItem < b) atomicAdd(&cnt[key[u] - (uint32_t)(S->coff + c)], 1u);
+    }
+    __syncthreads();
+    uint32_t own[kOwn], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+      own[i] = cnt[tid * kOwn + i];
+      sum += own[i];
+    }
+    const uint32_t incl = (uint32_t)wave_incl_scan((int)sum);
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    uint32_t run = (uint32_t)a + incl - sum;
+#pragma unroll
+    for (int q = 0; q < kItem / 64; ++q) run += q < wv ? wsum[q] : 0u;
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+      cnt[tid * kOwn + i] = run;
+      run += own[i];
+    }
+    __syncthreads();
+    for (int i = tid; i < nc; i += kItem) cstart[S->coff + c + i] = cnt[i];
+    __syncthreads();
+    a = b;
   }
+  if (li + nit == ni && tid == 0) cstart[S->coff + cells] = (uint32_t)end;
 }
 
+// The first ncells blocks write the cell ranges, per_cells items' shares each;
+// the rest permute a work item each.  The ranges come first, so that their
+// chains are covered by the permuting blocks: behind them the launch takes 164 us
+// at 4M against 147, and 13.6 against 11.9 at 262,144.
 __global__ __launch_bounds__(kItem) void k_permute(
-    const Item* __restrict__ items, int nitems, const SimDev* __restrict__ sims,
-    const uint32_t* __restrict__ perm, const uint32_t* __restrict__ skeys, int mode,
-    Positions pin, Fields fin, double2* __restrict__ xyp, Fields fout,
-    uint8_t* __restrict__ wrap, uint32_t* __restrict__ cstart, uint32_t* __restrict__ runs,
-    uint32_t* __restrict__ run_count) {
-  const Item it = items[xcd_item(nitems)];
-  if (it.sim < 0) return;  // unused pool slot: stays in place, owns no cells
+    const Item* __restrict__ items_all, int nitems_all, const Item* __restrict__ items, int nitems,
+    int ncells, int per_cells, const SimDev* __restrict__ sims, const uint32_t* __restrict__ perm,
+    const uint32_t* __restrict__ skeys, int mode, Positions pin, Fields fin,
+    double2* __restrict__ xyp, Fields fout, uint8_t* __restrict__ wrap,
+    uint32_t* __restrict__ cstart) {
+  if ((int)blockIdx.x < ncells) {
+    const int i0 = xcd_item(ncells) * per_cells;
+    for (int i = i0; i < i0 + per_cells && i < nitems;) {
+      // consecutive items of one simulation share their searches
+      const Item it = items[i];
+      int n = 1;
+      while (i + n < i0 + per_cells && i + n < nitems && items[i + n].sim == it.sim) ++n;
+      item_cells(it, n, sims + it.sim, skeys, cstart);
+      i += n;
+    }
+    return;
+  }
+  const Item it = items_all[xcd_item(nitems_all, (int)blockIdx.x - ncells)];
+  if (it.sim < 0) return;  // unused pool slot: stays in place
   const SimDev* S = sims + it.sim;
   const bool valid = (int)threadIdx.x < it.count;
   const int64_t t = it.first + (valid ? threadIdx.x : 0);
-  // Cell ranges of this simulation's cells [coff, coff + G^2]: cell q starts
-  // at the first particle whose key is >= q; the simulation's last particle
-  // closes the range.  The wave writes the contiguous block of cells
-  // (key[t0 - 1], key[t_last]] of its particles together, coalesced, each
-  // cell finding its particle by a binary search over the lanes' keys; a
-  // block wider than kWaveCells (a sparse stretch of the grid) goes to
-  // k_fill_runs instead, which spreads it over many blocks.  Cells outside
-  // every simulation's range are never read.
-  {
-    const int lane = threadIdx.x & 63;
-    const int w0 = threadIdx.x & ~63;
-    if (w0 < it.count) {
-      const int64_t t0 = it.first + w0;
-      const int nv = (it.count - w0) < 64 ? (it.count - w0) : 64;
-      const uint32_t kt = skeys[t0 + (lane < nv ? lane : nv - 1)];
-      const int64_t lo = (t0 == S->off ? S->coff : (int64_t)skeys[t0 - 1] + 1);
-      const int64_t hi = (int64_t)__shfl(kt, nv - 1, 64);
-      if (hi - lo + 1 <= kWaveCells || !queue_cells(runs, run_count, lo, hi, t0, nv, lane)) {
-        for (int64_t qb = lo; qb <= hi; qb += 64) {  // uniform: every lane shuffles
-          const int64_t q = qb + lane;
-          int a = 0, b = nv - 1;  // smallest lane with key >= q (lane nv-1 qualifies)
-          for (int st = 0; st < 6; ++st) {
-            const int mid = (a + b) >> 1;
-            const int64_t km = (int64_t)__shfl(kt, mid, 64);
-            if (km >= q) b = mid; else a = mid + 1;
-          }
-          if (q <= hi) cstart[q] = (uint32_t)(t0 + a);
-        }
-      }
-      const int64_t tl = t0 + nv - 1;
-      if (tl == S->off + S->n - 1) {
-        const int64_t end = S->coff + (int64_t)S->gx * S->gy;
-        if (end - hi <= kWaveCells || !queue_cells(runs, run_count, hi + 1, end, tl + 1, 0, lane))
-          for (int64_t q = hi + 1 + lane; q <= end; q += 64) cstart[q] = (uint32_t)(tl + 1);
-      }
-    }
-  }
   if (valid) {
     const uint32_t i = perm[t];
     if (mode < 0) mode = S->pmode;
@@ -2158,20 +2137,27 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
     hipLaunchKernelGGL(k_box, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, b.red_first,
                        b.red_count);
   }
-  hipLaunchKernelGGL(k_keys, grd_all, blk, 0, st, b.items_all, b.nitems_all, b.sims, b.pos_cur.x,
-                     b.pos_cur.y, b.fcur.vx, b.fcur.vy, perm_mode, b.sort.keys, b.err,
-                     b.retry_count, b.run_count, b.hole_cpp);
+  const KeySrc src = {b.sims, b.pos_cur.x, b.pos_cur.y, b.fcur.vx, b.fcur.vy, perm_mode, b.err,
+                      b.retry_count};
+  // one simulation: the sort's first read of the keys makes them
+  const bool fused = b.nsims == 1 && b.hole_cpp == 0 && sort_makes_keys(b.np);
+  if (!fused)
+    hipLaunchKernelGGL(k_keys, grd_all, blk, 0, st, b.items_all, b.nitems_all, src, b.sort.keys,
+                       b.hole_cpp);
   mark(0, 1);
   mark(1, 0);
   uint32_t *skeys = nullptr, *perm = nullptr;
-  sort_pairs(b.sort, b.np, b.key_bits, st, true, &skeys, &perm);
+  sort_pairs(b.sort, b.np, b.key_bits, st, fused ? &src : nullptr, &skeys, &perm);
   mark(1, 1);
   mark(2, 0);
-  hipLaunchKernelGGL(k_permute, grd_all, blk, 0, st, b.items_all, b.nitems_all, b.sims, perm, skeys,
-                     perm_mode, b.pos_cur, b.fcur, b.xyp, b.fnew, b.wrap, b.cstart, b.runs,
-                     b.run_count);
-  hipLaunchKernelGGL(k_fill_runs, dim3(1024), dim3(256), 0, st, b.runs, b.run_count, skeys,
-                     b.cstart);
+  // as many cell blocks as fit at once, beside which the permuting ones follow
+  // (permute at 1M / 4M: 1,024 blocks 46.1 / 148.4 us, 2,048 40.3 / 146.6, 4,096
+  // 37.4 / 151.9)
+  const int per_cells = (b.nitems + 2047) / 2048;
+  const int ncells = (b.nitems + per_cells - 1) / per_cells;
+  hipLaunchKernelGGL(k_permute, dim3(b.nitems_all + ncells), blk, 0, st, b.items_all, b.nitems_all,
+                     b.items, b.nitems, ncells, per_cells, b.sims, perm, skeys, perm_mode,
+                     b.pos_cur, b.fcur, b.xyp, b.fnew, b.wrap, b.cstart);
   mark(2, 1);
   mark(3, 0);
   {
@@ -2179,7 +2165,8 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
     // retry lists: four times as many blocks as fit at once, so that blocks
     // that drew quick searches make room for others (a few % faster than
     // one resident round)
-    const int fb_grid = fastpath ? 4096 : (b.nitems < 4096 ? b.nitems : 4096);
+    const int most = fastpath ? 64 * b.nitems : b.nitems;  // four queries per block
+    const int fb_grid = most < 4096 ? most : 4096;
 #define SPH_KNN(F32, BW)                                                                      \
   hipLaunchKernelGGL((k_knn<F32, BW>), dim3(b.nitems * wpi), dim3(64), 0, st, b.items,            \
                      b.nitems, b.sims, b.xyp, b.wrap, b.cstart, b.fnew.h, b.fnew.ep,           \
