@@ -66,7 +66,8 @@ struct PassBuffers {
   int red_parts_max;    // the largest red_parts over the simulations (1: one stage)
   uint2* retry;           // kNN retry list (np entries)
   uint32_t* retry_count;
-  int have_h;             // every particle has an h from an earlier pass
+  int have_h;             // every particle has an h from an earlier pass, except:
+  int some_new;           // some simulations do not (a server admitted them)
   int any_open;           // some simulation has an open axis (k_bbox, k_box run)
   WalkKnobs walk;         // tile-search shape of the kNN walk
   int* err;             // device error flags: [0] any, [1 + s] simulation s (1: a

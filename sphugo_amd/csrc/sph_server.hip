@@ -336,6 +336,7 @@ bool tick(sph_server* s) {
   }
   if (!rc) {
     c.bind();
+    c.pb.some_new = !admitted.empty();
     rc = enqueue_pass(c.pb, kPerSim, kPerSim, c.st, nullptr);
     if (rc) rc = fail(SPH_EDEVICE, "pass launch: %s", hipGetErrorString((hipError_t)rc));
     c.cur ^= 1;
@@ -483,7 +484,7 @@ extern "C" int sph_server_create(int64_t capacity, int32_t max_jobs, int32_t kma
   pb.key_bits = bits;
   pb.hole_cpp = kHoleCpp;
   pb.walk = kWalkDefault;
-  pb.have_h = 1;  // jobs without h take the exact search
+  pb.have_h = 1;
   c.cell_capacity = pb.ncells + 1;
   SimDev* d_sims = nullptr;
   int rc = 0;

@@ -745,8 +745,8 @@ __device__ inline float centred_step(double x, double x0, double l) {
   return (float)(0.5 - (f - floor(f)));
 }
 
-// First-pass search radius: local density from the occupancy of the
-// query's cell at a level holding a few particles.
+// Search radius of a query without an h: local density from the occupancy of
+// the query's cell at a level holding a few particles.
 __device__ inline double local_radius(const SimDev* S, const uint32_t* __restrict__ cstart,
                                       double xq, double yq) {
   const CellIdx ci = cell_of(S, xq, yq);
@@ -817,6 +817,7 @@ struct WalkShared {
 };
 constexpr double kThinSum = 2e-3;  // FP32C kernel sums below it are redone in FP64
 constexpr double kMissWide = -1.0, kMissLo = -2.0, kMissAnn = -3.0, kMissHi = -4.0;
+constexpr double kSeeded = -5.0;
 static_assert(sizeof(WalkShared) == 10240, "sixteen waves per CU");
 
 typedef __attribute__((address_space(3))) uint8_t LdsByte;
@@ -1208,6 +1209,53 @@ __device__ inline double rows_bitwise(WalkShared& sh, const double4* gq, uint32_
   return facc;
 }
 
+// Distance to the k-th neighbour of each query of `gmask` among the group's
+// staged candidates, by bisection of the squared distance (lane = candidate,
+// FP32; to within 1 %, a fraction of the walk's bracket).  gq[i].w is the radius
+// R that the group's box was made for and becomes the answer: up to R it is the
+// distance, beyond it (candidates outside the box are missing) it is negative,
+// an upper limit to search again within; gq[i].z becomes kSeeded.
+template <bool IMG>
+__device__ inline void seed_radii(WalkShared& sh, double4* gq, int ncand, uint32_t gmask,
+                                  uint32_t t0, int k, double lx, double ly, int lane) {
+  constexpr int NR = (kWalkCand + 63) / 64;
+  for (uint32_t rem = gmask; rem; rem &= rem - 1u) {
+    const int i = __builtin_ctz(rem);
+    const double4 q = gq[i];
+    const uint32_t ti = t0 + (uint32_t)i;
+    float d2[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int s = r * 64 + lane;
+      const bool in = s < ncand && (sh.pk[s] >> 4) != ti;
+      d2[r] = in ? (float)slot_d2<IMG>(sh, (uint32_t)s, q.x, q.y, lx, ly) : INFINITY;
+    }
+    auto count = [&](float v) {
+      int n = 0;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) n += __popcll(ballot(d2[r] <= v));
+      return n;
+    };
+    const float R2 = (float)(q.w * q.w);
+    const bool inside = count(R2) >= k;
+    float lo = inside ? 0.f : R2, hi = inside ? R2 : 16.f * R2;
+    double h = -2.0 * q.w;
+    if (inside || count(hi) >= k) {
+      for (int it = 0; it < 24 && hi - lo > 0.02f * hi; ++it) {
+        const float mid = 0.5f * (lo + hi);
+        if (count(mid) >= k) hi = mid; else lo = mid;
+      }
+      h = sqrt(0.5 * ((double)lo + (double)hi));
+      if (!inside) h = -1.02 * h;
+    }
+    if (lane == 0) {
+      gq[i].z = kSeeded;
+      gq[i].w = h;
+    }
+  }
+  wave_fence();
+}
+
 // kNN + density + sound speed + force record of the queries that have an h
 // from the last pass.  A wave takes up to 64 consecutive (Hilbert-ordered)
 // queries, lane = query, and searches groups of 16 of them one after the
@@ -1247,7 +1295,16 @@ __device__ inline double rows_bitwise(WalkShared& sh, const double4* gq, uint32_
 // 108 -> 31 us, 2,200 at k = 32 55 -> 13 us.  One wave per block: a wave that
 // ends frees its LDS at once (1.54 -> 1.39 ms); 10 KiB per wave and four waves
 // per SIMD without a spilled register, where five spilled 40 (1.39 -> 1.17 ms).
-template <bool FP32C, bool BITWISE>
+//
+// SEED: finds an h for the queries that have none (a simulation's first pass)
+// in place of their neighbours, from the same staging: `seed` 1 for the queries
+// without an h (2: for all), searching within local_radius, and 0 for those that
+// the first search left with a limit (negative).  The walk then takes them like
+// any other; before, all of them went to the exact search, a wave each.  kNN of
+// a first pass, before and now: 2,200 particles at k = 32 586 -> 69 us, 100,000 in
+// an open box 853 -> 138, 30,011 clustered at k = 64 in the bitwise form 980 -> 300;
+// a first call of 20 steps at 4M clustered 73.3 -> 60.0 ms.
+template <bool FP32C, bool BITWISE, bool SEED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_knn(
     const Item* __restrict__ items, int nitems, const SimDev* __restrict__ sims,
     const double2* __restrict__ XY, const uint8_t* __restrict__ WR,
@@ -1256,7 +1313,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const uint32_t* __restrict__ ID, uint32_t* __restrict__ nbr, int kstride,
     double* __restrict__ RHO, double* __restrict__ C, void* __restrict__ recp,
     KnnStats* __restrict__ stats, uint2* __restrict__ retry, uint32_t* __restrict__ retry_count,
-    WalkKnobs kn, uint32_t* __restrict__ walk_miss, int wpi) {
+    WalkKnobs kn, uint32_t* __restrict__ walk_miss, int wpi, int seed) {
   __shared__ WalkShared sh;
   const int lane0 = threadIdx.x;
   // wpi blocks (of one wave) per item (4, 8 or 16), each taking 256 / wpi
@@ -1284,9 +1341,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
   float qx0, qx1, qy0, qy1;
   {
     const double2 pq = XY[t];
-    const double hp = H[t];
-    const double delta = S->walk_delta;
-    can = ballot(valid && hp > 0);
+    double hp = H[t];
+    const double delta = SEED ? 0.0 : S->walk_delta;
+    if constexpr (SEED) {
+      // every image lies within 3 boxes
+      const double rcap = 3.0 * (lx > ly ? lx : ly);
+      const bool todo = valid && (seed == 0 ? hp < 0 : seed == 2 || !(hp > 0));
+      if (todo) hp = seed ? local_radius(S, cstart, pq.x, pq.y) : -hp;
+      if (hp > rcap) hp = rcap;
+      can = ballot(todo && hp > 0);
+    } else {
+      can = ballot(valid && hp > 0);
+    }
     const double Rlo = hp * (1 - delta), Rhi = hp * (1 + delta);
     const double Rm = Rhi * (1 + 1e-12) + 1e-15 * (lx + ly);
     const double fx = (pq.x - S->x0) * S->ivx, fy = (pq.y - S->y0) * S->ivy;
@@ -1295,7 +1361,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     qx1 = -(float)(fx + rx);
     qy0 = (float)(fy - ry);
     qy1 = -(float)(fy + ry);
-    sh.q[lane0] = make_double4(pq.x, pq.y, Rlo * Rlo, Rhi * Rhi);
+    sh.q[lane0] = make_double4(pq.x, pq.y, Rlo * Rlo, SEED ? Rhi : Rhi * Rhi);
   }
   unsigned nties = 0;
   const uint32_t table = kHilbertTable.w[lane0];
@@ -1437,6 +1503,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         continue;
       }
       wave_fence();
+      if constexpr (SEED) {
+        if (images) seed_radii<true>(sh, gq, ncand, gmask, t0, k, lx, ly, lane);
+        else seed_radii<false>(sh, gq, ncand, gmask, t0, k, lx, ly, lane);
+        pending &= ~gmask;
+        gsz = kGrp;
+        continue;
+      }
       int c_lo = 0, c_an = 0;
       const double xq = gq[ql].x, yq = gq[ql].y;
       const int nr = (ncand + 63) >> 6;
@@ -1495,6 +1568,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
   wave_fence();
   const double4 out = sh.q[lane0];
   const bool tried = (can >> lane0) & 1ull;
+  if constexpr (SEED) {
+    // a limit only for a second search
+    if (tried) H[t] = out.z == kSeeded && (seed || out.w > 0) ? out.w : 0.0;
+    return;
+  }
   const bool resolved = tried && out.z >= 0.0;
   if (resolved)
     write_result<FP32C>(S, t, out.x, out.y, out.z, out.w, EP, VPX, VPY, H, RHO, C, recp);
@@ -1702,28 +1780,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const double* __restrict__ VPY, const uint32_t* __restrict__ ID,
     uint32_t* __restrict__ nbr, int kstride, double* __restrict__ RHO,
     double* __restrict__ C, void* __restrict__ recp, KnnStats* __restrict__ stats,
-    const uint2* __restrict__ retry, const uint32_t* __restrict__ retry_count, int all_mode,
+    const uint2* __restrict__ retry, const uint32_t* __restrict__ retry_count,
     int* __restrict__ err) {
   __shared__ SearchShared wsh[4];
   const int wv = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   SearchShared& sh = wsh[wv];
   const int64_t nw = (int64_t)gridDim.x * 4;
-  const int64_t total = all_mode ? (int64_t)nitems * kItem : (int64_t)(*retry_count);
+  const int64_t total = (int64_t)(*retry_count);
   unsigned long long nretry = 0, nties = 0, nfail = 0;
   for (int64_t q = (int64_t)blockIdx.x * 4 + wv; q < total; q += nw) {
-    int64_t t;
-    int item;
-    if (all_mode) {
-      item = (int)(q / kItem);
-      const int qi = (int)(q % kItem);
-      if (qi >= items[item].count) continue;
-      t = items[item].first + qi;
-    } else {
-      const uint2 e = retry[q];
-      t = e.x;
-      item = (int)e.y;
-    }
+    const uint2 e = retry[q];
+    const int64_t t = e.x;
+    const int item = (int)e.y;
     const SimDev* S = sims + items[item].sim;
     const double2 pq = XY[t];
     const double xq = pq.x, yq = pq.y, hp = H[t];
@@ -2061,8 +2130,7 @@ __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
                                                 const double* __restrict__ red_part,
                                                 const int* __restrict__ item_first,
                                                 const int* __restrict__ item_count, Fields f,
-                                                int mode, uint32_t* __restrict__ walk_miss,
-                                                int walked) {
+                                                int mode, uint32_t* __restrict__ walk_miss) {
   __shared__ double sh[kNumRed][256];
   __shared__ uint32_t miss[2][kMissSlots];
   SimDev* S = sims + blockIdx.x;
@@ -2108,7 +2176,7 @@ __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
       move += miss[0][q];
       wide += miss[1][q];
     }
-    if (walked) S->walk_delta = adapt_delta(S->walk_delta, S->walk_delta0, move, wide, S->n);
+    S->walk_delta = adapt_delta(S->walk_delta, S->walk_delta0, move, wide, S->n);
     const double m = __longlong_as_double((long long)S->cfl_min_bits);
     S->dt_half = S->use_cfl ? 0.5 * (S->cfl * m) : S->dt_fixed;
     S->cfl_min_bits = (unsigned long long)__double_as_longlong(INFINITY);
@@ -2161,29 +2229,29 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
   mark(2, 1);
   mark(3, 0);
   {
-    const bool fastpath = b.have_h;
-    // retry lists: four times as many blocks as fit at once, so that blocks
-    // that drew quick searches make room for others (a few % faster than
-    // one resident round)
-    const int most = fastpath ? 64 * b.nitems : b.nitems;  // four queries per block
-    const int fb_grid = most < 4096 ? most : 4096;
-#define SPH_KNN(F32, BW)                                                                      \
-  hipLaunchKernelGGL((k_knn<F32, BW>), dim3(b.nitems * wpi), dim3(64), 0, st, b.items,            \
+    const int wpi = walk_waves_per_item(b.nitems, b.walk.group);
+#define SPH_KNN(F32, BW, SEED, seed)                                                          \
+  hipLaunchKernelGGL((k_knn<F32, BW, SEED>), dim3(b.nitems * wpi), dim3(64), 0, st, b.items,    \
                      b.nitems, b.sims, b.xyp, b.wrap, b.cstart, b.fnew.h, b.fnew.ep,           \
                      b.fnew.vpx, b.fnew.vpy, b.fnew.id, b.nbr, b.kmax, b.fnew.rho, b.fnew.c,   \
-                     b.rec, b.stats, b.retry, b.retry_count, b.walk, b.walk_miss, wpi)
+                     b.rec, b.stats, b.retry, b.retry_count, b.walk, b.walk_miss, wpi, seed)
+    // the retry list: four times as many blocks as fit at once, so that blocks
+    // that drew quick searches make room for others (a few % faster than
+    // one resident round); four queries per block
+    const int fb_grid = b.nitems < 64 ? 64 * b.nitems : 4096;
 #define SPH_FB(BW, F32)                                                                       \
   hipLaunchKernelGGL((k_knn_fallback<BW, F32>), dim3(fb_grid), dim3(256), 0, st, b.items,     \
                      b.nitems, b.sims, b.xyp, b.wrap, b.cstart, b.fnew.h,                       \
                      b.fnew.ep, b.fnew.vpx, b.fnew.vpy, b.fnew.id, b.nbr, b.kmax, b.fnew.rho,   \
-                     b.fnew.c, b.rec, b.stats, b.retry, b.retry_count, fastpath ? 0 : 1, b.err)
+                     b.fnew.c, b.rec, b.stats, b.retry, b.retry_count, b.err)
     mark(6, 0);
-    if (fastpath) {
-      const int wpi = walk_waves_per_item(b.nitems, b.walk.group);
-      if (b.bitwise) SPH_KNN(false, true);
-      else if (b.prec == kPrecFP32C) SPH_KNN(true, false);
-      else SPH_KNN(false, false);
+    if (!b.have_h || b.some_new) {
+      SPH_KNN(false, false, true, b.have_h ? 1 : 2);
+      SPH_KNN(false, false, true, 0);
     }
+    if (b.bitwise) SPH_KNN(false, true, false, 0);
+    else if (b.prec == kPrecFP32C) SPH_KNN(true, false, false, 0);
+    else SPH_KNN(false, false, false, 0);
     mark(6, 1);
     mark(7, 0);
     mark(7, 1);
@@ -2211,8 +2279,7 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
     hipLaunchKernelGGL(k_reduce_part, dim3(b.nsims * b.red_parts_max), dim3(256), 0, st, b.sims,
                        b.partials, b.red_first, b.red_count, b.red_part, b.red_parts_max);
   hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, b.red_part,
-                     b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss,
-                     b.have_h);
+                     b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss);
   mark(5, 1);
   return (int)hipGetLastError();
 }
