@@ -59,7 +59,7 @@ struct PassBuffers {
   uint32_t* cstart;     // ncells + 1
   uint32_t* nbr;        // np * kmax packed (index << 4 | image code)
   void* rec;            // np force records (RecD or RecF)
-  double* partials;     // nitems * kNumRed
+  double* partials;     // nitems * 4 * kNumRed (a wave's 64 particles, or an item's 256)
   KnnStats* stats;      // kStatSlots copies
   uint32_t* walk_miss;  // per simulation: the walk's miss counts (kMissSlots lines)
   double* red_part;     // per simulation: kRedSplit first-stage sums (kNumRed each)

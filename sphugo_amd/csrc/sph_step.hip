@@ -1710,21 +1710,19 @@ __device__ inline void stage_window(u32x4* lds, const T* __restrict__ g, int64_t
   }
 }
 
-struct NoFlush {
-  __device__ void operator()() const {}
-};
-
-// Visits the k entries of a neighbour row, N (4 or 8) at a time: the N
-// sources (src's records of the entries) are gathered together and the next N entries' row
-// chunks are loaded before the current N are processed, so that the row and
-// gather latencies overlap.  Full rounds gather their entries as they are; a
-// last partial round gathers the query's own slot `self` for the entries past
-// k.  NT: the row is read for the last time (non-temporal loads).  `flush`
-// runs after each round of N entries (block-compensated sums).
-template <int N, bool NT = false, typename S, typename Body, typename Flush = NoFlush>
-__device__ inline void row_visit(const NbrRow row, int k, uint32_t self, const S& src,
-                                 Body body, Flush flush = Flush()) {
+// Visits the entries [n0, k) of a neighbour row (n0 a multiple of 4), N (4 or
+// 8) at a time: the N sources (src's records of the entries) are gathered
+// together and the next N entries' row chunks are loaded before the current N
+// are processed, so that the row and gather latencies overlap.  Full rounds
+// gather their entries as they are; a last partial round gathers the query's
+// own slot `self` for the entries past k.  NT: the row is read for the last
+// time (non-temporal loads).  `flush` runs after each round of N entries, with
+// the next round's first.
+template <int N, bool NT = false, typename S, typename Body, typename Flush>
+__device__ inline void row_visit(const NbrRow row, int n0, int k, uint32_t self, const S& src,
+                                 Body body, Flush flush) {
   static_assert(N == 4 || N == 8, "one or two row chunks per round");
+  if (n0 >= k) return;
   using T = std::remove_cv_t<std::remove_reference_t<decltype(src.far(0u))>>;
   auto ld = [&](int c) {
     if constexpr (NT) return __builtin_nontemporal_load(row.chunk(c));
@@ -1733,9 +1731,8 @@ __device__ inline void row_visit(const NbrRow row, int k, uint32_t self, const S
   // entries past k are never read from the chunks (they gather `self`), so a
   // chunk past the row is zeros rather than a copy that waits for a load
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  u32x4 qa = ld(0);
-  u32x4 qb = (N == 8 && k > 4) ? ld(1) : zero;
-  int n0 = 0;
+  u32x4 qa = ld(n0 >> 2);
+  u32x4 qb = (N == 8 && k > n0 + 4) ? ld((n0 >> 2) + 1) : zero;
   for (; n0 + N <= k; n0 += N) {
     const uint32_t pks[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
     T pj[N];
@@ -1746,7 +1743,7 @@ __device__ inline void row_visit(const NbrRow row, int k, uint32_t self, const S
     }
 #pragma unroll
     for (int u = 0; u < N; ++u) body(pks[u], pj[u]);
-    flush();
+    flush(n0 + N);
   }
   if (n0 < k) {
     const uint32_t spk = self << 4;
@@ -1761,7 +1758,7 @@ __device__ inline void row_visit(const NbrRow row, int k, uint32_t self, const S
       if (n0 + u >= k) break;
       body(pks[u], pj[u]);
     }
-    flush();
+    flush(n0 + N);
   }
 }
 
@@ -1816,19 +1813,51 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // Force: one thread per particle, neighbours summed in list order (the
 // reference's order when the list is sorted, BITWISE), then kick, drift 2,
 // periodic wrap and reflection (sim/sph.go:327-401,122-193).
-template <bool FP32C, bool EXACT>
+//
+// A row's terms are added up in four sections of whole chunks, and the four
+// sums in order (the bitwise form: straight through, as the reference), so that
+// both splits of the work give the same bits.  PARTS 1: a thread per particle,
+// the block's 256 particles sharing a window.  PARTS 4: a block takes 64
+// particles and each of its waves one section of their rows, for launches whose
+// time is one thread's chain of gathers: 2,200 particles at k = 32 FP64 16 -> 8 us,
+// at k = 64 27 -> 11; FP32C 13 -> 7 and 20 -> 8.
+inline constexpr int kSections = 4;
+// The most items for PARTS 4, whose smaller windows hold fewer of the
+// neighbours and are staged four times as often.  FP64 force (with the event
+// records' 2 us) by PARTS 1 and 4, us: k = 16 24,576 particles 14.0 and 12.4,
+// 32,768 13.9 and 14.3; k = 32 32,768 19.4 and 16.0, 49,152 20.0 and 19.9; k = 64 49,152
+// 30.5 and 23.5; 262,144 at k = 32 38 and 60.
+inline int force_split_items(int kmax) { return 64 + 2 * kmax; }
+__host__ __device__ inline int section_begin(int k, int s) { return 4 * (((k + 3) / 4 * s) >> 2); }
+
+// The sum of the sections done, and the entry after the current one.
+struct SectionSum {
+  double x = 0.0, y = 0.0, e = 0.0;
+  int end, s = 0;
+  __device__ explicit SectionSum(int k) : end(0) { next(k); }
+  __device__ void next(int k) {  // past empty sections (k < 13)
+    const int at = end;
+    do end = section_begin(k, ++s); while (end == at && s < kSections);
+  }
+};
+
+template <bool FP32C, bool EXACT, int PARTS>
 __global__ __launch_bounds__(256) void k_force(
     const Item* __restrict__ items, int nitems, SimDev* __restrict__ sims,
     const void* __restrict__ recp, Fields f, const uint32_t* __restrict__ nbr, int kstride,
     int mode, Positions pout, double* __restrict__ partials, const double2* __restrict__ XY) {
+  static_assert(PARTS == 1 || (PARTS == kSections && !EXACT));
+  constexpr int kParticles = kItem / PARTS;  // of a block
   __shared__ double red[4][kNumRed + 1];
-  const int item_idx = xcd_item(nitems);
+  const int blk = xcd_item(nitems * PARTS);
+  const int item_idx = blk / PARTS;
   const Item it = items[item_idx];
   SimDev* S = sims + it.sim;
-  const int wv = threadIdx.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const bool valid = (int)threadIdx.x < it.count;
-  const int64_t t = it.first + (valid ? threadIdx.x : 0);
+  const int slot = PARTS == 1 ? (int)threadIdx.x : (blk % PARTS) * kParticles + lane;
+  const bool valid = slot < it.count;
+  const int64_t t = it.first + (valid ? slot : 0);
   const int k = S->k;
   const double mass = S->mass;
   const double lx = S->lx, ly = S->ly;
@@ -1839,18 +1868,23 @@ __global__ __launch_bounds__(256) void k_force(
   // first + 384) (16 KB FP32C, 32 KB FP64), which hold about 85 % of the
   // neighbours of Hilbert-ordered particles; the rest are gathered from
   // memory.  Force time at 4M clustered, k = 64: FP64 1.17 -> 0.87 ms,
-  // FP32C 0.57 -> 0.49 ms (with 4 records in flight instead of 8).
-  constexpr int kWin = 512;
-  constexpr int kBack = 128;
+  // FP32C 0.57 -> 0.49 ms (with 4 records in flight instead of 8).  The same
+  // around 64 particles: half the slots.
+  constexpr int kWin = PARTS == 1 ? 512 : 256;
+  constexpr int kBack = PARTS == 1 ? 128 : 96;
   using Rec = std::conditional_t<FP32C, RecF, RecD>;
   __shared__ u32x4 wrec[kWin * sizeof(Rec) / 16];
-  const int64_t wb = it.first - kBack;
+  const int64_t wb = it.first + (PARTS == 1 ? 0 : (blk % PARTS) * kParticles) - kBack;
   stage_window<Rec, kWin>(wrec, (const Rec*)recp, wb, S->off, S->off + S->n);
   __syncthreads();
   const WinSrc<Rec, kWin> wsrc{(const Rec*)recp, wrec, (uint32_t)wb};
   double xi, yi, hi, ci, rhoi, A;
   double sx = 0.0, sy = 0.0, se = 0.0;
   const NbrRow row = nbr_row(nbr, t, kstride);
+  // this thread's entries: the whole row, or its wave's section
+  const int n0 = PARTS == 1 ? 0 : section_begin(k, wv);
+  const int n1 = PARTS == 1 || wv == PARTS - 1 ? k : section_begin(k, wv + 1);
+  SectionSum total(k);
   if constexpr (!FP32C) {
     const RecD* rec = (const RecD*)recp;
     const RecD me = rec[t];
@@ -1860,7 +1894,7 @@ __global__ __launch_bounds__(256) void k_force(
     const double alpha = S->alpha, beta = S->beta, eta2 = S->eta2;
     const double hinv = EXACT ? 0.0 : 1.0 / hi;
     // 4 records (64 B each) in flight per lane, the next row chunk behind them
-    row_visit<4, true>(row, k, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb) {
+    row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb) {
       const double ox = (double)img_ix(pk & 15u) * lx, oy = (double)img_iy(pk & 15u) * ly;
       const double rABx = (nb.x - ox) - xi, rABy = (nb.y - oy) - yi;
       const double vABx = nb.vpx - vpxi, vABy = nb.vpy - vpyi;
@@ -1907,7 +1941,20 @@ __global__ __launch_bounds__(256) void k_force(
         sy += rABy * w;
         se += dot * dR;
       }
+    }, [&](int n) {
+      if (!EXACT && PARTS == 1 && n == total.end) {
+        total.x += sx;
+        total.y += sy;
+        total.e += se;
+        sx = sy = se = 0.0;
+        total.next(k);
+      }
     });
+    if constexpr (!EXACT && PARTS == 1) {
+      sx = total.x;
+      sy = total.y;
+      se = total.e;
+    }
   } else {
     const RecF* rec = (const RecF*)recp;
     const RecF me = rec[t];
@@ -1929,10 +1976,17 @@ __global__ __launch_bounds__(256) void k_force(
     const float alpha = (float)S->alpha, beta = (float)S->beta, eta2 = (float)S->eta2;
     // block-compensated sums (a Kahan step per round of 4 neighbours)
     BlockKahan ax_, ay_, ae_;
-    auto flush = [&]() {
+    auto flush = [&](int n) {
       ax_.flush();
       ay_.flush();
       ae_.flush();
+      if (PARTS == 1 && n == total.end) {
+        total.x += ax_.value();
+        total.y += ay_.value();
+        total.e += ae_.value();
+        ax_ = ay_ = ae_ = BlockKahan();
+        total.next(k);
+      }
     };
     kern_visit(kern, [&](auto kt) {
       using KT = decltype(kt);
@@ -1974,12 +2028,12 @@ __global__ __launch_bounds__(256) void k_force(
       // wave whose queries all take fixed-point displacements (the usual case)
       // runs a loop without the FP64 form, so every record loads whole.
       if (__all(fixed)) {
-        row_visit<4, true>(row, k, (uint32_t)t, wsrc, [&](uint32_t, const RecF& nb) {
+        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t, const RecF& nb) {
           pair(__builtin_fmaf((float)(int32_t)(nb.ux - me.ux), fsx, csx),
                __builtin_fmaf((float)(int32_t)(nb.uy - me.uy), fsy, csy), nb);
         }, flush);
       } else {
-        row_visit<4, true>(row, k, (uint32_t)t, wsrc, [&](uint32_t pk, const RecF& nb) {
+        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecF& nb) {
           float rx, ry;
           if (fixed) {
             rx = __builtin_fmaf((float)(int32_t)(nb.ux - me.ux), fsx, csx);
@@ -1994,9 +2048,24 @@ __global__ __launch_bounds__(256) void k_force(
         }, flush);
       }
     });
-    sx = ax_.value();
-    sy = ay_.value();
-    se = ae_.value();
+    sx = PARTS == 1 ? total.x : ax_.value();
+    sy = PARTS == 1 ? total.y : ay_.value();
+    se = PARTS == 1 ? total.e : ae_.value();
+  }
+  if constexpr (PARTS > 1) {
+    __shared__ double sec[3][PARTS][64];
+    sec[0][wv][lane] = sx;
+    sec[1][wv][lane] = sy;
+    sec[2][wv][lane] = se;
+    __syncthreads();
+    if (wv) return;
+    sx = sy = se = 0.0;
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) {
+      sx += sec[0][p][lane];
+      sy += sec[1][p][lane];
+      se += sec[2][p][lane];
+    }
   }
   double r_e = 0, r_rho = 0, r_E = 0, r_px = 0, r_py = 0, r_cfl = INFINITY;
   if (valid) {
@@ -2058,6 +2127,19 @@ __global__ __launch_bounds__(256) void k_force(
     const double other = __shfl_xor(r_cfl, o, 64);
     r_cfl = other < r_cfl ? other : r_cfl;
   }
+  if constexpr (PARTS > 1) {
+    if (lane == 0) {
+      double* p = partials + (int64_t)blk * kNumRed;
+      p[0] = r_e;
+      p[1] = r_rho;
+      p[2] = r_E;
+      p[3] = r_px;
+      p[4] = r_py;
+      if (r_cfl < INFINITY)
+        atomicMin(&S->cfl_min_bits, (unsigned long long)__double_as_longlong(r_cfl));
+    }
+    return;
+  }
   if (lane == 0) {
     red[wv][0] = r_e;
     red[wv][1] = r_rho;
@@ -2097,8 +2179,17 @@ __device__ inline void block_sum(double (*sh)[256], double (&acc)[kNumRed]) {
   }
 }
 
+// Item i's force partial r, from one or four values (a wave's 64 particles
+// each): the same sum either way.
+__device__ inline double item_partial(const double* __restrict__ partials, int parts, int64_t i,
+                                      int r) {
+  const double* p = partials + i * parts * kNumRed + r;
+  return parts == 1 ? p[0] : (p[0] + p[kNumRed]) + (p[2 * kNumRed] + p[3 * kNumRed]);
+}
+
 __global__ __launch_bounds__(256) void k_reduce_part(const SimDev* __restrict__ sims,
                                                      const double* __restrict__ partials,
+                                                     int parts_per_item,
                                                      const int* __restrict__ item_first,
                                                      const int* __restrict__ item_count,
                                                      double* __restrict__ red_part,
@@ -2117,7 +2208,7 @@ __global__ __launch_bounds__(256) void k_reduce_part(const SimDev* __restrict__ 
 #pragma unroll 4
   for (int i = ia + (int)threadIdx.x; i < ib; i += 256)
 #pragma unroll
-    for (int r = 0; r < kNumRed; ++r) acc[r] += partials[(int64_t)(i0 + i) * kNumRed + r];
+    for (int r = 0; r < kNumRed; ++r) acc[r] += item_partial(partials, parts_per_item, i0 + i, r);
   block_sum(sh, acc);
   if (threadIdx.x < kNumRed)
     red_part[((int64_t)sim * kRedSplit + part) * kNumRed + threadIdx.x] = sh[threadIdx.x][0];
@@ -2127,6 +2218,7 @@ __global__ __launch_bounds__(256) void k_reduce_part(const SimDev* __restrict__ 
 // next CFL half step, the TotalMomentum quirk value and the next bracket.
 __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
                                                 const double* __restrict__ partials,
+                                                int parts_per_item,
                                                 const double* __restrict__ red_part,
                                                 const int* __restrict__ item_first,
                                                 const int* __restrict__ item_count, Fields f,
@@ -2159,7 +2251,7 @@ __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
 #pragma unroll 8
     for (int i = tid; i < ni; i += 256)
 #pragma unroll
-      for (int r = 0; r < kNumRed; ++r) acc[r] += partials[(int64_t)(i0 + i) * kNumRed + r];
+      for (int r = 0; r < kNumRed; ++r) acc[r] += item_partial(partials, parts_per_item, i0 + i, r);
   } else if (tid < nparts) {
 #pragma unroll
     for (int r = 0; r < kNumRed; ++r)
@@ -2265,20 +2357,23 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
   }
   mark(3, 1);
   mark(4, 0);
-#define SPH_FORCE(F32, EX)                                                                     \
-  hipLaunchKernelGGL((k_force<F32, EX>), grd, dim3(256), 0, st, b.items, b.nitems, b.sims,     \
-                     (const void*)b.rec, b.fnew, b.nbr, b.kmax, force_mode, b.pos_cur, b.partials, \
-                     b.xyp)
-  if (b.prec == kPrecFP32C) SPH_FORCE(true, false);
-  else if (b.bitwise) SPH_FORCE(false, true);
-  else SPH_FORCE(false, false);
+  const int parts = b.bitwise || b.nitems > force_split_items(b.kmax) ? 1 : kSections;
+#define SPH_FORCE(F32, EX, P)                                                                  \
+  hipLaunchKernelGGL((k_force<F32, EX, P>), dim3(b.nitems * P), dim3(256), 0, st, b.items,      \
+                     b.nitems, b.sims, (const void*)b.rec, b.fnew, b.nbr, b.kmax, force_mode,  \
+                     b.pos_cur, b.partials, b.xyp)
+  if (b.bitwise) SPH_FORCE(false, true, 1);
+  else if (b.prec == kPrecFP32C && parts > 1) SPH_FORCE(true, false, kSections);
+  else if (b.prec == kPrecFP32C) SPH_FORCE(true, false, 1);
+  else if (parts > 1) SPH_FORCE(false, false, kSections);
+  else SPH_FORCE(false, false, 1);
 #undef SPH_FORCE
   mark(4, 1);
   mark(5, 0);
   if (b.red_parts_max > 1)
     hipLaunchKernelGGL(k_reduce_part, dim3(b.nsims * b.red_parts_max), dim3(256), 0, st, b.sims,
-                       b.partials, b.red_first, b.red_count, b.red_part, b.red_parts_max);
-  hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, b.red_part,
+                       b.partials, parts, b.red_first, b.red_count, b.red_part, b.red_parts_max);
+  hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, parts, b.red_part,
                      b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss);
   mark(5, 1);
   return (int)hipGetLastError();
