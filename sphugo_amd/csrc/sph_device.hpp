@@ -331,26 +331,15 @@ __device__ inline double kern_DF(int32_t kernel, double q) {
   if (q < 0.5) return (3 * q * q - 2 * q);
   return -(1 - q) * (1 - q);
 }
-// FP64 derivative with fused multiply-adds (the plain FP64 form's force,
-// whose contract is 1e-12 relative; the bitwise form keeps kern_DF)
-__device__ inline double kern_DF_fma(int32_t kernel, double q) {
-  if (kernel == kWendland) {
-    const double a = 1 - q;
-    return -10 * q * (a * a * a);
-  }
-  if (q < 0.5) return q * fma(3.0, q, -2.0);
-  const double a = 1 - q;
-  return -(a * a);
-}
-// FP32 forms (FP32C), fused multiply-adds where they fit.  The two pieces
-// of the cubic spline are both evaluated and one is selected: the lanes of
-// a wave take both sides anyway, and a select needs no exec-mask branch.
-// FP32 forms of each kernel type.  The type is per simulation, so loops
-// over neighbours are instantiated per type (kern_visit) rather than
-// branching on it per pair.
+// FP64 and FP32 forms of each kernel type, with fused multiply-adds (the
+// bitwise form keeps kern_F and kern_DF).  The type is per simulation, so
+// loops over neighbours are instantiated per type (kern_visit) rather than
+// branching on it per pair.  The two pieces of the cubic spline are both
+// evaluated, without an exec-mask branch: the lanes of a wave take both sides
+// anyway.  Its derivative, q (3 q - 2) below 1/2 and -(1 - q)^2 from there, is the
+// product of min(q, 1 - q) and min(3 q - 2, q - 1), which change over at the
+// same q.
 struct CubicF {
-  // FP64 kernel value with fused multiply-adds (the plain FP64 form's
-  // density, whose contract is 1e-12 relative; the bitwise form keeps kern_F)
   __device__ static double F64(double q) {
     const double a = 1 - q;
     const double lo = fma(q * q, q - 1, 1.0 / 6);
@@ -365,9 +354,11 @@ struct CubicF {
   }
   __device__ static float DF(float q) {
     const float a = 1.f - q;
-    const float lo = q * __builtin_fmaf(3.f, q, -2.f);
-    const float hi = -a * a;
-    return q < 0.5f ? lo : hi;
+    return __builtin_fminf(q, a) * __builtin_fminf(__builtin_fmaf(3.f, q, -2.f), -a);
+  }
+  __device__ static double DF64(double q) {
+    const double a = 1 - q;
+    return __builtin_fmin(q, a) * __builtin_fmin(fma(3.0, q, -2.0), -a);
   }
 };
 struct WendlandF {
@@ -384,6 +375,10 @@ struct WendlandF {
     const float a = 1.f - q;
     return -10.f * q * a * a * a;
   }
+  __device__ static double DF64(double q) {
+    const double a = 1 - q;
+    return -10 * q * (a * a * a);
+  }
 };
 __device__ inline float kern_Ff(int32_t kernel, float q) {
   return kernel == kWendland ? WendlandF::F(q) : CubicF::F(q);
@@ -398,23 +393,19 @@ __device__ inline void kern_visit(int32_t kernel, Fn&& f) {
   else f(CubicF{});
 }
 
-// FP64 reciprocal and reciprocal square root from the hardware estimates
-// refined by two Newton steps (explicit fma; results within about one ulp).
-// Used by the non-bitwise FP64 form, whose contract is 1e-12 relative.
+// FP64 reciprocal and reciprocal square root: the hardware's estimates (2^-24)
+// and one third-order step each, which leaves the rounding of its last
+// operations (within about one ulp).  Used by the non-bitwise FP64 form, whose
+// contract is 1e-12 relative.
 __device__ inline double rcp64(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, y, 1.0);
-  y = fma(y, e, y);
-  e = fma(-x, y, 1.0);
-  return fma(y, e, y);
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 __device__ inline double rsq64(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double hx = 0.5 * x;
-  double r = fma(-hx * y, y, 0.5);
-  y = fma(y, r, y);
-  r = fma(-hx * y, y, 0.5);
-  return fma(y, r, y);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
 // sqrt(x) / h for hinv near 1 / h: one Newton step on the reciprocal square

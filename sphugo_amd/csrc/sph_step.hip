@@ -1716,9 +1716,10 @@ __device__ inline void stage_window(u32x4* lds, const T* __restrict__ g, int64_t
 // are processed, so that the row and gather latencies overlap.  Full rounds
 // gather their entries as they are; a last partial round gathers the query's
 // own slot `self` for the entries past k.  NT: the row is read for the last
-// time (non-temporal loads).  `flush` runs after each round of N entries, with
-// the next round's first.
-template <int N, bool NT = false, typename S, typename Body, typename Flush>
+// time (non-temporal loads).  IMAGES: `body` is told (as a type) whether an
+// entry of the wave's round may be an image, which few waves' are.  `flush` runs
+// after each round of N entries, with the next round's first.
+template <int N, bool NT = false, bool IMAGES = false, typename S, typename Body, typename Flush>
 __device__ inline void row_visit(const NbrRow row, int n0, int k, uint32_t self, const S& src,
                                  Body body, Flush flush) {
   static_assert(N == 4 || N == 8, "one or two row chunks per round");
@@ -1741,8 +1742,18 @@ __device__ inline void row_visit(const NbrRow row, int n0, int k, uint32_t self,
       qa = ld((n0 + N) >> 2);
       if constexpr (N == 8) qb = n0 + 12 < k ? ld(((n0 + N) >> 2) + 1) : zero;
     }
+    auto round = [&](auto img) {
 #pragma unroll
-    for (int u = 0; u < N; ++u) body(pks[u], pj[u]);
+      for (int u = 0; u < N; ++u) body(pks[u], pj[u], img);
+    };
+    if constexpr (IMAGES) {
+      uint32_t im = 0;  // code 5: no image
+#pragma unroll
+      for (int u = 0; u < N; ++u) im |= pks[u] ^ 5u;
+      if (ballot(im & 15u)) round(std::true_type{}); else round(std::false_type{});
+    } else {
+      round(std::true_type{});
+    }
     flush(n0 + N);
   }
   if (n0 < k) {
@@ -1756,7 +1767,7 @@ __device__ inline void row_visit(const NbrRow row, int n0, int k, uint32_t self,
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       if (n0 + u >= k) break;
-      body(pks[u], pj[u]);
+      body(pks[u], pj[u], std::true_type{});
     }
     flush(n0 + N);
   }
@@ -1814,13 +1825,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 // reference's order when the list is sorted, BITWISE), then kick, drift 2,
 // periodic wrap and reflection (sim/sph.go:327-401,122-193).
 //
+// What bounds it: at 1M clustered, k = 64, FP64, a wave's chain of window reads,
+// far gathers and arithmetic with three waves per SIMD to overlap: the vector
+// units are busy 55 % of the time, LDS 40 %, the vector L1 50 %.  Halving the FP64
+// form's vector instructions (offsets only where a round holds an image,
+// viscosity and the spline's derivative without branches, third-order root and
+// reciprocal steps: 80 -> 37 per pair) took 50,021 particles at k = 32 from 21.2 to
+// 18.6 us, 100,000 from 25.8 to 22.9 and 262,144 from 40.5 to 39.2; 1M, whose
+// rows leave the window more often, stayed at 208.
+//
 // A row's terms are added up in four sections of whole chunks, and the four
 // sums in order (the bitwise form: straight through, as the reference), so that
 // both splits of the work give the same bits.  PARTS 1: a thread per particle,
 // the block's 256 particles sharing a window.  PARTS 4: a block takes 64
 // particles and each of its waves one section of their rows, for launches whose
 // time is one thread's chain of gathers: 2,200 particles at k = 32 FP64 16 -> 8 us,
-// at k = 64 27 -> 11; FP32C 13 -> 7 and 20 -> 8.
+// at k = 64 27 -> 11; FP32C 13 -> 7 and 20 -> 9.
 inline constexpr int kSections = 4;
 // The most items for PARTS 4, whose smaller windows hold fewer of the
 // neighbours and are staged four times as often.  FP64 force (with the event
@@ -1864,14 +1884,15 @@ __global__ __launch_bounds__(256) void k_force(
   const int kern = S->kernel;
   const double dt = S->dt_half;
   if (mode < 0) mode = S->fmode;
-  // the block's window of neighbour records in LDS: slots [first - 128,
-  // first + 384) (16 KB FP32C, 32 KB FP64), which hold about 85 % of the
-  // neighbours of Hilbert-ordered particles; the rest are gathered from
-  // memory.  Force time at 4M clustered, k = 64: FP64 1.17 -> 0.87 ms,
-  // FP32C 0.57 -> 0.49 ms (with 4 records in flight instead of 8).  The same
-  // around 64 particles: half the slots.
-  constexpr int kWin = PARTS == 1 ? 512 : 256;
-  constexpr int kBack = PARTS == 1 ? 128 : 96;
+  // The block's window of neighbour records in LDS, which holds most of the
+  // neighbours of Hilbert-ordered particles; the rest are gathered from memory.
+  // As wide as its registers' waves leave room for in LDS: 640 slots from first -
+  // 192 in FP64 (40 KB, three waves per SIMD), 896 from first - 320 in FP32C (28 KB,
+  // five; the bitwise form, four, 512).  Against 512 from first - 128: 1M clustered at k = 64 FP64 208 -> 206 us,
+  // 4M FP32C 473 -> 458; 1,024 in FP32C (LDS for four waves) 501.  Around 64
+  // particles 256 slots.
+  constexpr int kWin = PARTS > 1 ? 256 : (FP32C ? 896 : (EXACT ? 512 : 640));
+  constexpr int kBack = PARTS > 1 ? 96 : (FP32C ? 320 : (EXACT ? 128 : 192));
   using Rec = std::conditional_t<FP32C, RecF, RecD>;
   __shared__ u32x4 wrec[kWin * sizeof(Rec) / 16];
   const int64_t wb = it.first + (PARTS == 1 ? 0 : (blk % PARTS) * kParticles) - kBack;
@@ -1894,13 +1915,22 @@ __global__ __launch_bounds__(256) void k_force(
     const double alpha = S->alpha, beta = S->beta, eta2 = S->eta2;
     const double hinv = EXACT ? 0.0 : 1.0 / hi;
     // 4 records (64 B each) in flight per lane, the next row chunk behind them
-    row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb) {
-      const double ox = (double)img_ix(pk & 15u) * lx, oy = (double)img_iy(pk & 15u) * ly;
-      const double rABx = (nb.x - ox) - xi, rABy = (nb.y - oy) - yi;
-      const double vABx = nb.vpx - vpxi, vABy = nb.vpy - vpyi;
-      if constexpr (EXACT) {
+    auto flush = [&](int n) {
+      if (!EXACT && PARTS == 1 && n == total.end) {
+        total.x += sx;
+        total.y += sy;
+        total.e += se;
+        sx = sy = se = 0.0;
+        total.next(k);
+      }
+    };
+    if constexpr (EXACT) {
+      row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb, auto) {
         // the reference's arithmetic, operation for operation
+        const double ox = (double)img_ix(pk & 15u) * lx, oy = (double)img_iy(pk & 15u) * ly;
+        const double rABx = (nb.x - ox) - xi, rABy = (nb.y - oy) - yi;
         const double ex = (xi + ox) - nb.x, ey = (yi + oy) - nb.y;
+        const double vABx = nb.vpx - vpxi, vABy = nb.vpy - vpyi;
         const double d2 = ex * ex + ey * ey;
         const double dot = vABx * rABx + vABy * rABy;
         const double d = sqrt(d2);
@@ -1917,39 +1947,40 @@ __global__ __launch_bounds__(256) void k_force(
         sx += rABx * (piAB + A + nb.B) * dR / d;
         sy += rABy * (piAB + A + nb.B) * dR / d;
         se += dot * dR;
-      } else {
+      }, flush);
+    } else {
+      // within the 1e-12 contract of this form: the distance from r_AB (one
+      // rounding away from the query-side difference) and fused multiply-adds
+      // throughout
+      const double acih = alpha * cih;
+      kern_visit(kern, [&](auto kt) {
+        row_visit<4, true, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb,
+                                                                     auto img) {
 #pragma clang fp contract(fast)
-        // within the 1e-12 contract of this form: the distance from r_AB
-        // (one rounding away from the query-side difference) and fused
-        // multiply-adds throughout
-        const double r2 = rABx * rABx + rABy * rABy;
-        const double dot = vABx * rABx + vABy * rABy;
-        const double rinv = rsq64(r2);
-        const double q = (r2 * rinv) * hinv;
-        const double dR = kern_DF_fma(kern, q);
-        double piAB = 0.0;
-        if (dot < 0) {
-          // pi = mu (beta mu - alpha cAB) / rhoAB with one reciprocal:
-          // t = mu / rhoAB = dot hAB / ((r^2 + eta2) rhoAB)
+          double rABx = nb.x - xi, rABy = nb.y - yi;
+          if constexpr (decltype(img)::value) {
+            rABx = (nb.x - (double)img_ix(pk & 15u) * lx) - xi;
+            rABy = (nb.y - (double)img_iy(pk & 15u) * ly) - yi;
+          }
+          const double vABx = nb.vpx - vpxi, vABy = nb.vpy - vpyi;
+          const double r2 = rABx * rABx + rABy * rABy;
+          const double dot = vABx * rABx + vABy * rABy;
+          const double rinv = rsq64(r2);
+          const double q = (r2 * rinv) * hinv;
+          const double dR = decltype(kt)::DF64(q);
+          // viscosity where the pair approaches, for every pair from
+          // min(dot, 0): pi = mu (beta mu - alpha cAB) / rhoAB with one
+          // reciprocal, t = mu / rhoAB = dot hAB / ((r^2 + eta2) rhoAB)
           const double rhoAB = rhoih + nb.rho;
-          const double t = dot * (hih + nb.h) * rcp64((r2 + eta2) * rhoAB);
-          const double muAB = t * rhoAB;
-          piAB = (beta * muAB - alpha * (cih + nb.c)) * t;
-        }
-        const double w = (piAB + A + nb.B) * dR * rinv;
-        sx += rABx * w;
-        sy += rABy * w;
-        se += dot * dR;
-      }
-    }, [&](int n) {
-      if (!EXACT && PARTS == 1 && n == total.end) {
-        total.x += sx;
-        total.y += sy;
-        total.e += se;
-        sx = sy = se = 0.0;
-        total.next(k);
-      }
-    });
+          const double v = __builtin_fmin(dot, 0.0) * (hih + nb.h) * rcp64((r2 + eta2) * rhoAB);
+          const double x = beta * (v * rhoAB) - (alpha * nb.c + acih);
+          const double w = (x * v + (A + nb.B)) * dR * rinv;
+          sx += rABx * w;
+          sy += rABy * w;
+          se += dot * dR;
+        }, flush);
+      });
+    }
     if constexpr (!EXACT && PARTS == 1) {
       sx = total.x;
       sy = total.y;
@@ -1971,9 +2002,10 @@ __global__ __launch_bounds__(256) void k_force(
     rhoi = 2.0 * (double)me.rho;
     A = (double)me.B;
     // own rho, c, h halved as stored (the pair means are sums of halves)
-    const float vpxi = me.vpx, vpyi = me.vpy, cif = me.c, rhoif = me.rho, hif = me.h, Af = me.B;
+    const float vpxi = me.vpx, vpyi = me.vpy, rhoif = me.rho, hif = me.h, Af = me.B;
     const float hinv = __builtin_amdgcn_rcpf(2.0f * hif);
     const float alpha = (float)S->alpha, beta = (float)S->beta, eta2 = (float)S->eta2;
+    const float acif = alpha * me.c;
     // block-compensated sums (a Kahan step per round of 4 neighbours)
     BlockKahan ax_, ay_, ae_;
     auto flush = [&](int n) {
@@ -2011,14 +2043,14 @@ __global__ __launch_bounds__(256) void k_force(
         // both sides anyway): mu = dot hAB / (r^2 + eta2),
         // pi = mu (beta mu - alpha cAB) / rhoAB, with one reciprocal of
         // (r^2 + eta2) rhoAB
-        const float cAB = cif + nb.c;
+        const float acAB = __builtin_fmaf(alpha, nb.c, acif);
         const float rhoAB = rhoif + nb.rho;
         const float hAB = hif + nb.h;
         const float a_ = __builtin_fminf(dot, 0.f) * hAB;
         const float inv = __builtin_amdgcn_rcpf((d2 + eta2) * rhoAB);
         const float muAB = a_ * inv * rhoAB;
-        const float piAB = __builtin_fmaf(beta, muAB, -alpha * cAB) * (a_ * inv);
-        const float w = (piAB + Af + nb.B) * dR * dinv;
+        const float piAB = __builtin_fmaf(beta, muAB, -acAB) * (a_ * inv);
+        const float w = (piAB + (Af + nb.B)) * dR * dinv;
         ax_.add_mul(rx, w);
         ay_.add_mul(ry, w);
         ae_.add_mul(dot, dR);
@@ -2028,12 +2060,12 @@ __global__ __launch_bounds__(256) void k_force(
       // wave whose queries all take fixed-point displacements (the usual case)
       // runs a loop without the FP64 form, so every record loads whole.
       if (__all(fixed)) {
-        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t, const RecF& nb) {
+        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t, const RecF& nb, auto) {
           pair(__builtin_fmaf((float)(int32_t)(nb.ux - me.ux), fsx, csx),
                __builtin_fmaf((float)(int32_t)(nb.uy - me.uy), fsy, csy), nb);
         }, flush);
       } else {
-        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecF& nb) {
+        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecF& nb, auto) {
           float rx, ry;
           if (fixed) {
             rx = __builtin_fmaf((float)(int32_t)(nb.ux - me.ux), fsx, csx);
