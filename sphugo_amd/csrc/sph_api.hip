@@ -262,7 +262,7 @@ static int create_batch(int count, const sph_params* const* ps, const int64_t* n
   std::vector<int> red_first(count), red_count(count);
   for (int s = 0; s < count; ++s) {
     SimDev d;
-    const int lg = grid_log2(ns[s], 4.0);
+    const int lg = grid_log2(ns[s], kGridCpp);
     fill_simdev(d, ps[s], ns[s], lg);
     if (d.open) {
       if (!xs[s] || !ys[s]) return bail(fail(SPH_EINVAL, "positions must not be null"));
@@ -292,7 +292,7 @@ static int create_batch(int count, const sph_params* const* ps, const int64_t* n
   }
   if (coff >= (1LL << 32) - 1) return bail(fail(SPH_EINVAL, "too many cells"));
   h->cell_capacity = coff + 1;
-  layout_cells(h, 4.0);
+  layout_cells(h, kGridCpp);
   PassBuffers& pb = h->pb;
   pb.nsims = count;
   pb.nitems = (int)h->hitems.size();

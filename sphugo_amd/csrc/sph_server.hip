@@ -222,7 +222,7 @@ int upload_job(sph_server* s, Job* j) {
   const hipStream_t st = c.st;
   const int64_t n = j->n, o = j->off;
   SimDev& d = s->hsim[j->slot];
-  fill_simdev(d, &j->p, n, grid_log2(n, 4.0));
+  fill_simdev(d, &j->p, n, grid_log2(n, kGridCpp));
   init_open_box(d, j->in.data(), j->in.data() + n, n);
   d.off = o;
   d.coff = o * kHoleCpp + 1;

@@ -167,5 +167,13 @@ int enqueue_flags(sph_sim* s, int nerr);
 void take_flags(sph_sim* s, sph::KnnStats* stats, int* err, int nerr);
 int check_device_flags(sph_sim* s);
 int alloc_state(sph_sim* h, int64_t np, int nitems);
+// Cells per particle of a grid (at least; at most four times as many, as a
+// grid's size is a power of four) unless tuning chose another.  The walk looks
+// at cells of several particles, so the finest ones serve regions denser than
+// the mean, and their number costs key bits and cell ranges: per pass with 4
+// and 2 per particle, us: 77,777 uniform 114 and 107, 100,000 clustered at k = 64
+// 167 and 163, 524,288 clustered 356 and 346; sizes whose grid is the same either
+// way (262,144, 1,048,576) alike.  With 1, 1,048,576 clustered take 634 against 603.
+inline constexpr double kGridCpp = 2.0;
 int grid_log2(int64_t n, double cpp);
 }  // namespace sph
