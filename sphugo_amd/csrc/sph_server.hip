@@ -4,8 +4,8 @@
 // The pool holds `capacity` particle slots.  A job occupies a contiguous
 // range [off, off + n) and a simulation slot (its SimDev); unused ranges are
 // holes.  Every tick runs ONE force pass over the whole pool: the radix sort
-// keys a job's particles by coff + Hilbert(cell) with coff = off * 16 + 1 and a
-// hole slot t by t * 16, so the sort keeps every job inside its own range and
+// keys a job's particles by coff + Hilbert(cell) with coff = off * 8 + 1 and a
+// hole slot t by t * 8, so the sort keeps every job inside its own range and
 // every hole in place, and each job's cells never collide with another's.
 // Each job carries its own pass modes (first pass: initial kNN + forces
 // without a kick; then regular passes = one reference Step each), so jobs at
@@ -17,7 +17,7 @@
 // Admission is FIFO: the head of the queue waits until a slot and a
 // first-fit range of n slots are free.  One native worker thread owns the
 // device; clients submit and wait from any thread.  The cell grid of a job
-// is the one a standalone handle uses (about 4 cells per particle), so a job
+// is the one a standalone handle uses (2 to 8 cells per particle), so a job
 // produces exactly the results of sph_create + sph_step with the same
 // parameters, whatever else shares the pool.
 #include <hip/hip_runtime.h>
@@ -29,7 +29,9 @@
 #include <cstring>
 #include <deque>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -39,9 +41,11 @@ using namespace sph;
 
 namespace {
 
-constexpr uint32_t kHoleCpp = 16;  // cell keys reserved per pool slot
+constexpr uint32_t kHoleCpp = 8;   // cell keys reserved per pool slot
+static_assert(kHoleCpp >= 4 * kGridCpp, "a grid has fewer than 4 kGridCpp cells per particle");
 constexpr int kNumRes = 7;         // fields kept for a finished job
 constexpr int kResFields[kNumRes] = {SPH_X, SPH_Y, SPH_VX, SPH_VY, SPH_RHO, SPH_E, SPH_H};
+constexpr int kNumJobRed = kNumRed + 2;  // and dt_last, |v| of the last particle
 
 using Clock = std::chrono::steady_clock;
 
@@ -60,14 +64,13 @@ struct Job {
   sph_params p = {};
   int64_t n = 0;
   int32_t nsteps = 0;
-  std::vector<double> in;  // x, y, vx, vy, e: 5 rows of n
+  std::unique_ptr<double[]> in;   // x, y, vx, vy, e: 5 rows of n
   int32_t state = SPH_JOB_QUEUED;
   int slot = -1;
   int64_t off = -1;
   int32_t passes = 0;  // passes completed; the job ends after nsteps + 1
   Clock::time_point t_submit, t_start, t_done;
-  std::vector<double> out;  // kNumRes rows of n
-  double red[7] = {};       // reductions (sum e, sum rho, E, Px, Py, dt_last), |v| last
+  std::unique_ptr<double[]> out;  // kNumRes rows of n, then kNumJobRed reductions
   std::string error;
 };
 
@@ -93,15 +96,13 @@ struct sph_server {
   std::vector<Job*> slots;                          // running job per slot
   std::vector<std::pair<int64_t, int64_t>> holes;   // free ranges (off, len), sorted
   std::vector<SimDev> hsim;                         // host copy of each slot's SimDev
-  std::vector<SimDev> hsim_rb;                      // readback of finishing slots
-  std::vector<Item> h_items, h_items_all;
+  // first item and item count of each slot, then the work items of the jobs
+  // (grouped by slot) and of the holes: one upload
+  std::vector<Item> h_items;
   std::vector<int> h_rf, h_rc;
-  std::vector<uint32_t> iota;
-  Item* d_items = nullptr;
-  Item* d_items_all = nullptr;
-  int* d_rf = nullptr;
-  int* d_rc = nullptr;
-  double* d_stage = nullptr;  // kNumRes rows of capacity
+  std::vector<char> h_table;
+  char* d_table = nullptr;
+  double* d_stage = nullptr;  // one job's inputs or results
   std::vector<int> h_err;  // error flags: [0] any, [1 + slot] per job slot
   KnnStats h_stats = {};
   unsigned long long seen_failures = 0;
@@ -109,7 +110,6 @@ struct sph_server {
   // start of the next one (host buffers of a pending copy are not reused)
   std::vector<int> to_clear;
   bool items_dirty = false;
-  SimDev zero_sim = {};
 
   // statistics
   int64_t n_done = 0, n_failed = 0, particle_steps = 0, ticks = 0;
@@ -171,10 +171,12 @@ void push_items(std::vector<Item>& v, int sim, int64_t off, int64_t n) {
 
 int64_t max_items(int64_t cap, int max_jobs) { return cap / kItem + 3 * (int64_t)max_jobs + 4; }
 
+// Byte offset of the items in the table of work items.
+size_t table_items(int max_jobs) { return ((size_t)2 * max_jobs * sizeof(int) + 15) & ~(size_t)15; }
+
 // Work items of the running jobs (grouped by slot), plus the holes.
 int upload_items(sph_server* s) {
   s->h_items.clear();
-  s->h_items_all.clear();
   std::fill(s->h_rf.begin(), s->h_rf.end(), 0);
   std::fill(s->h_rc.begin(), s->h_rc.end(), 0);
   for (int q = 0; q < s->max_jobs; ++q) {
@@ -189,91 +191,113 @@ int upload_items(sph_server* s) {
   int64_t hi = 0;
   for (Job* j : s->slots)
     if (j && j->off + j->n > hi) hi = j->off + j->n;
-  s->h_items_all = s->h_items;
-  for (auto& h : s->holes)
-    if (h.first < hi) push_items(s->h_items_all, -1, h.first, std::min(h.second, hi - h.first));
   PassBuffers& pb = s->core.pb;
+  pb.nitems = (int)s->h_items.size();
+  for (auto& h : s->holes)
+    if (h.first < hi) push_items(s->h_items, -1, h.first, std::min(h.second, hi - h.first));
+  pb.nitems_all = (int)s->h_items.size();
   pb.any_open = 0;
   pb.red_parts_max = 1;
   for (int q = 0; q < s->max_jobs; ++q) {
     if (s->slots[q] && s->hsim[q].open) pb.any_open = 1;
     pb.red_parts_max = std::max(pb.red_parts_max, red_parts(s->h_rc[q]));
   }
-  pb.nitems = (int)s->h_items.size();
-  pb.nitems_all = (int)s->h_items_all.size();
   pb.np = hi;
   int bits = 1;
-  while ((1LL << bits) < hi * (int64_t)kHoleCpp) ++bits;  // keys lie in [0, 16 hi)
+  while ((1LL << bits) < hi * (int64_t)kHoleCpp) ++bits;  // keys lie in [0, 8 hi)
   pb.key_bits = bits;
-  const hipStream_t st = s->core.st;
-  HIPCHK(hipMemcpyAsync(s->d_items, s->h_items.data(), s->h_items.size() * sizeof(Item),
-                        hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(s->d_items_all, s->h_items_all.data(),
-                        s->h_items_all.size() * sizeof(Item), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(s->d_rf, s->h_rf.data(), s->max_jobs * sizeof(int), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(s->d_rc, s->h_rc.data(), s->max_jobs * sizeof(int), hipMemcpyHostToDevice, st));
+  const size_t rows = s->max_jobs * sizeof(int), items = s->h_items.size() * sizeof(Item);
+  const size_t at = table_items(s->max_jobs);
+  s->h_table.resize(at + items);
+  std::memcpy(s->h_table.data(), s->h_rf.data(), rows);
+  std::memcpy(s->h_table.data() + rows, s->h_rc.data(), rows);
+  std::memcpy(s->h_table.data() + at, s->h_items.data(), items);
+  HIPCHK(hipMemcpyAsync(s->d_table, s->h_table.data(), at + items, hipMemcpyHostToDevice,
+                        s->core.st));
   return 0;
 }
 
-// Place an admitted job's particles in its range (IDs 0..n-1 in input
-// order) and its parameters in its slot.
+// Admission and completion of a job take one copy and one launch each, in
+// place of 16 and 15: while the pool waits for a job's arrays nothing runs,
+// and every copy or launch cost it 5 to 30 us.
+
+// An admitted job's particles into its range (IDs 0..n-1 in input order, the
+// rest zero), its parameters into its slot.  in: x, y, vx, vy, e.
+__global__ __launch_bounds__(kItem) void k_place_job(const double* __restrict__ in, int64_t n,
+                                                     int64_t off, Positions p, Fields f, SimDev d,
+                                                     SimDev* __restrict__ sim) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *sim = d;
+  const int64_t i = (int64_t)blockIdx.x * kItem + threadIdx.x, t = off + i;
+  if (i >= n) return;
+  p.x[t] = in[i];
+  p.y[t] = in[n + i];
+  f.vx[t] = in[2 * n + i];
+  f.vy[t] = in[3 * n + i];
+  f.e[t] = in[4 * n + i];
+  f.id[t] = (uint32_t)i;
+  double* zero[] = {f.ax, f.ay, f.edot, f.vpx, f.vpy, f.ep, f.h, f.rho, f.c};
+#pragma unroll
+  for (double* a : zero) a[t] = 0.0;
+}
+
+// A job's results by ID, a row of n per kResFields, and its reductions.
+__global__ __launch_bounds__(kItem) void k_read_job(const Item* __restrict__ items, int64_t n,
+                                                    Positions p, Fields f,
+                                                    const SimDev* __restrict__ sim,
+                                                    double* __restrict__ out) {
+  const Item it = items[blockIdx.x];
+  if (blockIdx.x == 0 && threadIdx.x < kNumJobRed)
+    out[kNumRes * n + threadIdx.x] = threadIdx.x < kNumRed       ? sim->red[threadIdx.x]
+                                     : threadIdx.x == kNumRed ? sim->dt_last
+                                                              : sim->last_speed;
+  if ((int)threadIdx.x >= it.count) return;
+  const int64_t t = it.first + threadIdx.x, i = f.id[t];
+  out[i] = p.x[t];
+  out[n + i] = p.y[t];
+  out[2 * n + i] = f.vx[t];
+  out[3 * n + i] = f.vy[t];
+  out[4 * n + i] = f.rho[t];
+  out[5 * n + i] = f.e[t];
+  out[6 * n + i] = f.h[t];
+}
+
 int upload_job(sph_server* s, Job* j) {
   sph_sim& c = s->core;
-  const hipStream_t st = c.st;
-  const int64_t n = j->n, o = j->off;
+  const int64_t n = j->n;
   SimDev& d = s->hsim[j->slot];
   fill_simdev(d, &j->p, n, grid_log2(n, kGridCpp));
-  init_open_box(d, j->in.data(), j->in.data() + n, n);
-  d.off = o;
-  d.coff = o * kHoleCpp + 1;
-  d.pmode = kPermInit;
+  init_open_box(d, j->in.get(), j->in.get() + n, n);
+  d.off = j->off;
+  d.coff = j->off * kHoleCpp + 1;
+  d.pmode = kPermInit;  // regular steps from the second pass on (k_reduce)
   d.fmode = kForceNoKick;
   const double inf = INFINITY;
   std::memcpy(&d.cfl_min_bits, &inf, sizeof inf);
-  HIPCHK(hipMemcpyAsync(c.pb.sims + j->slot, &d, sizeof d, hipMemcpyHostToDevice, st));
-  const size_t b = n * sizeof(double);
-  const Fields& f = c.F[c.cur];
-  HIPCHK(hipMemcpyAsync(c.P[0].x + o, j->in.data(), b, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(c.P[0].y + o, j->in.data() + n, b, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(f.vx + o, j->in.data() + 2 * n, b, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(f.vy + o, j->in.data() + 3 * n, b, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(f.e + o, j->in.data() + 4 * n, b, hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(f.id + o, s->iota.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, st));
-  double* zero[] = {f.ax, f.ay, f.edot, f.vpx, f.vpy, f.ep, f.h, f.rho, f.c};
-  for (double* a : zero) HIPCHK(hipMemsetAsync(a + o, 0, b, st));
-  return 0;
-}
-
-// After its first pass a job switches to regular steps.
-int upload_modes(sph_server* s, int slot) {
-  SimDev& d = s->hsim[slot];
-  d.pmode = kPermPredict;
-  d.fmode = kForceKick;
-  char* dst = (char*)(s->core.pb.sims + slot) + offsetof(SimDev, pmode);
-  HIPCHK(hipMemcpyAsync(dst, &d.pmode, 2 * sizeof(int32_t), hipMemcpyHostToDevice, s->core.st));
+  HIPCHK(hipMemcpyAsync(s->d_stage, j->in.get(), 5 * n * sizeof(double), hipMemcpyHostToDevice,
+                        c.st));
+  hipLaunchKernelGGL(k_place_job, dim3((unsigned)((n + kItem - 1) / kItem)), dim3(kItem), 0, c.st,
+                     s->d_stage, n, j->off, c.P[0], c.F[c.cur], d, c.pb.sims + j->slot);
+  HIPCHK(hipGetLastError());
   return 0;
 }
 
 int clear_slot(sph_server* s, int slot) {
-  HIPCHK(hipMemcpyAsync(s->core.pb.sims + slot, &s->zero_sim, sizeof(SimDev),
-                        hipMemcpyHostToDevice, s->core.st));
+  HIPCHK(hipMemsetAsync(s->core.pb.sims + slot, 0, sizeof(SimDev), s->core.st));
   return 0;
 }
 
-// Fields and reductions of a job whose last pass was just enqueued.
-int enqueue_readback(sph_server* s, Job* j) {
+// Fields and reductions of a job whose last pass was just enqueued; returns
+// when they are there.
+int read_back(sph_server* s, Job* j) {
   sph_sim& c = s->core;
-  j->out.resize((size_t)kNumRes * j->n);
-  for (int r = 0; r < kNumRes; ++r) {
-    double* dst = s->d_stage + (int64_t)r * s->cap + j->off;
-    int rc = enqueue_read_field(c.pb, kResFields[r], j->slot, dst, c.st);
-    if (rc) return fail(SPH_EDEVICE, "readback launch: %s", hipGetErrorString((hipError_t)rc));
-    HIPCHK(hipMemcpyAsync(j->out.data() + (size_t)r * j->n, dst, j->n * sizeof(double),
-                          hipMemcpyDeviceToHost, c.st));
-  }
-  HIPCHK(hipMemcpyAsync(&s->hsim_rb[j->slot], c.pb.sims + j->slot, sizeof(SimDev),
-                        hipMemcpyDeviceToHost, c.st));
-  return 0;
+  const size_t len = (size_t)kNumRes * j->n + kNumJobRed;
+  j->out.reset(new (std::nothrow) double[len]);
+  if (!j->out) return fail(SPH_ENOMEM, "no memory for the results of %lld particles", (long long)j->n);
+  hipLaunchKernelGGL(k_read_job, dim3(s->h_rc[j->slot]), dim3(kItem), 0, c.st,
+                     c.pb.items + s->h_rf[j->slot], j->n, c.pb.pos_cur, c.pb.fcur,
+                     c.pb.sims + j->slot, s->d_stage);
+  HIPCHK(hipGetLastError());
+  return copy_out(&c, j->out.get(), s->d_stage, len * sizeof(double));
 }
 
 void fail_job(sph_server* s, Job* j, const std::string& msg) {
@@ -331,7 +355,6 @@ bool tick(sph_server* s) {
   for (Job* j : s->slots) {
     if (!j || rc) continue;
     occupied += j->n;
-    if (j->passes == 1) rc = upload_modes(s, j->slot);
     if (j->passes + 1 == j->nsteps + 1) finishing.push_back(j);
   }
   if (!rc) {
@@ -343,7 +366,7 @@ bool tick(sph_server* s) {
     c.bind();
   }
   for (Job* j : finishing)
-    if (!rc) rc = enqueue_readback(s, j);
+    if (!rc) rc = read_back(s, j);
   if (!rc) {
     rc = enqueue_flags(&c, (int)s->h_err.size());
     hipError_t e = hipSuccess;
@@ -402,10 +425,6 @@ bool tick(sph_server* s) {
     if (j->state == SPH_JOB_RUNNING) {
       j->passes += 1;
       if (j->passes < j->nsteps + 1) continue;
-      const SimDev& d = s->hsim_rb[q];
-      for (int r = 0; r < kNumRed; ++r) j->red[r] = d.red[r];
-      j->red[5] = d.dt_last;
-      j->red[6] = d.last_speed;
       j->state = SPH_JOB_DONE;
       j->t_done = now;
       s->n_done += 1;
@@ -488,16 +507,15 @@ extern "C" int sph_server_create(int64_t capacity, int32_t max_jobs, int32_t kma
   c.cell_capacity = pb.ncells + 1;
   SimDev* d_sims = nullptr;
   int rc = 0;
-  if ((rc = c.alloc(&s->d_items, nmax)) || (rc = c.alloc(&s->d_items_all, nmax)) ||
-      (rc = c.alloc(&d_sims, max_jobs)) || (rc = c.alloc(&s->d_rf, max_jobs)) ||
-      (rc = c.alloc(&s->d_rc, max_jobs)) || (rc = alloc_state(&c, capacity, (int)nmax)) ||
-      (rc = c.alloc(&s->d_stage, (int64_t)kNumRes * capacity)))
+  if ((rc = c.alloc(&s->d_table, (int64_t)(table_items(max_jobs) + nmax * sizeof(Item)))) ||
+      (rc = c.alloc(&d_sims, max_jobs)) || (rc = alloc_state(&c, capacity, (int)nmax)) ||
+      (rc = c.alloc(&s->d_stage, (int64_t)kNumRes * capacity + kNumJobRed)))
     return bail(rc);
-  pb.items = s->d_items;
-  pb.items_all = s->d_items_all;
+  pb.red_first = (int*)s->d_table;
+  pb.red_count = pb.red_first + max_jobs;
+  pb.items = (Item*)(s->d_table + table_items(max_jobs));
+  pb.items_all = pb.items;  // the jobs' come first
   pb.sims = d_sims;
-  pb.red_first = s->d_rf;
-  pb.red_count = s->d_rc;
   pb.nitems = 0;
   pb.nitems_all = 0;
   if (hipMemsetAsync(d_sims, 0, max_jobs * sizeof(SimDev), c.st) != hipSuccess ||
@@ -511,11 +529,8 @@ extern "C" int sph_server_create(int64_t capacity, int32_t max_jobs, int32_t kma
   s->slots.assign(max_jobs, nullptr);
   s->h_err.assign(1 + max_jobs, 0);
   s->hsim.assign(max_jobs, SimDev{});
-  s->hsim_rb.assign(max_jobs, SimDev{});
   s->h_rf.assign(max_jobs, 0);
   s->h_rc.assign(max_jobs, 0);
-  s->iota.resize(capacity);
-  for (int64_t i = 0; i < capacity; ++i) s->iota[i] = (uint32_t)i;
   s->holes.push_back({0, capacity});
   for (auto& e : s->ev_tick)
     if (hipEventCreate(&e) != hipSuccess) return bail(fail(SPH_EDEVICE, "hipEventCreate failed"));
@@ -557,10 +572,17 @@ extern "C" int sph_server_submit(sph_server* s, const sph_params* p, int64_t n, 
   j->p = *p;
   j->n = n;
   j->nsteps = nsteps;
-  j->in.assign((size_t)5 * n, 0.0);
+  j->in.reset(new (std::nothrow) double[(size_t)5 * n]);
+  if (!j->in) {
+    delete j;
+    return fail(SPH_ENOMEM, "no memory for a job of %lld particles", (long long)n);
+  }
   const double* src[5] = {x, y, vx, vy, e};
-  for (int r = 0; r < 5; ++r)
-    if (src[r]) std::memcpy(j->in.data() + (size_t)r * n, src[r], n * sizeof(double));
+  for (int r = 0; r < 5; ++r) {
+    double* row = j->in.get() + (size_t)r * n;
+    if (src[r]) std::memcpy(row, src[r], n * sizeof(double));
+    else std::fill(row, row + n, 0.0);
+  }
   for (int64_t i = 0; i < 2 * n; ++i)
     if (!std::isfinite(j->in[i])) {
       delete j;
@@ -637,7 +659,7 @@ extern "C" int sph_server_read_result(sph_server* s, int64_t job_id, int32_t fie
   if (j->state != SPH_JOB_DONE) return fail(SPH_ESTATE, "job %lld has not finished", (long long)job_id);
   const int r = res_index(field);
   if (r < 0) return fail(SPH_EINVAL, "field %d is not kept for finished jobs", field);
-  std::memcpy(out, j->out.data() + (size_t)r * j->n, j->n * sizeof(double));
+  std::memcpy(out, j->out.get() + (size_t)r * j->n, j->n * sizeof(double));
   return 0;
 }
 
@@ -647,7 +669,7 @@ extern "C" int sph_server_job_reductions(sph_server* s, int64_t job_id, double o
   Job* j = find_job(s, job_id);
   if (!j) return fail(SPH_EINVAL, "unknown job %lld", (long long)job_id);
   if (j->state != SPH_JOB_DONE) return fail(SPH_ESTATE, "job %lld has not finished", (long long)job_id);
-  for (int r = 0; r < 7; ++r) out[r] = j->red[r];
+  std::memcpy(out, j->out.get() + (size_t)kNumRes * j->n, kNumJobRed * sizeof(double));
   return 0;
 }
 

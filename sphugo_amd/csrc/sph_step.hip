@@ -2259,7 +2259,8 @@ __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
   __shared__ uint32_t miss[2][kMissSlots];
   SimDev* S = sims + blockIdx.x;
   if (S->n == 0) return;  // unused slot
-  if (mode < 0) mode = S->fmode;
+  const bool per_sim = mode < 0;
+  if (per_sim) mode = S->fmode;
   const int tid = threadIdx.x;
   // the walk's miss counts of this pass (copy q by thread q), read and
   // cleared for the next pass
@@ -2295,6 +2296,10 @@ __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
     for (int r = 0; r < kNumRed; ++r) S->red[r] = sh[r][0];
     S->last_speed = sqrt(vx_last * vx_last + vy_last * vy_last);
     if (mode == kForceKick) S->dt_last = S->dt_half;
+    if (per_sim) {  // regular steps after a job's first pass
+      S->pmode = kPermPredict;
+      S->fmode = kForceKick;
+    }
     uint32_t move = 0u, wide = 0u;
     for (int q = 0; q < kMissSlots; ++q) {
       move += miss[0][q];
