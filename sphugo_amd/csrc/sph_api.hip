@@ -628,9 +628,22 @@ extern "C" int sph_calculate_forces(sph_sim* s) {
   return sph_synchronize(s);
 }
 
+// One simulation's field: small ones in one launch by a block that orders them
+// in LDS, others scattered by ID and copied on.
+static int read_field_of(sph_sim* s, int sim, int field, double* out) {
+  s->bind();
+  const int64_t n = s->sim_n[sim], off = s->hsims[sim].off;
+  if (n <= kOrderedMax)
+    return read_ordered(s, out, field_data(s->pb, field) + off, s->pb.fcur.id + off, (int)n);
+  if (enqueue_read_field(s->pb, field, sim, s->d_scratch, s->st))
+    return fail(SPH_EDEVICE, "readback launch failed");
+  return copy_out(s, out, s->d_scratch, n * sizeof(double));
+}
+
 extern "C" int sph_read_field(sph_sim* s, int32_t field, double* out) {
   if (!s || !out) return fail(SPH_EINVAL, "null argument");
   if (field < 0 || field >= SPH_NFIELDS) return fail(SPH_EINVAL, "unknown field %d", field);
+  if (s->hsims.size() == 1) return read_field_of(s, 0, field, out);
   s->bind();
   int rc = enqueue_read_field(s->pb, field, -1, s->d_scratch, s->st);
   if (rc) return fail(SPH_EDEVICE, "readback launch failed");
@@ -798,10 +811,7 @@ extern "C" int sph_batch_read_field(sph_sim* s, int32_t sim, int32_t field, doub
   if (!s || !out) return fail(SPH_EINVAL, "null argument");
   if (sim < 0 || sim >= (int32_t)s->hsims.size()) return fail(SPH_EINVAL, "no simulation %d", sim);
   if (field < 0 || field >= SPH_NFIELDS) return fail(SPH_EINVAL, "unknown field %d", field);
-  s->bind();
-  if (enqueue_read_field(s->pb, field, sim, s->d_scratch, s->st))
-    return fail(SPH_EDEVICE, "readback launch failed");
-  return copy_out(s, out, s->d_scratch, s->sim_n[sim] * sizeof(double));
+  return read_field_of(s, sim, field, out);
 }
 
 extern "C" int sph_batch_write_field(sph_sim* s, int32_t sim, int32_t field, const double* in) {

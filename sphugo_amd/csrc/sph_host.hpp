@@ -84,6 +84,8 @@ inline int64_t nbr_entries(int64_t np, int kstride) { return (np + 63) / 64 * 64
 int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
                  hipEvent_t* ev /* 2*SPH_NTIMERS or null */);
 
+// a field's device array (current order)
+double* field_data(const PassBuffers& b, int field);
 int enqueue_read_field(const PassBuffers& b, int field, int sim, double* dev_out, hipStream_t st);
 int enqueue_write_field(PassBuffers& b, int field, int sim, const double* dev_in, hipStream_t st);
 // neighbour rows by ID (ids, d2 and, if dev_px is not null, the image

@@ -161,6 +161,9 @@ int fetch_sims(sph_sim* s);
 // readback staging (sph_stage.hip): copy `bytes` (a multiple of 4) of a device
 // array to the host after the stream's work so far; returns when they are there
 int copy_out(sph_sim* s, void* dst, const void* dev, size_t bytes);
+// the same of at most kOrderedMax doubles in the order of their IDs 0..n-1
+inline constexpr int kOrderedMax = 8192;
+int read_ordered(sph_sim* s, double* dst, const double* dev, const uint32_t* id, int n);
 // write the first nerr error flags and the counters' sums to the handle's
 // pinned block (enqueue_flags), and read them there once the stream is done
 int enqueue_flags(sph_sim* s, int nerr);

@@ -2418,7 +2418,7 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
 
 // ------------------------------------------------------------------------
 // readback / upload by particle ID
-__device__ inline double* field_ptr(const Positions& p, const Fields& f, int field) {
+__host__ __device__ inline double* field_ptr(const Positions& p, const Fields& f, int field) {
   switch (field) {
     case 0: return p.x;
     case 1: return p.y;
@@ -2460,6 +2460,8 @@ __global__ void k_gather_by_id(const Item* __restrict__ items, int nitems,
   const int64_t base = sim >= 0 ? 0 : sims[it.sim].off;
   field_ptr(p, f, field)[t] = in[base + f.id[t]];
 }
+
+double* field_data(const PassBuffers& b, int field) { return field_ptr(b.pos_cur, b.fcur, field); }
 
 int enqueue_read_field(const PassBuffers& b, int field, int sim, double* dev_out, hipStream_t st) {
   hipLaunchKernelGGL(k_scatter_by_id, dim3(b.nitems), dim3(kItem), 0, st, b.items, b.nitems, b.sims,

@@ -103,3 +103,25 @@ def test_neighbour_rows_of_each_width(ks):
         assert (ids[rows, k:] == 0xFFFFFFFF).all() and np.isnan(d2[rows, k:]).all()
         assert np.isnan(px[rows, k:]).all() and np.isnan(py[rows, k:]).all()
         first += n
+
+
+@pytest.mark.parametrize("n", [3, 8191, 8192, 8193])
+def test_small_fields_in_order(n):
+    """Either side of the most values ordered in LDS: alone and in a batch
+    behind another simulation, with IDs in a shuffled input order, after steps
+    that permute the particles."""
+    r = np.random.default_rng(n)
+    sts = [ics.uniform(m, seed=m) for m in (1001, n)]
+    ps = [L.default_params(k=2, mass=1.0 / len(s["x"]), hor=(0, 1), vert=(0, 1))
+          for s in sts]
+    b = L.Batch(ps, sts)
+    ids = r.permutation(n).astype(np.uint32)
+    st, p = sts[1], ps[1]
+    g = L.Sim(p, st["x"], st["y"], ids=ids)
+    g.calculate_forces()
+    b.calculate_forces()
+    assert (b.get_sim(1, "x") == st["x"]).all() and (b.get_sim(0, "y") == sts[0]["y"]).all()
+    assert (g.get("x")[ids] == st["x"]).all() and (g.get("y")[ids] == st["y"]).all()
+    v = r.standard_normal(n)
+    g.set("e", v)
+    assert (g.get("e") == v).all()
