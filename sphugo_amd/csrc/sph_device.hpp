@@ -11,6 +11,7 @@ constexpr int kMaxK = 64;         // neighbours per particle
 constexpr int kCandCap = 256;     // kNN candidates held per wave
 constexpr int kNumRed = 5;        // sum e, sum rho, E, Px, Py
 constexpr int kRedSplit = 16;     // first-stage reduction blocks per simulation
+constexpr int kDoneStride = 32;   // u32 per simulation's counter of blocks done (one line)
 // first-stage reduction blocks of a simulation with nitems work items (one
 // per 1024 items, at most kRedSplit; 1: its totals are summed in one stage)
 __host__ __device__ inline int red_parts(int nitems) {
@@ -73,7 +74,7 @@ struct SimDev {
   double red[kNumRed];  // reductions of the last pass
   double last_speed;    // |v| of the particle stored last
   // kNN walk bracket half-width of this simulation, adapted after each pass
-  // from the queries its walk could not resolve (k_reduce): misses because
+  // from the queries its walk could not resolve (set_totals): misses because
   // h moved past the bracket widen it, annulus overflows narrow it, and it
   // returns towards walk_delta0 (the configured value) when misses are rare
   double walk_delta;

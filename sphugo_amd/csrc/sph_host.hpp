@@ -64,6 +64,7 @@ struct PassBuffers {
   uint32_t* walk_miss;  // per simulation: the walk's miss counts (kMissSlots lines)
   double* red_part;     // per simulation: kRedSplit first-stage sums (kNumRed each)
   int red_parts_max;    // the largest red_parts over the simulations (1: one stage)
+  uint32_t* red_done;   // per simulation: blocks of the force that are done (kDoneStride)
   uint2* retry;           // kNN retry list (np entries)
   uint32_t* retry_count;
   int have_h;             // every particle has an h from an earlier pass, except:

@@ -269,7 +269,7 @@ int upload_job(sph_server* s, Job* j) {
   init_open_box(d, j->in.get(), j->in.get() + n, n);
   d.off = j->off;
   d.coff = j->off * kHoleCpp + 1;
-  d.pmode = kPermInit;  // regular steps from the second pass on (k_reduce)
+  d.pmode = kPermInit;  // regular steps from the second pass on (set_totals)
   d.fmode = kForceNoKick;
   const double inf = INFINITY;
   std::memcpy(&d.cfl_min_bits, &inf, sizeof inf);
@@ -522,6 +522,7 @@ extern "C" int sph_server_create(int64_t capacity, int32_t max_jobs, int32_t kma
       hipMemsetAsync(pb.stats, 0, kStatSlots * sizeof(KnnStats), c.st) != hipSuccess ||
       hipMemsetAsync(pb.walk_miss, 0, (int64_t)max_jobs * kMissSlots * kMissStride * 4, c.st) !=
           hipSuccess ||
+      hipMemsetAsync(pb.red_done, 0, (int64_t)max_jobs * kDoneStride * 4, c.st) != hipSuccess ||
       hipMemsetAsync(pb.err, 0, (1 + max_jobs) * sizeof(int), c.st) != hipSuccess ||
       hipMemsetAsync(pb.nbr, 0, nbr_entries(capacity, pb.kmax) * sizeof(uint32_t), c.st) != hipSuccess ||
       hipStreamSynchronize(c.st) != hipSuccess)

@@ -24,7 +24,7 @@
 //                   EDot over the packed records of its neighbours, fused
 //                   with kick, drift 2, periodic wrap and reflection
 //                   (sim/sph.go:327-401,122-193), partial sums and the CFL
-//                   minimum
+//                   minimum; in small launches the totals too
 //   k_reduce_part,  per-simulation FP64 totals in a fixed order, the next
 //   k_reduce        CFL half step and the next kNN walk bracket
 //
@@ -1630,7 +1630,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const unsigned nhi = __popcll(can & ballot(out.z == kMissHi));
   const unsigned nsplit = __popcll(can & ballot(out.z == kMissWide));
   if (lane0 == 0) {
-    // the simulation's bracket misses (k_reduce adapts its delta)
+    // the simulation's bracket misses (set_totals adapts its delta)
     uint32_t* ms = walk_miss + ((int64_t)it.sim * kMissSlots + (blockIdx.x & (kMissSlots - 1))) *
                                    kMissStride;
     if (nlo + nhi) atomicAdd(ms, nlo + nhi);
@@ -1907,11 +1907,108 @@ struct SectionSum {
   }
 };
 
-template <bool FP32C, bool EXACT, int PARTS>
+// ---- totals ----
+// From a simulation's sums: the totals, the next CFL half step and the next walk
+// bracket (move, wide: the walk's misses of this pass).
+__device__ inline void set_totals(SimDev* S, const double* sum, double cfl_min, uint32_t move,
+                                  uint32_t wide, bool per_sim, int mode) {
+#pragma unroll
+  for (int r = 0; r < kNumRed; ++r) S->red[r] = sum[r];
+  if (mode == kForceKick) S->dt_last = S->dt_half;
+  if (per_sim) {  // regular steps after a job's first pass
+    S->pmode = kPermPredict;
+    S->fmode = kForceKick;
+  }
+  S->walk_delta = adapt_delta(S->walk_delta, S->walk_delta0, move, wide, S->n);
+  S->dt_half = S->use_cfl ? 0.5 * (S->cfl * cfl_min) : S->dt_fixed;
+  S->cfl_min_bits = (unsigned long long)__double_as_longlong(INFINITY);
+}
+
+// In launches of up to kFinishItems work items the totals come from the force's
+// own launch: the block of a simulation that ends last adds its items' partial
+// sums up, in k_reduce's order.  Bound by latency: a launch of its own (k_reduce)
+// takes 4.7 us per pass, this adds 2.4 us to the force at 2,200 particles and 3.5
+// at 77,777 (304 items).  From about two blocks per CU on, every block's wait for its
+// stores and its counter lasts into the next block's time: 262,144 particles (1024
+// items) 38.2 -> 45.6 us against 6.4 for the launch, 1M 215 -> 225.6 against 10.5.
+inline constexpr int kFinishItems = 512;
+
+// Values that blocks of one launch hand to each other: stored and loaded past
+// the caches that their XCDs do not share.
+__device__ inline void put_shared(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline double get_shared(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Called by one wave of each of `of` blocks after its put_shared's: true for the
+// last of them, which may then get_shared what the others put.  The counter is
+// zero again for the next launch.
+__device__ inline bool last_of(uint32_t* counter, uint32_t of, int lane) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what was put has arrived
+  uint32_t v = 0;
+  if (lane == 0) {
+    v = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    if (v == of) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  v = readlane_u(v, 0);
+  asm volatile("" ::: "memory");
+  return v == of;
+}
+
+// By one wave of each of the simulation's blocks, `parts` of them per item; i0 is
+// its first item, ni their number (at most kFinishItems).
+__device__ inline void finish_totals(SimDev* S, int sim, int i0, int ni, int parts,
+                                     const double* __restrict__ partials,
+                                     uint32_t* __restrict__ done,
+                                     uint32_t* __restrict__ walk_miss, bool per_sim, int mode,
+                                     int lane) {
+  if (!last_of(done + (int64_t)sim * kDoneStride, (uint32_t)(ni * parts), lane)) return;
+  // the walk's miss counts of this pass (copy q by lane q), read and cleared for
+  // the next pass
+  int move = 0, wide = 0;
+  if (lane < kMissSlots) {
+    uint32_t* wm = walk_miss + ((int64_t)sim * kMissSlots + lane) * kMissStride;
+    move = (int)wm[0];
+    wide = (int)wm[1];
+    wm[0] = 0u;
+    wm[1] = 0u;
+  }
+  const double cfl_min = __longlong_as_double((long long)__hip_atomic_load(
+      &S->cfl_min_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  // lane l stands for k_reduce's threads l, l + 64, l + 128 and l + 192
+  double v[4][kNumRed];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+#pragma unroll
+    for (int r = 0; r < kNumRed; ++r) v[q][r] = 0.0;
+    for (int i = q * 64 + lane; i < ni; i += 256) {
+      const double* p = partials + (int64_t)(i0 + i) * parts * kNumRed;
+#pragma unroll
+      for (int r = 0; r < kNumRed; ++r)
+        v[q][r] += parts == 1 ? get_shared(p + r)
+                              : (get_shared(p + r) + get_shared(p + kNumRed + r)) +
+                                    (get_shared(p + 2 * kNumRed + r) + get_shared(p + 3 * kNumRed + r));
+    }
+  }
+  double sum[kNumRed];
+#pragma unroll
+  for (int r = 0; r < kNumRed; ++r)
+    sum[r] = group_sum((v[0][r] + v[2][r]) + (v[1][r] + v[3][r]), 64);
+  for (int o = kMissSlots / 2; o > 0; o >>= 1) {
+    move += __shfl_xor(move, o, 64);
+    wide += __shfl_xor(wide, o, 64);
+  }
+  if (lane == 0) set_totals(S, sum, cfl_min, (uint32_t)move, (uint32_t)wide, per_sim, mode);
+}
+
+// FINISH: the totals too (finish_totals).
+template <bool FP32C, bool EXACT, int PARTS, bool FINISH>
 __global__ __launch_bounds__(256) void k_force(
     const Item* __restrict__ items, int nitems, SimDev* __restrict__ sims,
     const void* __restrict__ recp, Fields f, const uint32_t* __restrict__ nbr, int kstride,
-    int mode, Positions pout, double* __restrict__ partials, const double2* __restrict__ XY) {
+    int mode, Positions pout, double* __restrict__ partials, const double2* __restrict__ XY,
+    uint32_t* __restrict__ red_done, uint32_t* __restrict__ walk_miss) {
   static_assert(PARTS == 1 || (PARTS == kSections && !EXACT));
   constexpr int kParticles = kItem / PARTS;  // of a block
   __shared__ double red[4][kNumRed + 1];
@@ -1929,7 +2026,8 @@ __global__ __launch_bounds__(256) void k_force(
   const double lx = S->lx, ly = S->ly;
   const int kern = S->kernel;
   const double dt = S->dt_half;
-  if (mode < 0) mode = S->fmode;
+  const bool per_sim = mode < 0;
+  if (per_sim) mode = S->fmode;
   // The block's window of neighbour records in LDS, which holds most of the
   // neighbours of Hilbert-ordered particles; the rest are gathered from memory.
   // As wide as its registers' waves leave room for in LDS: 640 slots from first -
@@ -2194,6 +2292,8 @@ __global__ __launch_bounds__(256) void k_force(
     r_E = mass * (e + 0.5 * sp2);
     r_px = mass * vx;
     r_py = mass * vy;
+    // the TotalMomentum quirk value
+    if (FINISH && t == S->off + S->n - 1) S->last_speed = sqrt(sp2);
   }
   // block reductions in a fixed order
   r_e = group_sum(r_e, 64);
@@ -2205,36 +2305,41 @@ __global__ __launch_bounds__(256) void k_force(
     const double other = __shfl_xor(r_cfl, o, 64);
     r_cfl = other < r_cfl ? other : r_cfl;
   }
-  if constexpr (PARTS > 1) {
+  auto put = [](double* p, double v) {
+    if constexpr (FINISH) put_shared(p, v);
+    else *p = v;
+  };
+  if constexpr (PARTS == 1) {
     if (lane == 0) {
-      double* p = partials + (int64_t)blk * kNumRed;
-      p[0] = r_e;
-      p[1] = r_rho;
-      p[2] = r_E;
-      p[3] = r_px;
-      p[4] = r_py;
-      if (r_cfl < INFINITY)
-        atomicMin(&S->cfl_min_bits, (unsigned long long)__double_as_longlong(r_cfl));
+      red[wv][0] = r_e;
+      red[wv][1] = r_rho;
+      red[wv][2] = r_E;
+      red[wv][3] = r_px;
+      red[wv][4] = r_py;
+      red[wv][5] = r_cfl;
     }
-    return;
+    __syncthreads();
+    if (wv) return;
+    if (lane < kNumRed)
+      put(partials + (int64_t)item_idx * kNumRed + lane,
+          (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]));
+#pragma unroll
+    for (int w = 0; w < 4; ++w) r_cfl = red[w][5] < r_cfl ? red[w][5] : r_cfl;
+  } else if (lane == 0) {
+    double* p = partials + (int64_t)blk * kNumRed;
+    put(p, r_e);
+    put(p + 1, r_rho);
+    put(p + 2, r_E);
+    put(p + 3, r_px);
+    put(p + 4, r_py);
   }
-  if (lane == 0) {
-    red[wv][0] = r_e;
-    red[wv][1] = r_rho;
-    red[wv][2] = r_E;
-    red[wv][3] = r_px;
-    red[wv][4] = r_py;
-    red[wv][5] = r_cfl;
-  }
-  __syncthreads();
-  if (threadIdx.x < kNumRed) {
-    const int r = threadIdx.x;
-    partials[(int64_t)item_idx * kNumRed + r] = (red[0][r] + red[1][r]) + (red[2][r] + red[3][r]);
-  }
-  if (threadIdx.x == 0) {
-    double m = red[0][5];
-    for (int w = 1; w < 4; ++w) m = red[w][5] < m ? red[w][5] : m;
-    if (m < INFINITY) atomicMin(&S->cfl_min_bits, (unsigned long long)__double_as_longlong(m));
+  if (lane == 0 && r_cfl < INFINITY)
+    atomicMin(&S->cfl_min_bits, (unsigned long long)__double_as_longlong(r_cfl));
+  if constexpr (FINISH) {
+    const int li = (int)((it.first - S->off) / kItem);
+    const int ni = (int)((S->n + kItem - 1) / kItem);
+    finish_totals(S, it.sim, item_idx - li, ni, PARTS, partials, red_done, walk_miss, per_sim, mode,
+                  lane);
   }
 }
 
@@ -2293,7 +2398,7 @@ __global__ __launch_bounds__(256) void k_reduce_part(const SimDev* __restrict__ 
 }
 
 // One block per simulation: the totals from the first stage's sums, the
-// next CFL half step, the TotalMomentum quirk value and the next bracket.
+// TotalMomentum quirk value and what follows from them.
 __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
                                                 const double* __restrict__ partials,
                                                 int parts_per_item,
@@ -2338,23 +2443,16 @@ __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
   }
   block_sum(sh, acc);
   if (tid == 0) {
+    double sum[kNumRed];
 #pragma unroll
-    for (int r = 0; r < kNumRed; ++r) S->red[r] = sh[r][0];
+    for (int r = 0; r < kNumRed; ++r) sum[r] = sh[r][0];
     S->last_speed = sqrt(vx_last * vx_last + vy_last * vy_last);
-    if (mode == kForceKick) S->dt_last = S->dt_half;
-    if (per_sim) {  // regular steps after a job's first pass
-      S->pmode = kPermPredict;
-      S->fmode = kForceKick;
-    }
     uint32_t move = 0u, wide = 0u;
     for (int q = 0; q < kMissSlots; ++q) {
       move += miss[0][q];
       wide += miss[1][q];
     }
-    S->walk_delta = adapt_delta(S->walk_delta, S->walk_delta0, move, wide, S->n);
-    const double m = __longlong_as_double((long long)S->cfl_min_bits);
-    S->dt_half = S->use_cfl ? 0.5 * (S->cfl * m) : S->dt_fixed;
-    S->cfl_min_bits = (unsigned long long)__double_as_longlong(INFINITY);
+    set_totals(S, sum, __longlong_as_double((long long)S->cfl_min_bits), move, wide, per_sim, mode);
   }
 }
 
@@ -2441,23 +2539,32 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
   mark(3, 1);
   mark(4, 0);
   const int parts = b.bitwise || b.nitems > force_split_items(b.kmax) ? 1 : kSections;
-#define SPH_FORCE(F32, EX, P)                                                                  \
-  hipLaunchKernelGGL((k_force<F32, EX, P>), dim3(b.nitems * P), dim3(256), 0, st, b.items,      \
+  const bool finish = b.nitems <= kFinishItems;
+#define SPH_FORCE_(F32, EX, P, FIN)                                                            \
+  hipLaunchKernelGGL((k_force<F32, EX, P, FIN>), dim3(b.nitems * P), dim3(256), 0, st, b.items, \
                      b.nitems, b.sims, (const void*)b.rec, b.fnew, b.nbr, b.kmax, force_mode,  \
-                     b.pos_cur, b.partials, b.xyp)
-  if (b.bitwise) SPH_FORCE(false, true, 1);
-  else if (b.prec == kPrecFP32C && parts > 1) SPH_FORCE(true, false, kSections);
-  else if (b.prec == kPrecFP32C) SPH_FORCE(true, false, 1);
-  else if (parts > 1) SPH_FORCE(false, false, kSections);
-  else SPH_FORCE(false, false, 1);
+                     b.pos_cur, b.partials, b.xyp, b.red_done, b.walk_miss)
+#define SPH_FORCE(F32, EX)                                                                     \
+  {                                                                                            \
+    if (finish) SPH_FORCE_(F32, EX, 1, true); else SPH_FORCE_(F32, EX, 1, false);              \
+  }
+  static_assert(64 + 2 * kMaxK <= kFinishItems, "launches that split rows finish in the force");
+  if (b.bitwise) SPH_FORCE(false, true)
+  else if (b.prec == kPrecFP32C && parts > 1) SPH_FORCE_(true, false, kSections, true);
+  else if (b.prec == kPrecFP32C) SPH_FORCE(true, false)
+  else if (parts > 1) SPH_FORCE_(false, false, kSections, true);
+  else SPH_FORCE(false, false)
+#undef SPH_FORCE_
 #undef SPH_FORCE
   mark(4, 1);
   mark(5, 0);
-  if (b.red_parts_max > 1)
-    hipLaunchKernelGGL(k_reduce_part, dim3(b.nsims * b.red_parts_max), dim3(256), 0, st, b.sims,
-                       b.partials, parts, b.red_first, b.red_count, b.red_part, b.red_parts_max);
-  hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, parts, b.red_part,
-                     b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss);
+  if (!finish) {
+    if (b.red_parts_max > 1)
+      hipLaunchKernelGGL(k_reduce_part, dim3(b.nsims * b.red_parts_max), dim3(256), 0, st, b.sims,
+                         b.partials, parts, b.red_first, b.red_count, b.red_part, b.red_parts_max);
+    hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, parts,
+                       b.red_part, b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss);
+  }
   mark(5, 1);
   return (int)hipGetLastError();
 }
