@@ -263,11 +263,11 @@ int sph_set_tuning(sph_sim* s, const double in[5]);
 
 /* ---- serve loop: continuous batching (no reference counterpart) ----
  * A native worker thread steps every admitted job in one shared device
- * pool: each tick is one force pass over all resident jobs, which may be at
- * different steps of their lives; a job that ends frees its particle range
- * for the next one in the queue (FIFO, first fit).  A job's results equal
- * those of sph_create + sph_step(nsteps) with the same inputs.  All calls
- * are thread-safe. */
+ * pool: each tick is a force pass (up to four while no job arrives or ends)
+ * over all resident jobs, which may be at different steps of their lives; a
+ * job that ends frees its particle range for the next one in the queue (FIFO,
+ * first fit).  A job's results equal those of sph_create + sph_step(nsteps)
+ * with the same inputs.  All calls are thread-safe. */
 typedef struct sph_server sph_server;
 
 #define SPH_JOB_QUEUED 0
@@ -304,9 +304,9 @@ int sph_server_job_reductions(sph_server* s, int64_t job_id, double out[7]);
 int sph_server_release(sph_server* s, int64_t job_id);
 /* jobs done, jobs failed, particle-steps done, seconds from the first submit
  * to the last completion, particle-steps/s over that span, p50 and p99
- * submit-to-done latency (ms), mean pool occupancy, ticks, jobs queued or
- * running now, mean tick duration (ms: uploads, one pass, readbacks) and
- * its device part (ms between events at the tick's start and end), then the
+ * submit-to-done latency (ms), mean pool occupancy, passes, jobs queued or
+ * running now, mean time per pass (ms, with uploads and readbacks) and its
+ * device part (ms between events at a tick's start and end), then the
  * two parts of the latency: p50 and p99 of the queue wait (submit to
  * admission, ms) and of the run time (admission to done, ms). */
 #define SPH_SERVER_NSTATS 16

@@ -3,7 +3,7 @@
 //
 // The pool holds `capacity` particle slots.  A job occupies a contiguous
 // range [off, off + n) and a simulation slot (its SimDev); unused ranges are
-// holes.  Every tick runs ONE force pass over the whole pool: the radix sort
+// holes.  Every force pass runs over the whole pool: the radix sort
 // keys a job's particles by coff + Hilbert(cell) with coff = off * 8 + 1 and a
 // hole slot t by t * 8, so the sort keeps every job inside its own range and
 // every hole in place, and each job's cells never collide with another's.
@@ -12,7 +12,8 @@
 // different points of their lives share every launch.  A job admitted with
 // nsteps runs nsteps + 1 passes (the reference's Step 0 computes forces
 // twice, sim/sph.go:70-76) and is read back by ID when its last pass ends;
-// its range and slot are reused from the next tick on.
+// its range and slot are reused from the next tick on.  A tick is one pass, or up to
+// kBurst while no job arrives or ends.
 //
 // Admission is FIFO: the head of the queue waits until a slot and a
 // first-fit range of n slots are free.  One native worker thread owns the
@@ -312,7 +313,15 @@ void fail_all_running(sph_server* s, const std::string& msg) {
     if (s->slots[q]) fail_job(s, s->slots[q], msg);
 }
 
-// One tick: admission, one pass over the pool, completions.
+// Passes of a tick that admits no job: up to this many, as far as no job ends
+// before the last of them.  What waits in the queue then waits for a job's end
+// anyway, and a job that arrives meanwhile waits for kBurst - 1 passes more.  A
+// pass per tick paid the flags' launch, the wait for it and the next launch's start
+// each time, 25 us: one tube job of 20 steps 2,387 -> 1,931 us, 12 jobs together
+// 17.4 -> 16.1 ms.
+constexpr int kBurst = 4;
+
+// One tick: admission, passes over the pool, completions.
 // Returns false when the worker should stop.
 bool tick(sph_server* s) {
   sph_sim& c = s->core;
@@ -352,12 +361,15 @@ bool tick(sph_server* s) {
   s->items_dirty = false;
   std::vector<Job*> finishing;
   int64_t occupied = 0;
+  int passes = admitted.empty() ? kBurst : 1;
+  for (Job* j : s->slots)
+    if (j) passes = std::min(passes, j->nsteps + 1 - j->passes);
   for (Job* j : s->slots) {
     if (!j || rc) continue;
     occupied += j->n;
-    if (j->passes + 1 == j->nsteps + 1) finishing.push_back(j);
+    if (j->passes + passes == j->nsteps + 1) finishing.push_back(j);
   }
-  if (!rc) {
+  for (int p = 0; p < passes && !rc; ++p) {
     c.bind();
     c.pb.some_new = !admitted.empty();
     rc = enqueue_pass(c.pb, kPerSim, kPerSim, c.st, nullptr);
@@ -389,8 +401,8 @@ bool tick(sph_server* s) {
     s->cv_done.notify_all();
     return false;
   }
-  s->ticks += 1;
-  s->occupancy_sum += (double)occupied / (double)s->cap;
+  s->ticks += passes;
+  s->occupancy_sum += passes * ((double)occupied / (double)s->cap);
   s->tick_ms_sum += ms_between(t_tick, Clock::now());
   float gms = 0.f;
   if (s->ev_tick[0] && hipEventElapsedTime(&gms, s->ev_tick[0], s->ev_tick[1]) == hipSuccess)
@@ -423,7 +435,7 @@ bool tick(sph_server* s) {
     Job* j = s->slots[q];
     if (!j) continue;
     if (j->state == SPH_JOB_RUNNING) {
-      j->passes += 1;
+      j->passes += passes;
       if (j->passes < j->nsteps + 1) continue;
       j->state = SPH_JOB_DONE;
       j->t_done = now;
