@@ -897,6 +897,12 @@ struct WalkShared {
 constexpr double kThinSum = 2e-3;  // FP32C kernel sums below it are redone in FP64
 constexpr double kMissWide = -1.0, kMissLo = -2.0, kMissAnn = -3.0, kMissHi = -4.0;
 constexpr double kSeeded = -5.0;
+// The exact search starts from 1.1 times a query's last h.  One that the walk found
+// too few neighbours for, within up to 1.1 h already, starts from the radius
+// that would hold 1.2 k at the density inside that (its h is set so that 1.1 h
+// is that radius): its first attempt had to fail, 4,700 particles of a tube took
+// 15.1 us in the exact search against 11.8, 77,777 11.5 against 10.6.
+constexpr double kFirstReach = 1.1, kMissReach = 1.2;
 static_assert(sizeof(WalkShared) == 10240, "sixteen waves per CU");
 
 typedef __attribute__((address_space(3))) uint8_t LdsByte;
@@ -1040,6 +1046,69 @@ __device__ inline void classify(WalkShared& sh, const double4* gq, int ncand, ui
         at += (uint32_t)__popcll(ma[r]);
       }
     }
+    c_lo = ql == i ? nc : c_lo;
+    c_an = ql == i ? na : c_an;
+  }
+}
+
+// The lists of the queries of `todo`, whose annulus holds more than kAnn, by
+// narrower brackets: the bracket of the squared distance is halved until it does
+// not.  (Equal distances are never parted: the exact search takes more than kAnn of
+// them.)  Few queries, but at k = 64 nine of ten of those that the exact search
+// took, 4M clustered 22,900 per pass -> 3,400: that search 104 -> 43 us, and 34 ->
+// 20 at 1M, while the walk's time stays (halving in classify's own loop, whose
+// registers are full, made it 5 % slower).  Queries with k certain neighbours are
+// left to the exact search: they are few in every size, and where launches are
+// short the wave that stays for one costs more than the search (2,200 particles 46.2
+// -> 46.9 us per step).
+template <bool IMG>
+__device__ inline void tighten(WalkShared& sh, const double4* gq, int ncand, uint32_t todo,
+                               uint32_t t0, int k, double lx, double ly, int lane, int& c_lo,
+                               int& c_an) {
+  constexpr int NR = (kWalkCand + 63) / 64;
+  for (uint32_t rem = todo; rem; rem &= rem - 1u) {
+    const int i = __builtin_ctz(rem);
+    const double4 q = gq[i];
+    const uint32_t ti = t0 + (uint32_t)i;
+    double d2[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int s = r * 64 + lane;
+      const bool in = s < ncand && (sh.pk[s] >> 4) != ti;
+      d2[r] = in ? slot_d2<IMG>(sh, (uint32_t)s, q.x, q.y, lx, ly) : INFINITY;
+    }
+    auto below = [&](double v) {
+      int n = 0;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) n += __popcll(ballot(d2[r] < v));
+      return n;
+    };
+    // nlo of them lie below lo, fewer than k; nhi below hi, k or more
+    double lo = q.z, hi = q.w;
+    int nlo = below(lo), nhi = k + kAnn;
+    for (int it = 0; it < 24 && nhi - nlo > kAnn; ++it) {
+      const double mid = 0.5 * (lo + hi);
+      const int n = below(mid);
+      if (n >= k) {
+        hi = mid;
+        nhi = n;
+      } else {
+        lo = mid;
+        nlo = n;
+      }
+    }
+    int nc = 0, na = 0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const unsigned long long mc = ballot(d2[r] < lo), ma = ballot(d2[r] < hi) & ~mc;
+      // (past kAnn the counts say so and the lists are not read)
+      if (d2[r] < lo) sh.row[i][nc + lane_prefix(mc)] = (uint8_t)(r * 64 + lane);
+      else if (d2[r] < hi && na + lane_prefix(ma) < kAnn)
+        sh.annl[i][na + lane_prefix(ma)] = (uint8_t)(r * 64 + lane);
+      nc += __popcll(mc);
+      na += __popcll(ma);
+    }
+    const int ql = lane & (kGrp - 1);
     c_lo = ql == i ? nc : c_lo;
     c_an = ql == i ? na : c_an;
   }
@@ -1401,7 +1470,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     qy1 = -(float)(fy + ry);
     sh.q[lane0] = make_double4(pq.x, pq.y, Rlo * Rlo, SEED ? Rhi : Rhi * Rhi);
   }
-  unsigned nties = 0;
+  unsigned nties = 0, ntight = 0;
   const uint32_t table = kHilbertTable.w[lane0];
   const uint32_t* cells = cstart + S->coff;
 
@@ -1549,7 +1618,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         continue;
       }
       int c_lo = 0, c_an = 0;
-      const double xq = gq[ql].x, yq = gq[ql].y;
       const int nr = (ncand + 63) >> 6;
 #define SPH_CLASSIFY(NR)                                                                        \
   {                                                                                             \
@@ -1561,7 +1629,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
       else if (nr == 2) SPH_CLASSIFY(2)
       else SPH_CLASSIFY(1)
 #undef SPH_CLASSIFY
+      const uint32_t dense =
+          (uint32_t)ballot(grp && c_lo < k && c_an > kAnn && c_lo + c_an >= k) & 0xFFFFu;
+      if (dense) {
+        ntight += (unsigned)__builtin_popcount(dense);
+        wave_fence();
+        if (images) tighten<true>(sh, gq, ncand, dense, t0, k, lx, ly, lane, c_lo, c_an);
+        else tighten<false>(sh, gq, ncand, dense, t0, k, lx, ly, lane, c_lo, c_an);
+      }
       wave_fence();
+      const double xq = gq[ql].x, yq = gq[ql].y;
       const bool ok = grp && c_lo < k && c_an <= kAnn && c_lo + c_an >= k;
       auto finish = [&](auto img) {
         constexpr bool IMG = decltype(img)::value;
@@ -1597,8 +1674,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         }
       };
       if (images) finish(std::true_type{}); else finish(std::false_type{});
-      if (grp && !ok && part == 0)
+      if (grp && !ok && part == 0) {
         gq[ql].z = c_lo >= k ? kMissLo : (c_an > kAnn ? kMissAnn : kMissHi);
+        // a radius for the exact search from the neighbours inside Rhi
+        const double more = kMissReach * k / (c_lo + c_an > 0 ? c_lo + c_an : 1);
+        gq[ql].w = __builtin_amdgcn_sqrt(gq[ql].w * (more < 4.0 ? more : 4.0));
+      }
       pending &= ~gmask;
       gsz = kGrp;
     }
@@ -1621,7 +1702,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     uint32_t base = 0;
     if (lane0 == 0) base = atomicAdd(retry_count, (uint32_t)__popcll(m));
     base = readlane_u(base, 0);
-    if (left) retry[base + lane_prefix(m)] = make_uint2(t, (uint32_t)item_idx);
+    if (left) {
+      retry[base + lane_prefix(m)] = make_uint2(t, (uint32_t)item_idx);
+      if (tried && out.z == kMissHi) H[t] = out.w * (1.0 / kFirstReach);
+    }
   }
   // counters: queries with an h that needed the exact search, and why
   const unsigned nfall = __popcll(m & can);
@@ -1634,7 +1718,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     uint32_t* ms = walk_miss + ((int64_t)it.sim * kMissSlots + (blockIdx.x & (kMissSlots - 1))) *
                                    kMissStride;
     if (nlo + nhi) atomicAdd(ms, nlo + nhi);
-    if (nann) atomicAdd(ms + 1, nann);
+    if (nann + ntight) atomicAdd(ms + 1, nann + ntight);
     KnnStats* sp = stat_slot(stats);
     stat_add(&sp->retries, nfall);
     stat_add(&sp->ties, nties);
@@ -1850,7 +1934,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const double2 pq = XY[t];
     const double xq = pq.x, yq = pq.y, hp = H[t];
     const PredVal pred = {EP[t], VPX[t], VPY[t]};
-    const double R0 = hp > 0 ? hp * 1.1 : local_radius(S, cstart, xq, yq);
+    const double R0 = hp > 0 ? hp * kFirstReach : local_radius(S, cstart, xq, yq);
     const unsigned long long nfail0 = nfail;
     const SearchOut so = wave_search<BITWISE>(S, t, xq, yq, R0, XY, WR, cstart, ID, table,
                                               nbr_row(nbr, t, kstride), sh, nretry, nties, nfail);

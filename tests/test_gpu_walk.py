@@ -11,6 +11,7 @@ distances and h bit-exact; density and sound speed 1e-12 (plain FP64) and 1e-5
 import numpy as np
 import pytest
 
+import oracle as O
 from sphugo_amd import _lib as L
 from sphugo_amd import ics
 
@@ -91,3 +92,41 @@ def test_bitwise_walk_is_exact(name, k):
         for f in ("rho", "c", "h", "ax", "ay", "edot"):
             assert (g.get(f) == o.get(f)).all(), f
         g.calculate_forces()
+
+
+# open boxes whose particles move together or apart between two passes: the last
+# h's bracket then holds k neighbours too many (squeezed beyond 1 + delta), too few
+# (stretched), either from place to place, or more than its annulus takes (delta
+# 0.1 at k = 64)
+@pytest.mark.parametrize("move,delta", [(1 / 1.2, 0.025), (1 / 1.5, 0.1), (1.0, 0.1), (1.25, 0.025),
+                                        ("mixed", 0.05)])
+@pytest.mark.parametrize("layout,n,k", [("uniform", 257, 64), ("uniform", 4099, 33),
+                                        ("lattice", 576, 40), ("clumps", 4111, 64)])
+@pytest.mark.parametrize("prec", [L.PREC_FP64, L.PREC_FP32C])
+def test_bracket_beside_the_kth_distance(move, delta, layout, n, k, prec):
+    st = {"uniform": lambda: ics.uniform(n, seed=n + k), "lattice": lambda: _lattice(24),
+          "clumps": lambda: _clumps(n, n + k)}[layout]()
+    phys = dict(k=k, mass=st["mass"], gamma=5 / 3, visc_alpha=1.0, visc_beta=2.0, dt_half=0.001,
+                hor=(-L.DBL_MAX, L.DBL_MAX), vert=(-L.DBL_MAX, L.DBL_MAX))
+    init = [st[f] for f in ("x", "y", "vx", "vy", "e")]
+    g = L.Sim(L.default_params(precision=prec, **phys), *init)
+    o = O.OracleSim(O.default_params(knn_mode=O.KNN_EXACT, **phys), *init)
+    for s in (g, o):
+        for f, v in (("vpx", st["vx"]), ("vpy", st["vy"]), ("epred", st["e"])):
+            s.set(f, v)
+    g.calculate_forces()
+    L.set_tuning(g, delta=delta)
+    for f in ("x", "y"):
+        v = st[f] * move if move != "mixed" else st[f] + 0.05 * np.sin(9 * st[f])
+        g.set(f, v)
+        o.set(f, v)
+    c0 = g.knn_counters()
+    g.calculate_forces()
+    c1 = g.knn_counters()
+    o.calculate_forces()
+    _check_knn(g, o)
+    bar = 1e-12 if prec == L.PREC_FP64 else 1e-5
+    assert _rel(g.get("rho"), o.get("rho")).max() <= bar
+    # an annulus too full needs no exact search
+    if layout == "uniform" and move == 1:
+        assert c1["retries"] - c0["retries"] <= n // 20, (c0, c1)
