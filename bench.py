@@ -45,12 +45,11 @@ def algo_bytes(kernel: str, k: int, precision: str = "fp32c") -> int:
     read or written once (state 8 B, IDs and keys 4 B), materialised
     neighbour lists 4 B per entry; neighbour gathers count as on-chip reuse."""
     rec = 32 if precision == "fp32c" else 64            # force record (RecF / RecD)
-    uxy = 8 if precision == "fp32c" else 0              # fixed-point positions
     return {
         "keys": 32 + 4,                                   # x, y, vx, vy -> key
-        "permute": 4 + 4 + 9 * 8 + 4 + 10 * 8 + 4 + 1 + uxy,  # perm, key, gather, write
+        "permute": 4 + 4 + 9 * 8 + 4 + 10 * 8 + 4 + 1,    # perm, key, gather, write
         "knn_walk": 16 + 8 + 4 * k + 4,                   # xy, h_prev -> list, count
-        "knn_finish": 4 + 16 + 3 * 8 + 4 * k + 3 * 8 + rec,  # count, xy, pred -> list in; h, rho, c, record
+        "knn_finish": 3 * 8 + 3 * 8 + rec,                # in the walk's launch: pred -> h, rho, c, record
         "force": 4 * k + 80 + 64,                         # list, own state -> a, edot, v, e, x, y
     }[kernel]
 
@@ -489,14 +488,17 @@ def main():
     # dominant single kernel and its roofline
     km = head["kernel_ms"]
     prec_name = "fp32c" if "fp32c" in res else "fp64"
-    cands = ("knn_walk", "knn_finish", "force", "permute", "keys")
+    cands = ("knn_walk", "force", "permute", "keys")
     dom = max(cands, key=lambda n: km[n])
-    bytes_launch = algo_bytes(dom, k, prec_name) * st["n"]
+    # the walk's launch also sums the density and writes the force records
+    per = sum(algo_bytes(n, k, prec_name)
+              for n in ((dom, "knn_finish") if dom == "knn_walk" else (dom,)))
+    bytes_launch = per * st["n"]
     ach = bytes_launch / (km[dom] * 1e-3) / 1e9
     traffic = profiled_traffic(prec_name, dom) if args.workload == "clustered" else None
     roof = {"bound": "hbm", "kernel": dom, "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": traffic,
-            "algo_bytes_per_particle": algo_bytes(dom, k, prec_name), "avg_ms": km[dom]}
+            "algo_bytes_per_particle": per, "avg_ms": km[dom]}
     df = ("knn_walk", "knn_finish", "force")
     t_df = km["knn_density"] + km["force"]
     b_df = sum(algo_bytes(n, k, prec_name) for n in df) * st["n"]
