@@ -77,7 +77,7 @@ extern "C" {
 #define SPH_T_PERMUTE 2
 #define SPH_T_KNN_DENSITY 3
 #define SPH_T_FORCE 4
-#define SPH_T_REDUCE 5
+#define SPH_T_REDUCE 5 /* nothing in small launches, whose force adds the totals up */
 /* the three launches inside SPH_T_KNN_DENSITY */
 #define SPH_T_KNN_WALK 6     /* bracketed walk, density, force records */
 #define SPH_T_KNN_FINISH 7   /* nothing (part of the walk) */

@@ -18,8 +18,7 @@
 //                   misses go to a retry list
 //                   (sim/nearest-neighbour.go:28-165, sim/sph.go:306-323,
 //                   421-429)
-//   k_knn_fallback  exact wavefront-per-query search for the retry list (or
-//                   for every query of the first pass)
+//   k_knn_fallback  exact wavefront-per-query search for the retry list
 //   k_force         thread per particle: pressure + artificial viscosity +
 //                   EDot over the packed records of its neighbours, fused
 //                   with kick, drift 2, periodic wrap and reflection
@@ -1392,8 +1391,8 @@ __device__ inline void seed_radii(WalkShared& sh, double4* gq, int ncand, uint32
 // side, where halving down to single queries kept one wave busy (30,000
 // clustered: 196 against 136 us per step).
 //
-// What bounds it: vector issue, 77 % of all issue slots at 4M clustered, k = 64
-// (about 130 vector instructions per query; 1.28 GB written, 0.29 GB read).
+// What bounds it: vector issue, 75 % of all issue slots at 4M clustered, k = 64
+// (124 vector instructions per query; 1.31 GB written, 0.29 GB read).
 // One query's candidates side by side in the lanes need no per-query lists and
 // no lane waits for the longest of 64 lists, and a group of 16 queries is a
 // short chain of loads, so small launches finish early.  Against the walk with
