@@ -412,9 +412,13 @@ __device__ inline double rsq64(double x) {
 // sqrt(x) / h for hinv near 1 / h: one Newton step on the reciprocal square
 // root, then a residual step on the root and one on the quotient, which leave
 // both rounded as the exact operations round them (but for rare last-place
-// cases).  1 - q keeps its digits that way where q is near 1.
+// cases).  1 - q keeps its digits that way where q is near 1.  The estimate is held
+// to that of the smallest double (2^537, by its high word): at x = 0 (a neighbour at
+// the same point) it stays finite, and the products with x give 0.
 __device__ inline double sqrt_over(double x, double h, double hinv) {
   double y = __builtin_amdgcn_rsq(x);
+  const uint32_t top = (uint32_t)__double2hiint(y);
+  y = __hiloint2double((int)(top < 0x61800000u ? top : 0x61800000u), __double2loint(y));
   const double t = 0.5 * x * y;
   y = fma(y, fma(-t, y, 0.5), y);
   const double s0 = x * y;
