@@ -33,11 +33,10 @@ using sph::Positions;
 using sph::SimDev;
 
 namespace sph {
-// Pinned blocks of a handle's readbacks (sph_stage.hip), taken when first used.
+// What a handle keeps for its readbacks (sph_stage.hip).
 struct Stage {
-  char* small = nullptr;   // one small copy
-  char* ring = nullptr;    // slots of a large copy
-  hipEvent_t ev[8] = {};   // per slot: filled
+  char* flags = nullptr;   // pinned block from enqueue_flags to take_flags
+  hipEvent_t ev[8] = {};   // per slot of a large copy: filled
 };
 void stage_open(Stage& s);
 void stage_close(Stage& s);
@@ -164,8 +163,8 @@ int copy_out(sph_sim* s, void* dst, const void* dev, size_t bytes);
 // the same of at most kOrderedMax doubles in the order of their IDs 0..n-1
 inline constexpr int kOrderedMax = 8192;
 int read_ordered(sph_sim* s, double* dst, const double* dev, const uint32_t* id, int n);
-// write the first nerr error flags and the counters' sums to the handle's
-// pinned block (enqueue_flags), and read them there once the stream is done
+// write the first nerr error flags and the counters' sums to a pinned block
+// (enqueue_flags), and read them there once the stream is done
 int enqueue_flags(sph_sim* s, int nerr);
 void take_flags(sph_sim* s, sph::KnnStats* stats, int* err, int nerr);
 int check_device_flags(sph_sim* s);

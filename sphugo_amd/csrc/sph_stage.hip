@@ -18,50 +18,67 @@
 
 namespace sph {
 
-constexpr size_t kSmallBlock = 512 << 10;  // one small copy, or the flags of a full server
 constexpr size_t kSmallCopy = 256 << 10;   // larger copies take the slots
 constexpr size_t kSlot = 1 << 20;          // one slot of a large copy
-constexpr int kSlots = 8;
+constexpr int kSlots = 8;                  // slots of a ring
+static_assert(sizeof(Stage::ev) / sizeof(hipEvent_t) == kSlots, "an event per slot");
 
 namespace {
 
-// Pinned blocks of one size, shared by the handles of a process: a handle
-// takes one when it first needs it and returns it when it is destroyed.  At
-// most `keep` free blocks are held, and none once no handle is left.
+// Pinned memory of one size, shared by the handles of a process: a call takes what
+// it needs and returns it when it ends, so a program with many handles holds as
+// many pieces as its calls at one time use and at most kKeep free ones of a size,
+// and none once no handle is left.  A block serves the small copies, the flags and
+// copies of one slot; a ring, which takes 400 to 650 us to allocate against a
+// block's 50 (the first read of 800 KB in a process 534 -> 347 us), those of more,
+// which run 2 % faster in one piece than in separate blocks (45 MB of neighbour rows
+// 2,470 against 2,530 us).
+constexpr size_t kKeep = 16;
 struct PinnedPool {
   size_t bytes;
-  size_t keep;
-  std::vector<void*> idle;
+  size_t keep;  // at most kKeep
+  void* idle[kKeep];
+  size_t n;
 };
 std::mutex g_mu;
-PinnedPool g_small = {kSmallBlock, 16, {}}, g_ring = {kSlot * kSlots, 4, {}};
+PinnedPool g_blocks = {kSlot, 16, {}, 0}, g_rings = {kSlot * kSlots, 4, {}, 0};
 int g_handles = 0;
 
-void* take(PinnedPool& p) {
+char* take(PinnedPool& p) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (!p.idle.empty()) {
-      void* b = p.idle.back();
-      p.idle.pop_back();
-      return b;
-    }
+    if (p.n) return (char*)p.idle[--p.n];
   }
   void* b = nullptr;
   if (hipHostMalloc(&b, p.bytes, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess)
     return nullptr;
-  return b;
+  return (char*)b;
 }
 
-void give(PinnedPool& p, void* b) {
+void give(PinnedPool& p, char* b) {
   if (!b) return;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (p.idle.size() < p.keep) {
-      p.idle.push_back(b);
+    if (p.n < p.keep) {
+      p.idle[p.n++] = b;
       return;
     }
   }
   (void)hipHostFree(b);  // teardown
+}
+
+// A block or a ring for the length of a call; p is null where there is none.
+struct Pinned {
+  PinnedPool& pool;
+  char* const p;
+  explicit Pinned(PinnedPool& from) : pool(from), p(take(from)) {}
+  Pinned(const Pinned&) = delete;
+  Pinned& operator=(const Pinned&) = delete;
+  ~Pinned() { give(pool, p); }
+};
+
+int no_block() {
+  return fail(SPH_ENOMEM, "pinned host allocation failed");
 }
 
 }  // namespace
@@ -77,25 +94,17 @@ void stage_close(Stage& s) {
       (void)hipEventDestroy(e);
       e = nullptr;
     }
-  give(g_small, s.small);
-  give(g_ring, s.ring);
-  s.small = s.ring = nullptr;
-  std::vector<void*> drop;
+  give(g_blocks, s.flags);
+  s.flags = nullptr;
+  void* drop[2 * kKeep];
+  size_t n = 0;
   {
     std::lock_guard<std::mutex> lk(g_mu);
     if (--g_handles == 0)
-      for (PinnedPool* p : {&g_small, &g_ring}) {
-        drop.insert(drop.end(), p->idle.begin(), p->idle.end());
-        p->idle.clear();
-      }
+      for (PinnedPool* p : {&g_blocks, &g_rings})
+        while (p->n) drop[n++] = p->idle[--p->n];
   }
-  for (void* b : drop) (void)hipHostFree(b);
-}
-
-static int small_block(Stage& s) {
-  if (!s.small && !(s.small = (char*)take(g_small)))
-    return fail(SPH_ENOMEM, "pinned host allocation of %zu bytes failed", kSmallBlock);
-  return 0;
+  while (n) (void)hipHostFree(drop[--n]);
 }
 
 // n16 16-byte words and the tail4 4-byte words after them
@@ -119,16 +128,17 @@ static int enqueue_copy_out(void* pinned, const void* dev, size_t bytes, hipStre
 // announces each slot or sets `stop`, and the workers copy without blocking.
 static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
   Stage& sg = s->stage;
-  if (!sg.ring && !(sg.ring = (char*)take(g_ring)))
-    return fail(SPH_ENOMEM, "pinned host allocation of %zu bytes failed", kSlot * kSlots);
-  for (auto& e : sg.ev)
-    if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   const size_t nslot = (bytes + kSlot - 1) / kSlot;
+  const size_t nring = nslot > 1 ? kSlots : 1;
+  Pinned ring(nslot > 1 ? g_rings : g_blocks);
+  if (!ring.p) return no_block();
+  for (size_t i = 0; i < nring; ++i)
+    if (!sg.ev[i]) HIPCHK(hipEventCreateWithFlags(&sg.ev[i], hipEventDisableTiming));
   auto length = [&](size_t c) { return c + 1 < nslot ? kSlot : bytes - c * kSlot; };
   auto send = [&](size_t c) -> int {
-    if (enqueue_copy_out(sg.ring + c % kSlots * kSlot, dev + c * kSlot, length(c), s->st))
+    if (enqueue_copy_out(ring.p + c % nring * kSlot, dev + c * kSlot, length(c), s->st))
       return fail(SPH_EDEVICE, "readback launch failed");
-    HIPCHK(hipEventRecord(sg.ev[c % kSlots], s->st));
+    HIPCHK(hipEventRecord(sg.ev[c % nring], s->st));
     return 0;
   };
   std::atomic<size_t> ready{0};    // slots filled so far
@@ -138,7 +148,7 @@ static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
   auto share = [&](size_t c, int who, int n) {
     const size_t len = length(c), part = (len / n + 63) & ~(size_t)63;
     const size_t a = part * who < len ? part * who : len, b = who + 1 == n || a + part > len ? len : a + part;
-    memcpy(dst + c * kSlot + a, sg.ring + c % kSlots * kSlot + a, b - a);
+    memcpy(dst + c * kSlot + a, ring.p + c % nring * kSlot + a, b - a);
   };
   std::vector<std::thread> pool;
   std::atomic<int> members{0};  // set before the first slot is announced
@@ -153,7 +163,7 @@ static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
     }
   };
   int rc = 0;
-  for (size_t c = 0; c < nslot && c < (size_t)kSlots && !rc; ++c) rc = send(c);
+  for (size_t c = 0; c < nslot && c < nring && !rc; ++c) rc = send(c);
   if (!rc) {
     try {
       pool.reserve(want - 1);
@@ -163,18 +173,18 @@ static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
     members.store(nthreads, std::memory_order_relaxed);
   }
   for (size_t c = 0; c < nslot && !rc; ++c) {
-    const hipError_t e = hipEventSynchronize(sg.ev[c % kSlots]);
+    const hipError_t e = hipEventSynchronize(sg.ev[c % nring]);
     if (e != hipSuccess) {
       rc = fail(SPH_EDEVICE, "readback: %s", hipGetErrorString(e));
       break;
     }
     ready.store(c + 1, std::memory_order_release);
     share(c, 0, nthreads);
-    if (c + kSlots < nslot) {
+    if (c + nring < nslot) {
       // the slot is filled again once every worker has taken its share
       while (copied.load(std::memory_order_acquire) < (c + 1) * (size_t)(nthreads - 1))
         std::this_thread::yield();
-      rc = send(c + kSlots);
+      rc = send(c + nring);
     }
   }
   if (rc) stop.store(true);
@@ -200,23 +210,24 @@ __global__ __launch_bounds__(1024) void k_read_ordered(const double* __restrict_
 }
 
 int read_ordered(sph_sim* s, double* dst, const double* dev, const uint32_t* id, int n) {
-  if (int rc = small_block(s->stage)) return rc;
-  hipLaunchKernelGGL(k_read_ordered, dim3(1), dim3(1024), 0, s->st, dev, id, n,
-                     (double*)s->stage.small);
+  Pinned b(g_blocks);
+  if (!b.p) return no_block();
+  hipLaunchKernelGGL(k_read_ordered, dim3(1), dim3(1024), 0, s->st, dev, id, n, (double*)b.p);
   if (hipGetLastError() != hipSuccess) return fail(SPH_EDEVICE, "readback launch failed");
   HIPCHK(hipStreamSynchronize(s->st));
-  memcpy(dst, s->stage.small, n * sizeof(double));
+  memcpy(dst, b.p, n * sizeof(double));
   return 0;
 }
 
 int copy_out(sph_sim* s, void* dst, const void* dev, size_t bytes) {
   if (bytes == 0) return 0;
   if (bytes > kSmallCopy) return copy_slots(s, (char*)dst, (const char*)dev, bytes);
-  if (int rc = small_block(s->stage)) return rc;
-  if (enqueue_copy_out(s->stage.small, dev, bytes, s->st))
+  Pinned b(g_blocks);
+  if (!b.p) return no_block();
+  if (enqueue_copy_out(b.p, dev, bytes, s->st))
     return fail(SPH_EDEVICE, "readback launch failed");
   HIPCHK(hipStreamSynchronize(s->st));
-  memcpy(dst, s->stage.small, bytes);
+  memcpy(dst, b.p, bytes);
   return 0;
 }
 
@@ -240,19 +251,22 @@ __global__ __launch_bounds__(256) void k_flags(const int* __restrict__ err, int 
 }
 
 int enqueue_flags(sph_sim* s, int nerr) {
-  if (sizeof(KnnStats) + (size_t)nerr * sizeof(int) > kSmallBlock)
+  if (sizeof(KnnStats) + (size_t)nerr * sizeof(int) > kSlot)
     return fail(SPH_EINVAL, "too many flags for one block");
-  if (int rc = small_block(s->stage)) return rc;
+  Stage& sg = s->stage;
+  if (!sg.flags && !(sg.flags = take(g_blocks))) return no_block();
   hipLaunchKernelGGL(k_flags, dim3(1), dim3(256), 0, s->st, s->pb.err, nerr, s->pb.stats,
-                     (unsigned long long*)s->stage.small,
-                     (int*)(s->stage.small + sizeof(KnnStats)));
+                     (unsigned long long*)sg.flags, (int*)(sg.flags + sizeof(KnnStats)));
   if (hipGetLastError() != hipSuccess) return fail(SPH_EDEVICE, "flags launch failed");
   return 0;
 }
 
 void take_flags(sph_sim* s, KnnStats* stats, int* err, int nerr) {
-  memcpy(stats, s->stage.small, sizeof *stats);
-  memcpy(err, s->stage.small + sizeof *stats, (size_t)nerr * sizeof(int));
+  Stage& sg = s->stage;
+  memcpy(stats, sg.flags, sizeof *stats);
+  memcpy(err, sg.flags + sizeof *stats, (size_t)nerr * sizeof(int));
+  give(g_blocks, sg.flags);
+  sg.flags = nullptr;
 }
 
 }  // namespace sph
