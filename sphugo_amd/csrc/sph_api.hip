@@ -414,7 +414,7 @@ int sph::check_device_flags(sph_sim* s) {
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(s->st));
   KnnStats st;
-  take_flags(s, &st, &err, 1);
+  if ((rc = take_flags(s, &st, &err, 1))) return rc;
   s->last_stats = st;
   if (err) return fail(SPH_ERANGE, "a particle left the periodic images [-L, 2L) of the box");
   if (st.failures) return fail(SPH_ERANGE, "kNN: %llu searches found fewer than k neighbours",
@@ -773,7 +773,7 @@ extern "C" int sph_knn_stats(sph_sim* s, int64_t* retries, int64_t* ties) {
   int err, rc = enqueue_flags(s, 1);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(s->st));
-  take_flags(s, &st, &err, 1);
+  if ((rc = take_flags(s, &st, &err, 1))) return rc;
   if (retries) *retries = (int64_t)st.retries;
   if (ties) *ties = (int64_t)st.ties;
   return 0;
@@ -785,7 +785,7 @@ extern "C" int sph_knn_counters(sph_sim* s, int64_t out[7]) {
   int err, rc = enqueue_flags(s, 1);
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(s->st));
-  take_flags(s, &st, &err, 1);
+  if ((rc = take_flags(s, &st, &err, 1))) return rc;
   const unsigned long long v[7] = {st.retries, st.ties, st.failures, st.miss_lo,
                                    st.miss_hi, st.miss_ann, st.split_fallback};
   for (int i = 0; i < 7; ++i) out[i] = (int64_t)v[i];

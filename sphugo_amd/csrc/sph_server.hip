@@ -385,7 +385,7 @@ bool tick(sph_server* s) {
     if (!rc && s->ev_tick[1]) e = hipEventRecord(s->ev_tick[1], c.st);
     if (!rc && e == hipSuccess) e = hipStreamSynchronize(c.st);
     if (e != hipSuccess) rc = fail(SPH_EDEVICE, "tick: %s", hipGetErrorString(e));
-    if (!rc) take_flags(&c, &s->h_stats, s->h_err.data(), (int)s->h_err.size());
+    if (!rc) rc = take_flags(&c, &s->h_stats, s->h_err.data(), (int)s->h_err.size());
   }
   std::lock_guard<std::mutex> lk(s->mu);
   if (rc) {

@@ -35,7 +35,7 @@ using sph::SimDev;
 namespace sph {
 // What a handle keeps for its readbacks (sph_stage.hip).
 struct Stage {
-  char* flags = nullptr;   // pinned block from enqueue_flags to take_flags
+  char* flags = nullptr;   // pinned block (or none) from enqueue_flags to take_flags
   hipEvent_t ev[8] = {};   // per slot of a large copy: filled
 };
 void stage_open(Stage& s);
@@ -164,9 +164,10 @@ int copy_out(sph_sim* s, void* dst, const void* dev, size_t bytes);
 inline constexpr int kOrderedMax = 8192;
 int read_ordered(sph_sim* s, double* dst, const double* dev, const uint32_t* id, int n);
 // write the first nerr error flags and the counters' sums to a pinned block
-// (enqueue_flags), and read them there once the stream is done
+// (enqueue_flags), and read them there once the stream is done (take_flags, which
+// copies them itself where there is no block)
 int enqueue_flags(sph_sim* s, int nerr);
-void take_flags(sph_sim* s, sph::KnnStats* stats, int* err, int nerr);
+int take_flags(sph_sim* s, sph::KnnStats* stats, int* err, int nerr);
 int check_device_flags(sph_sim* s);
 int alloc_state(sph_sim* h, int64_t np, int nitems);
 // Cells per particle of a grid (at least; at most four times as many, as a

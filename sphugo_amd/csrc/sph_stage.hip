@@ -44,15 +44,18 @@ std::mutex g_mu;
 PinnedPool g_blocks = {kSlot, 16, {}, 0}, g_rings = {kSlot * kSlots, 4, {}, 0};
 int g_handles = 0;
 
+// null where the runtime has no pinned memory to give: the reads then go through
+// its own copy
 char* take(PinnedPool& p) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
     if (p.n) return (char*)p.idle[--p.n];
   }
   void* b = nullptr;
-  if (hipHostMalloc(&b, p.bytes, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess)
-    return nullptr;
-  return (char*)b;
+  if (hipHostMalloc(&b, p.bytes, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess)
+    return (char*)b;
+  (void)hipGetLastError();  // or the next launch would report it
+  return nullptr;
 }
 
 void give(PinnedPool& p, char* b) {
@@ -67,7 +70,7 @@ void give(PinnedPool& p, char* b) {
   (void)hipHostFree(b);  // teardown
 }
 
-// A block or a ring for the length of a call; p is null where there is none.
+// A block or a ring for the length of a call (or null).
 struct Pinned {
   PinnedPool& pool;
   char* const p;
@@ -76,10 +79,6 @@ struct Pinned {
   Pinned& operator=(const Pinned&) = delete;
   ~Pinned() { give(pool, p); }
 };
-
-int no_block() {
-  return fail(SPH_ENOMEM, "pinned host allocation failed");
-}
 
 }  // namespace
 
@@ -107,6 +106,12 @@ void stage_close(Stage& s) {
   while (n) (void)hipHostFree(drop[--n]);
 }
 
+static int copy_pageable(sph_sim* s, void* dst, const void* dev, size_t bytes) {
+  HIPCHK(hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s->st));
+  HIPCHK(hipStreamSynchronize(s->st));
+  return 0;
+}
+
 // n16 16-byte words and the tail4 4-byte words after them
 __global__ __launch_bounds__(256) void k_copy_out(const char* __restrict__ src,
                                                   char* __restrict__ dst, int64_t n16, int tail4) {
@@ -131,7 +136,7 @@ static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
   const size_t nslot = (bytes + kSlot - 1) / kSlot;
   const size_t nring = nslot > 1 ? kSlots : 1;
   Pinned ring(nslot > 1 ? g_rings : g_blocks);
-  if (!ring.p) return no_block();
+  if (!ring.p) return copy_pageable(s, dst, dev, bytes);
   for (size_t i = 0; i < nring; ++i)
     if (!sg.ev[i]) HIPCHK(hipEventCreateWithFlags(&sg.ev[i], hipEventDisableTiming));
   auto length = [&](size_t c) { return c + 1 < nslot ? kSlot : bytes - c * kSlot; };
@@ -211,9 +216,10 @@ __global__ __launch_bounds__(1024) void k_read_ordered(const double* __restrict_
 
 int read_ordered(sph_sim* s, double* dst, const double* dev, const uint32_t* id, int n) {
   Pinned b(g_blocks);
-  if (!b.p) return no_block();
-  hipLaunchKernelGGL(k_read_ordered, dim3(1), dim3(1024), 0, s->st, dev, id, n, (double*)b.p);
+  hipLaunchKernelGGL(k_read_ordered, dim3(1), dim3(1024), 0, s->st, dev, id, n,
+                     b.p ? (double*)b.p : s->d_scratch);
   if (hipGetLastError() != hipSuccess) return fail(SPH_EDEVICE, "readback launch failed");
+  if (!b.p) return copy_pageable(s, dst, s->d_scratch, n * sizeof(double));
   HIPCHK(hipStreamSynchronize(s->st));
   memcpy(dst, b.p, n * sizeof(double));
   return 0;
@@ -223,7 +229,7 @@ int copy_out(sph_sim* s, void* dst, const void* dev, size_t bytes) {
   if (bytes == 0) return 0;
   if (bytes > kSmallCopy) return copy_slots(s, (char*)dst, (const char*)dev, bytes);
   Pinned b(g_blocks);
-  if (!b.p) return no_block();
+  if (!b.p) return copy_pageable(s, dst, dev, bytes);
   if (enqueue_copy_out(b.p, dev, bytes, s->st))
     return fail(SPH_EDEVICE, "readback launch failed");
   HIPCHK(hipStreamSynchronize(s->st));
@@ -251,22 +257,33 @@ __global__ __launch_bounds__(256) void k_flags(const int* __restrict__ err, int 
 }
 
 int enqueue_flags(sph_sim* s, int nerr) {
-  if (sizeof(KnnStats) + (size_t)nerr * sizeof(int) > kSlot)
-    return fail(SPH_EINVAL, "too many flags for one block");
   Stage& sg = s->stage;
-  if (!sg.flags && !(sg.flags = take(g_blocks))) return no_block();
+  if (sizeof(KnnStats) + (size_t)nerr * sizeof(int) > kSlot) return 0;  // take_flags copies them
+  if (!sg.flags && !(sg.flags = take(g_blocks))) return 0;
   hipLaunchKernelGGL(k_flags, dim3(1), dim3(256), 0, s->st, s->pb.err, nerr, s->pb.stats,
                      (unsigned long long*)sg.flags, (int*)(sg.flags + sizeof(KnnStats)));
   if (hipGetLastError() != hipSuccess) return fail(SPH_EDEVICE, "flags launch failed");
   return 0;
 }
 
-void take_flags(sph_sim* s, KnnStats* stats, int* err, int nerr) {
+int take_flags(sph_sim* s, KnnStats* stats, int* err, int nerr) {
   Stage& sg = s->stage;
+  if (!sg.flags) {
+    KnnStats slot[kStatSlots];
+    int rc = copy_pageable(s, slot, s->pb.stats, sizeof slot);
+    if (!rc) rc = copy_pageable(s, err, s->pb.err, (size_t)nerr * sizeof(int));
+    if (rc) return rc;
+    *stats = {};
+    for (const KnnStats& v : slot)
+      for (size_t i = 0; i < sizeof v / sizeof(unsigned long long); ++i)
+        ((unsigned long long*)stats)[i] += ((const unsigned long long*)&v)[i];
+    return 0;
+  }
   memcpy(stats, sg.flags, sizeof *stats);
   memcpy(err, sg.flags + sizeof *stats, (size_t)nerr * sizeof(int));
   give(g_blocks, sg.flags);
   sg.flags = nullptr;
+  return 0;
 }
 
 }  // namespace sph
