@@ -9,6 +9,8 @@
 // one slot (with up to four threads: new pages cost more than the bytes) while
 // the next ones fill: 18, 23, 51 us and 2.1 ms for the same reads.
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -128,9 +130,13 @@ static int enqueue_copy_out(void* pinned, const void* dev, size_t bytes, hipStre
   return (int)hipGetLastError();
 }
 
-// The host side of a large copy: `workers` threads and the caller copy their
-// share of every slot the caller announces.  Every wait ends: the caller
-// announces each slot or sets `stop`, and the workers copy without blocking.
+// The host side of a large copy: up to three workers and the caller copy their
+// share of every slot the caller announces.  The stream may have much to do before
+// the first one (the passes of a server's tick): the workers ask for it, in turns,
+// no longer than kAsk and sleep from then on (asleep at once, 32 simulations' fields
+// were 2 % slower: a woken thread comes 10 us after its slot).  Every wait ends: the
+// caller announces each slot or sets `stop`, and the workers copy without blocking.
+constexpr std::chrono::microseconds kAsk{200};
 static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
   Stage& sg = s->stage;
   const size_t nslot = (bytes + kSlot - 1) / kSlot;
@@ -157,7 +163,20 @@ static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
   };
   std::vector<std::thread> pool;
   std::atomic<int> members{0};  // set before the first slot is announced
+  std::mutex mu;
+  std::condition_variable first;  // the first slot, or `stop`
+  auto begun = [&] { return ready.load() > 0 || stop.load(); };
+  auto wake = [&] {
+    { std::lock_guard<std::mutex> lk(mu); }  // none between its test and its sleep
+    first.notify_all();
+  };
   auto work = [&](int who) {
+    const auto until = std::chrono::steady_clock::now() + kAsk;
+    while (!begun() && std::chrono::steady_clock::now() < until) std::this_thread::yield();
+    if (!begun()) {
+      std::unique_lock<std::mutex> lk(mu);
+      first.wait(lk, begun);
+    }
     for (size_t c = 0; c < nslot; ++c) {
       while (ready.load(std::memory_order_acquire) <= c) {
         if (stop.load(std::memory_order_relaxed)) return;
@@ -183,7 +202,8 @@ static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
       rc = fail(SPH_EDEVICE, "readback: %s", hipGetErrorString(e));
       break;
     }
-    ready.store(c + 1, std::memory_order_release);
+    ready.store(c + 1);
+    if (c == 0 && nthreads > 1) wake();
     share(c, 0, nthreads);
     if (c + nring < nslot) {
       // the slot is filled again once every worker has taken its share
@@ -192,7 +212,10 @@ static int copy_slots(sph_sim* s, char* dst, const char* dev, size_t bytes) {
       rc = send(c + nring);
     }
   }
-  if (rc) stop.store(true);
+  if (rc) {
+    stop.store(true);
+    wake();
+  }
   for (auto& t : pool) t.join();
   // what was sent before a failure must not outlive the ring's contents
   if (rc) (void)hipStreamSynchronize(s->st);

@@ -3,6 +3,7 @@ host threads."""
 import os
 import subprocess
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -105,3 +106,18 @@ def test_reads_without_pinned_memory(tmp_path):
     r = subprocess.run([sys.executable, str(prog), str(lib), ROOT], capture_output=True, text=True,
                        timeout=100)
     assert r.returncode == 0 and r.stdout.split()[-1] == "whole", r.stdout + r.stderr[-2000:]
+
+
+def test_waiting_for_the_gpu_takes_one_thread():
+    """A large read behind a queue of steps: until they are done only the caller
+    waits (its own wait is the runtime's, which may spin)."""
+    g = _sim(1 << 20, k=16, dt_half=1e-9)
+    g.step(1)
+    g.get("x")
+    g.step_async(300)
+    wall, cpu = time.perf_counter(), time.process_time()
+    g.get("x")
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert wall > 0.02  # long beside the copy itself
+    assert cpu < 2 * wall
+    g.synchronize()
