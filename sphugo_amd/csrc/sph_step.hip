@@ -2762,8 +2762,11 @@ __global__ __launch_bounds__(256) void k_read_nbrs(const Item* __restrict__ item
       x = pj.x - ox;
       y = pj.y - oy;
     }
+    // what the row is ordered by: a distance that is no number (a particle of a state
+    // gone bad) comes last, so that every place is taken once
+    const double by = d2 == d2 ? d2 : INFINITY;
     wave_fence();
-    sd[r][e] = d2;
+    sd[r][e] = by;
     sid[r][e] = id;
     wave_fence();
     int at = e;
@@ -2772,7 +2775,7 @@ __global__ __launch_bounds__(256) void k_read_nbrs(const Item* __restrict__ item
       for (int m = 0; m < k; ++m) {
         const double v = sd[r][m];
         const uint32_t w = sid[r][m];
-        at += v < d2 || (v == d2 && (w < id || (w == id && m < e)));
+        at += v < by || (v == by && (w < id || (w == id && m < e)));
       }
     }
     if (e < kout) {
