@@ -1631,10 +1631,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const uint32_t dense =
           (uint32_t)ballot(grp && c_lo < k && c_an > kAnn && c_lo + c_an >= k) & 0xFFFFu;
       if (dense) {
-        ntight += (unsigned)__builtin_popcount(dense);
         wave_fence();
         if (images) tighten<true>(sh, gq, ncand, dense, t0, k, lx, ly, lane, c_lo, c_an);
         else tighten<false>(sh, gq, ncand, dense, t0, k, lx, ly, lane, c_lo, c_an);
+        // those that it resolved: the others count as misses below
+        ntight += (unsigned)__builtin_popcount(
+            dense & (uint32_t)ballot(c_an <= kAnn && c_lo + c_an >= k));
       }
       wave_fence();
       const double xq = gq[ql].x, yq = gq[ql].y;
