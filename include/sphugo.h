@@ -263,10 +263,14 @@ int sph_set_tuning(sph_sim* s, const double in[5]);
 
 /* ---- serve loop: continuous batching (no reference counterpart) ----
  * A native worker thread steps every admitted job in one shared device
- * pool: each tick is a force pass (up to four while no job arrives or ends)
- * over all resident jobs, which may be at different steps of their lives; a
- * job that ends frees its particle range for the next one in the queue (FIFO,
- * first fit).  A job's results equal those of sph_create + sph_step(nsteps)
+ * pool, force pass by force pass over all resident jobs, which may be at
+ * different steps of their lives; a job that ends frees its particle range for
+ * the next one in the queue (FIFO, first fit).  The worker looks at the queue
+ * and at the jobs' errors between passes, after every one or, where at most
+ * about 500,000 particles run (a pass of some 0.4 ms), after up to four in
+ * which no job ends: a job that arrives meanwhile is admitted, a job that
+ * failed ends, and the steps that sph_server_job_info reports count on, that
+ * much later.  A job's results equal those of sph_create + sph_step(nsteps)
  * with the same inputs.  All calls are thread-safe. */
 typedef struct sph_server sph_server;
 
