@@ -71,14 +71,14 @@ extern "C" {
 #define SPH_H 13 /* k-th neighbour distance, NNDists[0] */
 #define SPH_NFIELDS 14
 
-/* per-kernel timer slots (SPH_FLAG_TIMING) */
-#define SPH_T_KEYS 0
+/* per-kernel timer slots (SPH_FLAG_TIMING); what launches nothing counts nothing */
+#define SPH_T_KEYS 0 /* nothing where the sort makes one simulation's keys */
 #define SPH_T_SORT 1
 #define SPH_T_PERMUTE 2
 #define SPH_T_KNN_DENSITY 3
 #define SPH_T_FORCE 4
 #define SPH_T_REDUCE 5 /* nothing in small launches, whose force adds the totals up */
-/* the three launches inside SPH_T_KNN_DENSITY */
+/* the launches inside SPH_T_KNN_DENSITY */
 #define SPH_T_KNN_WALK 6     /* bracketed walk, density, force records */
 #define SPH_T_KNN_FINISH 7   /* nothing (part of the walk) */
 #define SPH_T_KNN_FALLBACK 8 /* exact wavefront search of the remaining queries */

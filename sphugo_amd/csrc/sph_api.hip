@@ -400,6 +400,7 @@ static int run_pass(sph_sim* s, int perm_mode, int force_mode) {
     HIPCHK(hipStreamSynchronize(s->st));
     for (int t = 0; t < SPH_NTIMERS; ++t) {
       float ms = 0;
+      if (!(s->pb.timed >> t & 1u)) continue;
       if (hipEventElapsedTime(&ms, s->ev[2 * t], s->ev[2 * t + 1]) == hipSuccess) {
         s->t_ms[t] += ms;
         s->t_cnt[t] += 1;

@@ -70,18 +70,19 @@ struct PassBuffers {
   int have_h;             // every particle has an h from an earlier pass, except:
   int some_new;           // some simulations do not (a server admitted them)
   int any_open;           // some simulation has an open axis (k_bbox, k_box run)
+  uint32_t timed;         // kernel classes timed in the last pass, a bit each
   WalkKnobs walk;         // tile-search shape of the kNN walk
   int* err;             // device error flags: [0] any, [1 + s] simulation s (1: a
                         // particle left the images, 2: kNN found fewer than k)
   SortBuffers sort;
 };
 
-// Enqueue one force pass (keys, sort, permute, kNN + density, force,
-// reductions) on `st`.  Timing events (may be null) are recorded around
-// each kernel class.
 // u32 entries of the neighbour lists of np queries (64-query tiles)
 inline int64_t nbr_entries(int64_t np, int kstride) { return (np + 63) / 64 * 64 * kstride; }
 
+// Enqueue one force pass (keys, sort, permute, kNN + density, force,
+// reductions) on `st`.  Timing events (may be null) are recorded around
+// each kernel class that launches something (PassBuffers::timed).
 int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
                  hipEvent_t* ev /* 2*SPH_NTIMERS or null */);
 

@@ -2550,27 +2550,30 @@ __global__ void k_init_sims(SimDev* sims, int nsims) {
 // ------------------------------------------------------------------------
 int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
                  hipEvent_t* ev) {
+  b.timed = 0;
   auto mark = [&](int slot, int end) {
-    if (ev) (void)hipEventRecord(ev[2 * slot + end], st);  // timing only
+    if (!ev) return;
+    (void)hipEventRecord(ev[2 * slot + end], st);  // timing only
+    b.timed |= 1u << slot;
   };
   const dim3 blk(kItem);
   const dim3 grd(b.nitems);
   const dim3 grd_all(b.nitems_all);
-  mark(0, 0);
+  const KeySrc src = {b.sims, b.pos_cur.x, b.pos_cur.y, b.fcur.vx, b.fcur.vy, perm_mode, b.err,
+                      b.retry_count};
+  // one simulation: the sort's first read of the keys makes them
+  const bool fused = b.nsims == 1 && b.hole_cpp == 0 && sort_makes_keys(b.np);
+  if (!fused || b.any_open) mark(0, 0);
   if (b.any_open) {
     hipLaunchKernelGGL(k_bbox, grd, blk, 0, st, b.items, b.nitems, b.sims, b.pos_cur.x,
                        b.pos_cur.y, b.fcur.vx, b.fcur.vy, perm_mode, b.partials);
     hipLaunchKernelGGL(k_box, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, b.red_first,
                        b.red_count);
   }
-  const KeySrc src = {b.sims, b.pos_cur.x, b.pos_cur.y, b.fcur.vx, b.fcur.vy, perm_mode, b.err,
-                      b.retry_count};
-  // one simulation: the sort's first read of the keys makes them
-  const bool fused = b.nsims == 1 && b.hole_cpp == 0 && sort_makes_keys(b.np);
   if (!fused)
     hipLaunchKernelGGL(k_keys, grd_all, blk, 0, st, b.items_all, b.nitems_all, src, b.sort.keys,
                        b.hole_cpp);
-  mark(0, 1);
+  if (!fused || b.any_open) mark(0, 1);
   mark(1, 0);
   uint32_t *skeys = nullptr, *perm = nullptr;
   sort_pairs(b.sort, b.np, b.key_bits, st, fused ? &src : nullptr, &skeys, &perm);
@@ -2611,8 +2614,6 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
     else if (b.prec == kPrecFP32C) SPH_KNN(true, false, false, 0);
     else SPH_KNN(false, false, false, 0);
     mark(6, 1);
-    mark(7, 0);
-    mark(7, 1);
     mark(8, 0);
     if (b.bitwise) SPH_FB(true, false);
     else if (b.prec == kPrecFP32C) SPH_FB(false, true);
@@ -2642,15 +2643,15 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
 #undef SPH_FORCE_
 #undef SPH_FORCE
   mark(4, 1);
-  mark(5, 0);
   if (!finish) {
+    mark(5, 0);
     if (b.red_parts_max > 1)
       hipLaunchKernelGGL(k_reduce_part, dim3(b.nsims * b.red_parts_max), dim3(256), 0, st, b.sims,
                          b.partials, parts, b.red_first, b.red_count, b.red_part, b.red_parts_max);
     hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, parts,
                        b.red_part, b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss);
+    mark(5, 1);
   }
-  mark(5, 1);
   return (int)hipGetLastError();
 }
 
