@@ -204,7 +204,7 @@ int sph::alloc_state(sph_sim* h, int64_t np, int nitems) {
       (rc = h->alloc(&pb.nbr, nbr_entries(np, pb.kmax))) ||
       (rc = h->alloc((char**)&pb.rec,
                      np * (int64_t)(h->prec == SPH_PREC_FP32C ? sizeof(RecF) : sizeof(RecD)))) ||
-      (rc = h->alloc(&pb.partials, (int64_t)nitems * 4 * kNumRed)) ||
+      (rc = h->alloc(&pb.partials, partial_rows(nitems, pb.kmax) * kNumRed)) ||
       (rc = h->alloc(&pb.stats, kStatSlots)) || (rc = h->alloc(&pb.err, 1 + pb.nsims)) ||
       (rc = h->alloc(&pb.walk_miss, (int64_t)pb.nsims * kMissSlots * kMissStride)) ||
       (rc = h->alloc(&pb.red_part, (int64_t)pb.nsims * kRedSplit * kNumRed)) ||

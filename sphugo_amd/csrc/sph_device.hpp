@@ -249,11 +249,6 @@ __device__ inline int xcd_item(int nitems, int b) {
 }
 __device__ inline int xcd_item(int nitems) { return xcd_item(nitems, (int)blockIdx.x); }
 
-__device__ inline int64_t floordiv(int64_t a, int64_t b) {
-  int64_t q = a / b;
-  if ((a % b != 0) && ((a < 0) != (b < 0))) --q;
-  return q;
-}
 // floor(a / 2^s): the arithmetic shift (every grid and level has 2^s cells
 // per axis, so no 64-bit division is needed on the device)
 __device__ inline int64_t floordiv_pow2(int64_t a, int s) { return a >> s; }
@@ -381,12 +376,6 @@ struct WendlandF {
     return -10 * q * (a * a * a);
   }
 };
-__device__ inline float kern_Ff(int32_t kernel, float q) {
-  return kernel == kWendland ? WendlandF::F(q) : CubicF::F(q);
-}
-__device__ inline float kern_DFf(int32_t kernel, float q) {
-  return kernel == kWendland ? WendlandF::DF(q) : CubicF::DF(q);
-}
 // Calls f(CubicF{}) or f(WendlandF{}) for the simulation's kernel type.
 template <typename Fn>
 __device__ inline void kern_visit(int32_t kernel, Fn&& f) {
@@ -463,10 +452,6 @@ __device__ inline int wave_incl_scan(int v) {
 // butterfly sum over groups of `width` lanes (power of two); every lane of
 // a group ends with the same value (a+b == b+a exactly)
 __device__ inline double group_sum(double v, int width) {
-  for (int o = width >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ inline float group_sumf(float v, int width) {
   for (int o = width >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }

@@ -59,7 +59,7 @@ struct PassBuffers {
   uint32_t* cstart;     // ncells + 1
   uint32_t* nbr;        // np * kmax packed (index << 4 | image code)
   void* rec;            // np force records (RecD or RecF)
-  double* partials;     // nitems * 4 * kNumRed (a wave's 64 particles, or an item's 256)
+  double* partials;     // kNumRed per item, or per 64 particles where the force splits rows
   KnnStats* stats;      // kStatSlots copies
   uint32_t* walk_miss;  // per simulation: the walk's miss counts (kMissSlots lines)
   double* red_part;     // per simulation: kRedSplit first-stage sums (kNumRed each)
@@ -79,6 +79,9 @@ struct PassBuffers {
 
 // u32 entries of the neighbour lists of np queries (64-query tiles)
 inline int64_t nbr_entries(int64_t np, int kstride) { return (np + 63) / 64 * 64 * kstride; }
+
+// rows of `partials` for launches of up to nitems items
+int64_t partial_rows(int nitems, int kmax);
 
 // Enqueue one force pass (keys, sort, permute, kNN + density, force,
 // reductions) on `st`.  Timing events (may be null) are recorded around

@@ -1747,28 +1747,15 @@ inline int walk_waves_per_item(int nitems, int group) {
 template <typename T>
 __device__ inline uint64_t rec_off(uint32_t pk) {
   constexpr int sz = (int)sizeof(T);
-  static_assert(sz == 8 || sz == 16 || sz == 32 || sz == 64, "record size");
-  const uint32_t m = pk & ~15u;
-  if constexpr (sz == 8) return m >> 1;
-  else if constexpr (sz == 16) return m;
-  else return (uint64_t)m << (sz == 32 ? 1 : 2);
+  static_assert(sz == 32 || sz == 64, "record size");
+  return (uint64_t)(pk & ~15u) << (sz == 32 ? 1 : 2);
 }
 
-// Sources of the neighbour gathers, indexed by packed entry.  A gather runs
+// Source of the neighbour gathers, indexed by packed entry.  A gather runs
 // in three steps over a round's entries: near() issues the first load and
 // says whether it is the value, pin() waits for those loads, far() loads the
-// rest.  An array: one global load.
-template <typename T>
-struct ArrSrc {
-  const T* __restrict__ g;
-  __device__ bool near(uint32_t pk, T& v) const {
-    v = *(const T*)((const char*)g + rec_off<T>(pk));
-    return true;
-  }
-  __device__ void pin(T&) const {}
-  __device__ T far(uint32_t pk) const { return *(const T*)((const char*)g + rec_off<T>(pk)); }
-};
-
+// rest.
+//
 // An array read through a block's LDS window: entries [wb, wb + W)
 // (indices mod 2^32) come from the staged copy, the rest from the array.
 // Particles are in Hilbert order, so most neighbours of a block's 256
@@ -1833,38 +1820,28 @@ __device__ inline void stage_window(u32x4* lds, const T* __restrict__ g, int64_t
   }
 }
 
-// Visits the entries [n0, k) of a neighbour row (n0 a multiple of 4), N (4 or
-// 8) at a time: the N sources (src's records of the entries) are gathered
-// together and the next N entries' row chunks are loaded before the current N
-// are processed, so that the row and gather latencies overlap.  Full rounds
-// gather their entries as they are; a last partial round gathers the query's
-// own slot `self` for the entries past k.  NT: the row is read for the last
-// time (non-temporal loads).  IMAGES: `body` is told (as a type) whether an
-// entry of the wave's round may be an image, which few waves' are.  `flush` runs
-// after each round of N entries, with the next round's first.
-template <int N, bool NT = false, bool IMAGES = false, typename S, typename Body, typename Flush>
+// Visits the entries [n0, k) of a neighbour row (n0 a multiple of 4) in rounds of
+// four: their sources (src's records of the entries) are gathered together and
+// the next row chunk is loaded before the current one is processed, so that the
+// row and gather latencies overlap; the row is read for the last time
+// (non-temporal loads).  Full rounds gather their entries as they are; a last
+// partial round gathers the query's own slot `self` for the entries past k.
+// IMAGES: `body` is told (as a type) whether an entry of the wave's round may be an
+// image, which few waves' are.  `flush` runs after each round, with the next
+// round's first entry.
+template <bool IMAGES = false, typename S, typename Body, typename Flush>
 __device__ inline void row_visit(const NbrRow row, int n0, int k, uint32_t self, const S& src,
                                  Body body, Flush flush) {
-  static_assert(N == 4 || N == 8, "one or two row chunks per round");
+  constexpr int N = 4;
   if (n0 >= k) return;
   using T = std::remove_cv_t<std::remove_reference_t<decltype(src.far(0u))>>;
-  auto ld = [&](int c) {
-    if constexpr (NT) return __builtin_nontemporal_load(row.chunk(c));
-    else return *row.chunk(c);
-  };
-  // entries past k are never read from the chunks (they gather `self`), so a
-  // chunk past the row is zeros rather than a copy that waits for a load
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  u32x4 qa = ld(n0 >> 2);
-  u32x4 qb = (N == 8 && k > n0 + 4) ? ld((n0 >> 2) + 1) : zero;
+  auto ld = [&](int c) { return __builtin_nontemporal_load(row.chunk(c)); };
+  u32x4 q = ld(n0 >> 2);
   for (; n0 + N <= k; n0 += N) {
-    const uint32_t pks[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+    const uint32_t pks[N] = {q.x, q.y, q.z, q.w};
     T pj[N];
     gather<N>(src, pks, pj);
-    if (n0 + N < k) {
-      qa = ld((n0 + N) >> 2);
-      if constexpr (N == 8) qb = n0 + 12 < k ? ld(((n0 + N) >> 2) + 1) : zero;
-    }
+    if (n0 + N < k) q = ld((n0 + N) >> 2);
     auto round = [&](auto img) {
 #pragma unroll
       for (int u = 0; u < N; ++u) body(pks[u], pj[u], img);
@@ -1881,7 +1858,7 @@ __device__ inline void row_visit(const NbrRow row, int n0, int k, uint32_t self,
   }
   if (n0 < k) {
     const uint32_t spk = self << 4;
-    const uint32_t pks[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+    const uint32_t pks[N] = {q.x, q.y, q.z, q.w};
     uint32_t gpk[N];
 #pragma unroll
     for (int u = 0; u < N; ++u) gpk[u] = n0 + u < k ? pks[u] : spk;
@@ -1979,6 +1956,9 @@ inline constexpr int kSections = 4;
 // 32,768 13.9 and 14.3; k = 32 32,768 19.4 and 16.0, 49,152 20.0 and 19.9; k = 64 49,152
 // 30.5 and 23.5; 262,144 at k = 32 38 and 60.
 inline int force_split_items(int kmax) { return 64 + 2 * kmax; }
+int64_t partial_rows(int nitems, int kmax) {
+  return std::max<int64_t>(nitems, (int64_t)kSections * std::min(nitems, force_split_items(kmax)));
+}
 __host__ __device__ inline int section_begin(int k, int s) { return 4 * (((k + 3) / 4 * s) >> 2); }
 
 // The sum of the sections done, and the entry after the current one.
@@ -2154,7 +2134,7 @@ __global__ __launch_bounds__(256) void k_force(
       }
     };
     if constexpr (EXACT) {
-      row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb, auto) {
+      row_visit(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb, auto) {
         // the reference's arithmetic, operation for operation
         const double ox = (double)img_ix(pk & 15u) * lx, oy = (double)img_iy(pk & 15u) * ly;
         const double rABx = (nb.x - ox) - xi, rABy = (nb.y - oy) - yi;
@@ -2183,7 +2163,7 @@ __global__ __launch_bounds__(256) void k_force(
       // throughout
       const double acih = alpha * cih;
       kern_visit(kern, [&](auto kt) {
-        row_visit<4, true, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb,
+        row_visit<true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecD& nb,
                                                                      auto img) {
 #pragma clang fp contract(fast)
           double rABx = nb.x - xi, rABy = nb.y - yi;
@@ -2289,12 +2269,12 @@ __global__ __launch_bounds__(256) void k_force(
       // wave whose queries all take fixed-point displacements (the usual case)
       // runs a loop without the FP64 form, so every record loads whole.
       if (__all(fixed)) {
-        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t, const RecF& nb, auto) {
+        row_visit(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t, const RecF& nb, auto) {
           pair(__builtin_fmaf((float)(int32_t)(nb.ux - me.ux), fsx, csx),
                __builtin_fmaf((float)(int32_t)(nb.uy - me.uy), fsy, csy), nb);
         }, flush);
       } else {
-        row_visit<4, true>(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecF& nb, auto) {
+        row_visit(row, n0, n1, (uint32_t)t, wsrc, [&](uint32_t pk, const RecF& nb, auto) {
           float rx, ry;
           if (fixed) {
             rx = __builtin_fmaf((float)(int32_t)(nb.ux - me.ux), fsx, csx);
@@ -2447,17 +2427,8 @@ __device__ inline void block_sum(double (*sh)[256], double (&acc)[kNumRed]) {
   }
 }
 
-// Item i's force partial r, from one or four values (a wave's 64 particles
-// each): the same sum either way.
-__device__ inline double item_partial(const double* __restrict__ partials, int parts, int64_t i,
-                                      int r) {
-  const double* p = partials + i * parts * kNumRed + r;
-  return parts == 1 ? p[0] : (p[0] + p[kNumRed]) + (p[2 * kNumRed] + p[3 * kNumRed]);
-}
-
 __global__ __launch_bounds__(256) void k_reduce_part(const SimDev* __restrict__ sims,
                                                      const double* __restrict__ partials,
-                                                     int parts_per_item,
                                                      const int* __restrict__ item_first,
                                                      const int* __restrict__ item_count,
                                                      double* __restrict__ red_part,
@@ -2476,7 +2447,7 @@ __global__ __launch_bounds__(256) void k_reduce_part(const SimDev* __restrict__ 
 #pragma unroll 4
   for (int i = ia + (int)threadIdx.x; i < ib; i += 256)
 #pragma unroll
-    for (int r = 0; r < kNumRed; ++r) acc[r] += item_partial(partials, parts_per_item, i0 + i, r);
+    for (int r = 0; r < kNumRed; ++r) acc[r] += partials[(int64_t)(i0 + i) * kNumRed + r];
   block_sum(sh, acc);
   if (threadIdx.x < kNumRed)
     red_part[((int64_t)sim * kRedSplit + part) * kNumRed + threadIdx.x] = sh[threadIdx.x][0];
@@ -2486,7 +2457,6 @@ __global__ __launch_bounds__(256) void k_reduce_part(const SimDev* __restrict__ 
 // TotalMomentum quirk value and what follows from them.
 __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
                                                 const double* __restrict__ partials,
-                                                int parts_per_item,
                                                 const double* __restrict__ red_part,
                                                 const int* __restrict__ item_first,
                                                 const int* __restrict__ item_count, Fields f,
@@ -2520,7 +2490,7 @@ __global__ __launch_bounds__(256) void k_reduce(SimDev* __restrict__ sims,
 #pragma unroll 8
     for (int i = tid; i < ni; i += 256)
 #pragma unroll
-      for (int r = 0; r < kNumRed; ++r) acc[r] += item_partial(partials, parts_per_item, i0 + i, r);
+      for (int r = 0; r < kNumRed; ++r) acc[r] += partials[(int64_t)(i0 + i) * kNumRed + r];
   } else if (tid < nparts) {
 #pragma unroll
     for (int r = 0; r < kNumRed; ++r)
@@ -2647,9 +2617,9 @@ int enqueue_pass(PassBuffers& b, int perm_mode, int force_mode, hipStream_t st,
     mark(5, 0);
     if (b.red_parts_max > 1)
       hipLaunchKernelGGL(k_reduce_part, dim3(b.nsims * b.red_parts_max), dim3(256), 0, st, b.sims,
-                         b.partials, parts, b.red_first, b.red_count, b.red_part, b.red_parts_max);
-    hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, parts,
-                       b.red_part, b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss);
+                         b.partials, b.red_first, b.red_count, b.red_part, b.red_parts_max);
+    hipLaunchKernelGGL(k_reduce, dim3(b.nsims), dim3(256), 0, st, b.sims, b.partials, b.red_part,
+                       b.red_first, b.red_count, b.fnew, force_mode, b.walk_miss);
     mark(5, 1);
   }
   return (int)hipGetLastError();
