@@ -197,7 +197,8 @@ int sph_set_timing(sph_sim* s, int32_t on);
 int sph_knn_stats(sph_sim* s, int64_t* retries, int64_t* ties);
 /* All kNN counters since sph_create: retries, ties, failures, bracket
  * misses (k inside the inner radius, fewer than k inside the outer radius,
- * annulus over capacity), tiles sent to the wavefront search. */
+ * annulus over capacity, however often halved), queries whose group of four was
+ * still too full. */
 int sph_knn_counters(sph_sim* s, int64_t out[7]);
 
 /* ---- checkpoint and resume (no reference counterpart: the reference keeps

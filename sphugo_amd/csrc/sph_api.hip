@@ -472,8 +472,8 @@ extern "C" int sph_set_graph(sph_sim* s, int32_t on) {
 
 // Autotuner: times force passes over the candidate grid resolutions on the
 // current state (only before the first step) and keeps the fastest.  The
-// step-0 pass that follows searches every query exactly, as an untuned
-// handle's does.  The grid changes the order in which neighbours are found
+// step-0 pass that follows finds every h anew, as an untuned handle's does, so
+// nothing of the tuning passes but the choice is left.  The grid changes the order in which neighbours are found
 // and so the summation order: results stay bit-identical in the bitwise
 // form and within the 1e-12 (FP64) and 1e-5 (FP32C density) contracts
 // otherwise; neighbour sets and h are the same.
@@ -566,7 +566,7 @@ extern "C" int sph_autotune(sph_sim* s, double* best_ms, double* best_cpp) {
   HIPCHK(hipMemcpyAsync(s->pb.sims, s->hsims.data(), s->hsims.size() * sizeof(SimDev),
                         hipMemcpyHostToDevice, s->st));
   HIPCHK(hipStreamSynchronize(s->st));
-  s->pb.have_h = 0;  // step 0 searches exactly, as without tuning
+  s->pb.have_h = 0;  // step 0 is a first pass, as without tuning
   if (best_ms) *best_ms = best;
   if (best_cpp) *best_cpp = bcpp;
   return check_device_flags(s);

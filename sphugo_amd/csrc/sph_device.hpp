@@ -83,13 +83,13 @@ struct SimDev {
 
 // Bracket adaptation after a pass with n queries, from its walk's misses
 // because h moved past the bracket (fewer than k within it, or k within its
-// inner radius) and its annulus overflows: a miss rate above 1/128
-// of either kind moves delta by a quarter (towards the kind that dominates),
+// inner radius) and its annulus overflows (resolved in the walk by halving the
+// annulus, or missed): a rate above 1/128 of either kind moves delta by a quarter (towards the kind that dominates),
 // not past [kDeltaMin, kDeltaMax]; once both stay below a quarter of that
 // rate it moves a tenth back towards the configured d0, and in between it
 // holds (so a burst of motion widens it for as long as it lasts, and it
-// does not settle at the edge of the widening threshold).  Neighbour sets and h do not depend on delta (every miss is
-// searched exactly); the share of queries the walk resolves does, and
+// does not settle at the edge of the widening threshold).  Neighbour sets and h
+// do not depend on delta (every miss is searched exactly); the share of queries the walk resolves does, and
 // outside the bitwise form so does the order in which a row's neighbours
 // are summed.  The counts are integers, so the adaptation is deterministic.
 constexpr double kDeltaMin = 0.0125, kDeltaMax = 0.1;
@@ -220,13 +220,14 @@ struct WalkKnobs {
 constexpr WalkKnobs kWalkDefault = {0.025, 24, 64, 8, 0};
 
 struct KnnStats {
-  unsigned long long retries;         // searches needing a second radius
+  unsigned long long retries;         // queries with an h that the walk left to the exact
+                                      // search, and that search's second radii
   unsigned long long ties;            // exact d2 ties at the k-th boundary
   unsigned long long failures;        // searches that found fewer than k
   unsigned long long miss_lo;         // bracket: k or more inside h(1-delta)
   unsigned long long miss_hi;         // bracket: fewer than k inside h(1+delta)
-  unsigned long long miss_ann;        // bracket: annulus over capacity
-  unsigned long long split_fallback;  // tile too wide even for 8 lanes
+  unsigned long long miss_ann;        // bracket: annulus over capacity, however often halved
+  unsigned long long split_fallback;  // box too full even for a group of 4
 };
 
 // kNN counters are spread over kStatSlots copies, chosen by block, so that
@@ -385,8 +386,9 @@ __device__ inline void kern_visit(int32_t kernel, Fn&& f) {
 
 // FP64 reciprocal and reciprocal square root: the hardware's estimates (2^-24)
 // and one third-order step each, which leaves the rounding of its last
-// operations (within about one ulp).  Used by the non-bitwise FP64 form, whose
-// contract is 1e-12 relative.
+// operations: over 2 M arguments at most 1.00 and 1.24 times 2^-53, 0.43 and 0.48
+// in the root mean square, as with two Newton steps (1.00 and 1.25, 0.43 and 0.47).
+// Used by the non-bitwise FP64 form, whose contract is 1e-12 relative.
 __device__ inline double rcp64(double x) {
   const double y = __builtin_amdgcn_rcp(x);
   const double e = fma(-x, y, 1.0);
@@ -401,7 +403,7 @@ __device__ inline double rsq64(double x) {
 // sqrt(x) / h for hinv near 1 / h: one Newton step on the reciprocal square
 // root, then a residual step on the root and one on the quotient, which leave
 // both rounded as the exact operations round them (but for rare last-place
-// cases).  1 - q keeps its digits that way where q is near 1.  The estimate is held
+// cases: at most 1.44 times 2^-53, as sqrt(x) / h; x rsq(x) hinv has 3.4).  1 - q keeps its digits that way where q is near 1.  The estimate is held
 // to that of the smallest double (2^537, by its high word): at x = 0 (a neighbour at
 // the same point) it stays finite, and the products with x give 0.
 __device__ inline double sqrt_over(double x, double h, double hinv) {

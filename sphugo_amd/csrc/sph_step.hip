@@ -900,7 +900,9 @@ constexpr double kSeeded = -5.0;
 // too few neighbours for, within up to 1.1 h already, starts from the radius
 // that would hold 1.2 k at the density inside that (its h is set so that 1.1 h
 // is that radius): its first attempt had to fail, 4,700 particles of a tube took
-// 15.1 us in the exact search against 11.8, 77,777 11.5 against 10.6.
+// 15.1 us in the exact search against 11.8, 77,777 11.5 against 10.6.  For k, 1.2 k,
+// 1.5 k and 2 k, as timed apart: the tube 16.8, 14.2, 15.0 and 16.2 us, 77,777 14.5,
+// 12.4, 12.7 and 13.2, 262,144 16.7, 14.2, 14.5 and 16.1, 1M 26.7, 24.2, 24.9 and 26.8.
 constexpr double kFirstReach = 1.1, kMissReach = 1.2;
 static_assert(sizeof(WalkShared) == 10240, "sixteen waves per CU");
 
@@ -1398,7 +1400,7 @@ __device__ inline void seed_radii(WalkShared& sh, double4* gq, int ncand, uint32
 // short chain of loads, so small launches finish early.  Against the walk with
 // a query per lane and its separate selection and density kernel that this
 // replaced: 4M FP32C 1.40 -> 1.12 ms, 1M FP64 0.45 -> 0.33 ms, 77,777 at k = 19
-// 108 -> 31 us, 2,200 at k = 32 55 -> 13 us.  One wave per block: a wave that
+// 108 -> 31 us, 2,200 at k = 32 55 -> 15 us.  One wave per block: a wave that
 // ends frees its LDS at once (1.54 -> 1.39 ms); 10 KiB per wave and four waves
 // per SIMD without a spilled register, where five spilled 40 (1.39 -> 1.17 ms).
 //
@@ -1880,8 +1882,9 @@ __device__ inline void row_visit(const NbrRow row, int n0, int k, uint32_t self,
 // query's predicted fields before the search, three stages' candidates together;
 // the query is a scalar, so its simulation's parameters come by scalar loads, and
 // a cell's Hilbert index takes a third of the steps from the table.  Before and now,
-// us: 2,200 particles 10.1 -> 9.4, 77,777 12.4 -> 11.4, 262,144 14.3 -> 12.6, 1M
-// clustered 37.6 -> 34.3, 4M 119 -> 104, 32 batched simulations 14.9 -> 13.3.
+// us: 2,200 particles 10.1 -> 9.4, 77,777 12.4 -> 11.4, 262,144 14.3 -> 12.6, 32
+// batched simulations 14.9 -> 13.3; with the queries of full annuli, which the walk
+// has taken since (tighten), 1M clustered 37.6 -> 34.3, 4M 119 -> 104.
 template <bool BITWISE, bool FP32C>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_knn_fallback(
     const Item* __restrict__ items, const SimDev* __restrict__ sims, const double2* __restrict__ XY,
