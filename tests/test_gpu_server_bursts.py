@@ -35,10 +35,10 @@ def _check(srv, j, p, st, nsteps):
 def test_jobs_that_arrive_while_another_runs():
     srv = L.Server(20000, max_jobs=8, kmax=16)
     jobs = []
-    for i, (n, nsteps) in enumerate([(3001, 301), (1000, 7), (257, 1), (2048, 10), (1500, 2),
+    for i, (n, nsteps) in enumerate([(3001, 1501), (1000, 7), (257, 1), (2048, 10), (1500, 2),
                                      (900, 33)]):
         st = ics.blast(n, seed=50 + i)
-        p = _p(n)
+        p = _p(n, dt_half=1e-5)
         jobs.append((srv.submit(p, st, nsteps), p, st, nsteps))
         time.sleep(0.0023)
     assert srv.info(jobs[0][0])["state"] == "running"
