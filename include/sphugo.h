@@ -268,7 +268,7 @@ int sph_set_tuning(sph_sim* s, const double in[5]);
  * different steps of their lives; a job that ends frees its particle range for
  * the next one in the queue (FIFO, first fit).  The worker looks at the queue
  * and at the jobs' errors between passes, after every one or, where at most
- * about 500,000 particles run (a pass of some 0.4 ms), after up to four in
+ * about a million particles run (a pass of some 0.7 ms), after up to four in
  * which no job ends: a job that arrives meanwhile is admitted, a job that
  * failed ends, and the steps that sph_server_job_info reports count on, that
  * much later.  A job's results equal those of sph_create + sph_step(nsteps)

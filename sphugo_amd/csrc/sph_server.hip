@@ -321,11 +321,15 @@ void fail_all_running(sph_server* s, const std::string& msg) {
 // the wait for it and the next launch's start each time, 25 us.  One pass per tick,
 // two, four and eight: a job of 4,700 particles and 21 steps 1.98, 1.74, 1.58 and 1.53
 // ms, a pass of 65,536 particles 137, 121, 117 and 133 us, of 262,144 240, 226, 221
-// and 246, so four.  With four against one, 524,288 particles take 364 us per
-// pass against 384 and a million 679 against 689, while an arrival's mean wait goes
-// from 0.15 to 0.5 and from 0.3 to 0.9 ms, so the line lies between.
+// and 246, so four.  With four against one, a million particles take 679 us per
+// pass against 689, 4M the same either way, while an arrival's mean wait goes
+// from 0.3 to 1.2 and from 0.9 to 4.4 ms.  In a mix of jobs of 1,024 to
+// 2^20 particles at 70 % load, mean latency (most of it the runs) and median queue
+// wait: bound by 2,048 items 73 and 0.34 ms against 69 and 0.70 unbounded beside it;
+// 4,096 items 67 and 0.44, 8,192 67 and 0.63, unbounded 66 and 0.73 (runs of one kind
+// differ by 2 ms).
 constexpr int kBurst = 4;
-constexpr int kBurstItems = 2048;
+constexpr int kBurstItems = 4096;
 
 // One tick: admission, passes over the pool, completions.
 // Returns false when the worker should stop.

@@ -78,9 +78,9 @@ def test_failure_between_two_looks_at_the_flags():
 
 
 def test_arrivals_wait_for_one_pass_of_a_large_job():
-    """A pass over a million particles takes 0.6 ms and more; a job that arrives is
-    admitted after the one that runs, half a pass away on average."""
-    n, nsteps = 1 << 20, 500
+    """Beside two million particles a job that arrives is admitted after the pass that
+    runs, half a pass away on average."""
+    n, nsteps = 2000000, 300
     st, small = ics.uniform(n, seed=1), ics.uniform(300, seed=2)
     srv = L.Server(n + 4096, max_jobs=8, kmax=16)
     big = srv.submit(_p(n, dt_half=1e-9), st, nsteps)
