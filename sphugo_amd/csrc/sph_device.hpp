@@ -400,22 +400,21 @@ __device__ inline double rsq64(double x) {
   return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// sqrt(x) / h for hinv near 1 / h: one Newton step on the reciprocal square
-// root, then a residual step on the root and one on the quotient, which leave
-// both rounded as the exact operations round them (but for rare last-place
-// cases: at most 1.44 times 2^-53, as sqrt(x) / h; x rsq(x) hinv has 3.4).  1 - q keeps its digits that way where q is near 1.  The estimate is held
-// to that of the smallest double (2^537, by its high word): at x = 0 (a neighbour at
-// the same point) it stays finite, and the products with x give 0.
+// sqrt(x) / h in [0, 1] for hinv near 1 / h: one Newton step on the reciprocal
+// square root, then a residual step on the root and one on the quotient, which
+// leave both rounded as the exact operations round them (but for rare last-place
+// cases: at most 1.44 times 2^-53, as sqrt(x) / h; x rsq(x) hinv has 3.4).  1 - q
+// keeps its digits that way where q is near 1.  At x = 0 (a neighbour at the same
+// point) the estimate is infinite and its products with x no number: the maximum
+// makes that 0 (both bounds are the last operation's own clamp, no instruction).
 __device__ inline double sqrt_over(double x, double h, double hinv) {
   double y = __builtin_amdgcn_rsq(x);
-  const uint32_t top = (uint32_t)__double2hiint(y);
-  y = __hiloint2double((int)(top < 0x61800000u ? top : 0x61800000u), __double2loint(y));
   const double t = 0.5 * x * y;
   y = fma(y, fma(-t, y, 0.5), y);
   const double s0 = x * y;
   const double s = fma(fma(-s0, s0, x), 0.5 * y, s0);
   const double q = s * hinv;
-  return fma(fma(-q, h, s), hinv, q);
+  return __builtin_fmin(__builtin_fmax(fma(fma(-q, h, s), hinv, q), 0.0), 1.0);
 }
 
 // ---- wave helpers (wave64) ----
